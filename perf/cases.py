@@ -83,7 +83,7 @@ def draw(rng):
         return {"kind": kind, "rows": rows, "cols": _log(rng, 100, 100_000_000 // rows),
                 "dtype": rng.choice(("float32", "float32", "float16", "int32"))}
     if kind == "columns":
-        cols = _log(rng, 3, 1000)
+        cols = _log(rng, 8, 1000)
         return {"kind": kind, "rows": _log(rng, 30_000, 100_000_000 // cols), "cols": cols,
                 "dtype": rng.choice(("float32", "float32", "float64"))}
     if kind == "scan":
