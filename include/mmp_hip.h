@@ -471,6 +471,17 @@ int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                const void *A, int64_t lda, int64_t sA, const void *B,
                int64_t ldb, int64_t sB, void *C, int64_t ldc, int64_t sC);
 
+/* mmp_matmul with operands stored transposed: trans_a, A holds (K,M) with
+ * row stride lda >= M; trans_b, B holds (N,K) with row stride ldb >= K.
+ * Transposed operands: MMP_F32 and MMP_F64.  Products whose outputs are too
+ * few to fill the device split the K range: their partial products take
+ * memory from the allocator for the call (not while the stream is captured:
+ * such a call runs unsplit). */
+int mmp_matmul_t(int dtype, int trans_a, int trans_b, int64_t batch, int64_t M,
+                 int64_t N, int64_t K, const void *A, int64_t lda, int64_t sA,
+                 const void *B, int64_t ldb, int64_t sB, void *C, int64_t ldc,
+                 int64_t sC);
+
 /* ======================================================================== */
 /* Runtime compilation: replaces createLibraryFromString + setFunction +    */
 /* runFunction (_metal_backend.py:237-257, 313-357) for the fusion engine  */

@@ -208,6 +208,7 @@ EXPORTS = (
     "mmp_unary", "mmp_binary", "mmp_binary_scalar", "mmp_copy",
     "mmp_copy_strided", "mmp_fill",
     "mmp_reduce", "mmp_reduce_noalloc", "mmp_argreduce", "mmp_scan", "mmp_matmul",
+    "mmp_matmul_t",
     "mmp_sort", "mmp_searchsorted", "mmp_take", "mmp_gather", "mmp_scatter", "mmp_nonzero",
     "mmp_mask_tile_counts", "mmp_mask_positions", "mmp_mask_compact",
     "mmp_bincount", "mmp_histogram",

@@ -123,6 +123,8 @@ _SIGNATURES = {
     "mmp_svd": [_c_int, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp],
     "mmp_matmul": [_c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64,
                    _c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64],
+    "mmp_matmul_t": [_c_int, _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64,
+                     _c_i64, _c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64],
     "mmp_rtc_compile": [ctypes.c_char_p, ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(_c_vp)],
     "mmp_rtc_build": [ctypes.c_char_p, ctypes.c_char_p, ctypes.c_char_p, _c_vp, _c_sz,
                       ctypes.POINTER(_c_sz)],
@@ -525,6 +527,12 @@ class HipBackend:
                C: int, ldc: int, sC: int) -> None:
         _check(self._lib.mmp_matmul(dcode, batch, M, N, K, A, lda, sA, B, ldb, sB,
                                     C, ldc, sC), "mmp_matmul")
+
+    def matmul_t(self, dcode: int, ta: bool, tb: bool, batch: int, M: int, N: int, K: int,
+                 A: int, lda: int, sA: int, B: int, ldb: int, sB: int,
+                 C: int, ldc: int, sC: int) -> None:
+        _check(self._lib.mmp_matmul_t(dcode, ta, tb, batch, M, N, K, A, lda, sA, B, ldb, sB,
+                                      C, ldc, sC), "mmp_matmul_t")
 
     # ------------------------------------------ reference kernel interface
     def execute_kernel(self, shader_src: str, func_name, grid_size, buffers) -> None:

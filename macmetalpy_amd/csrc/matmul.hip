@@ -7,9 +7,9 @@
 // Row-major operands: A (M, K) row stride lda, B (K, N) row stride ldb,
 // C (M, N) row stride ldc; batch strides sA, sB, sC (0 broadcasts).
 //
-// Floating kernels: a 128 x 128 output tile per 256-thread workgroup, four
-// wave64s in a 2 x 2 arrangement, each owning 64 x 64 = 4 x 4 MFMA 16x16
-// tiles (64 fp32 accumulators per lane).  K advances in 128-byte slabs
+// Floating kernels: a 128 x 128 (or 64 x 64, k_gemm4) output tile per
+// 256-thread workgroup, four wave64s in a 2 x 2 arrangement, each owning
+// 64 x 64 = 4 x 4 MFMA 16x16 tiles (64 fp32 accumulators per lane).  K advances in 128-byte slabs
 // (BK = 64 halves / 32 floats / 16 doubles) through two LDS buffers: the
 // next slab is fetched into registers while the current one feeds the
 // MFMAs, then written to the other buffer (one barrier per slab).
@@ -29,8 +29,11 @@
 //    LDS into swizzled stages: k_gemm4_dma3 (256 x 128 tiles, persistent,
 //    three stages) when the tiles fill whole rounds of the CUs, else
 //    k_gemm4_dma (128 x 128 tiles).
-// Partial tiles and unaligned operands use guarded scalar loads (zero fill)
-// and guarded stores.  Integer matmul: LDS-tiled exact kernel with
+//    Everything else of these types is k_gemm4: any extents and alignment,
+//    operands as they are or transposed, the K range split over workgroups
+//    where the output has few tiles.
+// Partial tiles and unaligned operands of the 16-bit kernels use guarded
+// scalar loads (zero fill) and guarded stores.  Integer matmul: LDS-tiled exact kernel with
 // wrap-around arithmetic (NumPy's integer matmul wraps).
 #include "mmp_ops.h"
 #include "mmp_internal.h"
@@ -429,60 +432,115 @@ template <> struct Mfma4<double> {
   static __device__ __forceinline__ int out_row(int g, int r) { return g + 4 * r; }
 };
 
-template <typename T, bool EDGE>
+// General float32 / float64 product.  Any extents, alignment and row strides;
+// A may be stored transposed (TA: element (m, k) at A[k * lda + m]) and so may
+// B (TB: element (k, n) at B[n * ldb + k]), so that x.T @ y and x @ y.T read
+// their operands where they lie instead of through a transposed copy.  A tile
+// of 32 I x 32 J outputs per 256-thread workgroup: four waves (2 x 2), each
+// I x J MFMA 16 x 16 tiles; K advances in 128-byte slabs through two LDS
+// buffers, the next slab fetched into registers while this one feeds the
+// MFMAs.
+//
+// Loads.  Every slab but the tile's last is read with unguarded 16-byte
+// vectors, also where rows are not 16-byte aligned (element alignment is
+// enough for a global load).  Rows (columns) past the edge re-read the last
+// one, or the next row's start: such values only reach outputs that are not
+// stored.  `edge` says when even that could leave the operand: bit 0, the
+// last slab is guarded element by element and zero filled (it is a partial
+// one, or a vector at the end of the operand's last row would run over it);
+// bit 1, every slab is (rows shorter than a vector, or so long that the
+// 32-bit lane offsets do not reach).
+//
+// blockIdx.z takes slabs [z * kspan, (z + 1) * kspan) and writes its own
+// partial product sZ elements further on (k_sum_splits adds them).  `sub`:
+// C -= A B in place of C = A B.
+//
+// Bound by the MFMAs at full tiles: float32 3000 x 2500 x 2001 369 -> 276 us
+// (81 -> 109 TFLOP/s) against guarded element loads throughout; float64
+// X.T @ X of 100,000 x 500 15.8 ms -> 0.84 ms (60 TFLOP/s; 68 is what a large
+// product reaches), of that 0.28 ms no longer spent on transposed copies.
+template <typename T, bool TA, bool TB, int I, int J>
 __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, const T *__restrict__ B,
                                                     T *__restrict__ C, int M, int N, int K,
                                                     long long lda, long long ldb, long long ldc,
                                                     long long sA, long long sB, long long sC,
-                                                    int tiles_n) {
+                                                    long long sZ, int tiles_n, int kspan, int edge,
+                                                    int sub) {
   constexpr int V = 16 / sizeof(T);        // elements per 16-byte vector
   constexpr int BK = 128 / sizeof(T);      // 32 floats / 16 doubles per slab
   constexpr int KG = BK / 4;               // k per lane group per slab
-  constexpr int LDA = BK + V;              // padded A row (k-contiguous)
-  constexpr int LDB = BN + V;              // padded B row (n-contiguous)
-  constexpr int AV = BM * BK / V / kBlock; // A vectors per thread (4)
-  constexpr int BV = BK * BN / V / kBlock; // B vectors per thread (4)
+  constexpr int TM = 32 * I, TN = 32 * J;  // output tile
+  constexpr int LDA = TA ? TM + V : BK + V;  // padded LDS rows: m- or k-contiguous
+  constexpr int LDB = TB ? BK + V : TN + V;
+  constexpr int AV = TM * BK / V / kBlock;  // vectors per thread
+  constexpr int BV = TN * BK / V / kBlock;
+  constexpr int A_VPR = TA ? TM / V : BK / V;  // vectors per row of the tile
+  constexpr int B_VPR = TB ? BK / V : TN / V;
   typedef typename Mfma4<T>::acc_t ACC;
-  __shared__ __attribute__((aligned(16))) T As[2][BM * LDA];
-  __shared__ __attribute__((aligned(16))) T Bs[2][BK * LDB];
+  typedef T VU __attribute__((ext_vector_type(V), aligned(sizeof(T))));  // unaligned global vector
+  typedef T VL __attribute__((ext_vector_type(V)));
+  __shared__ __attribute__((aligned(16))) T As[2][(TA ? BK : TM) * LDA];
+  __shared__ __attribute__((aligned(16))) T Bs[2][(TB ? TN : BK) * LDB];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
   const long long bz = blockIdx.y;
-  const int m0 = tm * BM, n0 = tn * BN;
-  const T *Ag = A + bz * sA;
-  const T *Bg = B + bz * sB;
+  const int m0 = tm * TM, n0 = tn * TN;
+  const T *Ag = A + bz * sA + (TA ? (long long)m0 : (long long)m0 * lda);
+  const T *Bg = B + bz * sB + (TB ? (long long)n0 * ldb : (long long)n0);
 
-  constexpr int A_VPR = BK / V;   // vectors per A row (8)
-  constexpr int B_VPR = BN / V;   // vectors per B row (32 / 64)
-  u32x4 ra[AV], rb[BV];
+  // Lane offsets of the unguarded loads, from the slab's first element.
+  unsigned ao[AV], bo[BV];
+#pragma unroll
+  for (int p = 0; p < AV; ++p) {
+    const int idx = tid + p * kBlock, r = idx / A_VPR, v = (idx % A_VPR) * V;
+    if constexpr (TA)
+      ao[p] = (unsigned)r * (unsigned)lda + (unsigned)(m0 + v < M ? v : 0);
+    else
+      ao[p] = (unsigned)min(r, M - 1 - m0) * (unsigned)lda + (unsigned)v;
+  }
+#pragma unroll
+  for (int p = 0; p < BV; ++p) {
+    const int idx = tid + p * kBlock, r = idx / B_VPR, v = (idx % B_VPR) * V;
+    if constexpr (TB)
+      bo[p] = (unsigned)min(r, N - 1 - n0) * (unsigned)ldb + (unsigned)v;
+    else
+      bo[p] = (unsigned)r * (unsigned)ldb + (unsigned)(n0 + v < N ? v : 0);
+  }
+  VL ra[AV], rb[BV];
+  const int nk = (K + BK - 1) / BK;
+  const int kb = blockIdx.z * kspan, ke = min(nk, kb + kspan);
 
-  auto load = [&](int k0) {
+  auto load = [&](int kt) {
+    const int k0 = kt * BK;
+    if (!((edge & 2) || ((edge & 1) && kt == nk - 1))) {
+      const T *ga = Ag + (TA ? (long long)k0 * lda : (long long)k0);
+      const T *gb = Bg + (TB ? (long long)k0 : (long long)k0 * ldb);
+#pragma unroll
+      for (int p = 0; p < AV; ++p) ra[p] = *reinterpret_cast<const VU *>(ga + ao[p]);
+#pragma unroll
+      for (int p = 0; p < BV; ++p) rb[p] = *reinterpret_cast<const VU *>(gb + bo[p]);
+      return;
+    }
 #pragma unroll
     for (int p = 0; p < AV; ++p) {
-      const int idx = tid + p * kBlock;
-      const int r = m0 + idx / A_VPR, k = k0 + (idx % A_VPR) * V;
-      if constexpr (!EDGE) {
-        ra[p] = *reinterpret_cast<const u32x4 *>(Ag + (long long)r * lda + k);
-      } else {
-        T h[V];
+      const int idx = tid + p * kBlock, r = idx / A_VPR, v = (idx % A_VPR) * V;
 #pragma unroll
-        for (int e = 0; e < V; ++e) h[e] = (r < M && k + e < K) ? Ag[(long long)r * lda + k + e] : (T)0;
-        __builtin_memcpy(&ra[p], h, 16);
+      for (int e = 0; e < V; ++e) {
+        const int m = TA ? v + e : r, k = k0 + (TA ? r : v + e);
+        ra[p][e] = (m0 + m < M && k < K)
+                       ? Ag[TA ? (long long)k * lda + m : (long long)m * lda + k] : (T)0;
       }
     }
 #pragma unroll
     for (int p = 0; p < BV; ++p) {
-      const int idx = tid + p * kBlock;
-      const int k = k0 + idx / B_VPR, n = n0 + (idx % B_VPR) * V;
-      if constexpr (!EDGE) {
-        rb[p] = *reinterpret_cast<const u32x4 *>(Bg + (long long)k * ldb + n);
-      } else {
-        T h[V];
+      const int idx = tid + p * kBlock, r = idx / B_VPR, v = (idx % B_VPR) * V;
 #pragma unroll
-        for (int e = 0; e < V; ++e) h[e] = (k < K && n + e < N) ? Bg[(long long)k * ldb + n + e] : (T)0;
-        __builtin_memcpy(&rb[p], h, 16);
+      for (int e = 0; e < V; ++e) {
+        const int n = TB ? r : v + e, k = k0 + (TB ? v + e : r);
+        rb[p][e] = (n0 + n < N && k < K)
+                       ? Bg[TB ? (long long)n * ldb + k : (long long)k * ldb + n] : (T)0;
       }
     }
   };
@@ -490,62 +548,135 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, co
 #pragma unroll
     for (int p = 0; p < AV; ++p) {
       const int idx = tid + p * kBlock;
-      *reinterpret_cast<u32x4 *>(&As[buf][(idx / A_VPR) * LDA + (idx % A_VPR) * V]) = ra[p];
+      *reinterpret_cast<VL *>(&As[buf][(idx / A_VPR) * LDA + (idx % A_VPR) * V]) = ra[p];
     }
 #pragma unroll
     for (int p = 0; p < BV; ++p) {
       const int idx = tid + p * kBlock;
-      *reinterpret_cast<u32x4 *>(&Bs[buf][(idx / B_VPR) * LDB + (idx % B_VPR) * V]) = rb[p];
+      *reinterpret_cast<VL *>(&Bs[buf][(idx / B_VPR) * LDB + (idx % B_VPR) * V]) = rb[p];
     }
   };
 
-  ACC acc[4][4];
+  ACC acc[I][J];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = ACC{0, 0, 0, 0};
+    for (int j = 0; j < J; ++j) acc[i][j] = ACC{0, 0, 0, 0};
 
-  const int nk = (K + BK - 1) / BK;
-  load(0);
-  store(0);
-  __syncthreads();
   const int fr = lane & 15, g = lane >> 4;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) load((kt + 1) * BK);
-    T af[4][KG], bf[4][KG];
+  if (kb < ke) {
+    load(kb);
+    store(0);
+  }
+  __syncthreads();
+  for (int kt = kb; kt < ke; ++kt) {
+    const int cur = (kt - kb) & 1;
+    if (kt + 1 < ke) load(kt + 1);
+    // V of the slab's k per lane group at a time: all KG at once would not
+    // leave a double tile's accumulators their registers
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const T *src = &As[cur][(wm * 64 + i * 16 + fr) * LDA + g * KG];
+    for (int t0 = 0; t0 < KG; t0 += V) {
+      T af[I][V], bf[J][V];
 #pragma unroll
-      for (int t = 0; t < KG; t += V)
-        *reinterpret_cast<u32x4 *>(&af[i][t]) = *reinterpret_cast<const u32x4 *>(src + t);
+      for (int i = 0; i < I; ++i) {
+        const int m = wm * 16 * I + i * 16 + fr;
+        if constexpr (TA) {
+#pragma unroll
+          for (int t = 0; t < V; ++t) af[i][t] = As[cur][(g * KG + t0 + t) * LDA + m];
+        } else {
+          *reinterpret_cast<VL *>(&af[i][0]) =
+              *reinterpret_cast<const VL *>(&As[cur][m * LDA + g * KG + t0]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int n = wn * 16 * J + j * 16 + fr;
+        if constexpr (TB) {
+          *reinterpret_cast<VL *>(&bf[j][0]) =
+              *reinterpret_cast<const VL *>(&Bs[cur][n * LDB + g * KG + t0]);
+        } else {
+#pragma unroll
+          for (int t = 0; t < V; ++t) bf[j][t] = Bs[cur][(g * KG + t0 + t) * LDB + n];
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < V; ++t)
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+          for (int j = 0; j < J; ++j) acc[i][j] = Mfma4<T>::mfma(af[i][t], bf[j][t], acc[i][j]);
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int t = 0; t < KG; ++t) bf[j][t] = Bs[cur][(g * KG + t) * LDB + wn * 64 + j * 16 + fr];
-#pragma unroll
-    for (int t = 0; t < KG; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = Mfma4<T>::mfma(af[i][t], bf[j][t], acc[i][j]);
-    if (kt + 1 < nk) store(cur ^ 1);
+    if (kt + 1 < ke) store(cur ^ 1);
     __syncthreads();
   }
 
-  T *Cb = C + bz * sC;
+  T *Cb = C + bz * sC + (long long)blockIdx.z * sZ;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm * 64 + i * 16 + Mfma4<T>::out_row(g, r);
-        const int col = n0 + wn * 64 + j * 16 + fr;
-        if (!EDGE || (row < M && col < N)) Cb[(long long)row * ldc + col] = acc[i][j][r];
+        const int row = m0 + wm * 16 * I + i * 16 + Mfma4<T>::out_row(g, r);
+        const int col = n0 + wn * 16 * J + j * 16 + fr;
+        if (row < M && col < N) {
+          T *o = Cb + (long long)row * ldc + col;
+          *o = sub ? *o - acc[i][j][r] : acc[i][j][r];
+        }
       }
+}
+
+// C[b][row][col] = sum over z of P[z][b][row][col] in float64, the partial
+// products of a split K range.  ZL threads of a workgroup share an output:
+// each adds its z = zl, zl + ZL, ... in eight running sums, and the sums meet
+// in a tree (a fixed order, and short chains: thousands of partials cost no
+// accuracy or time that one thread's long chain would).
+template <typename T, int ZL>
+__global__ __launch_bounds__(kBlock) void k_sum_splits(const T *__restrict__ P, T *__restrict__ C,
+                                                       int M, int N, long long ldc, long long sC,
+                                                       long long total, int splits) {
+  constexpr int OL = kBlock / ZL;  // outputs per workgroup
+  __shared__ double red[ZL][OL];
+  const int ol = threadIdx.x % OL, zl = threadIdx.x / OL;
+  const long long t = (long long)blockIdx.x * OL + ol;
+  double s[8] = {};
+  if (t < total) {
+    int z = zl;
+    for (; z + 7 * ZL < splits; z += 8 * ZL) {
+      T v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = P[(long long)(z + u * ZL) * total + t];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s[u] += (double)v[u];
+    }
+    for (int u = 0; u < 7; ++u)
+      if (z + u * ZL < splits) s[u] += (double)P[(long long)(z + u * ZL) * total + t];
+  }
+  red[zl][ol] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  __syncthreads();
+  for (int h = ZL / 2; h > 0; h >>= 1) {
+    if (zl < h) red[zl][ol] += red[zl + h][ol];
+    __syncthreads();
+  }
+  if (zl == 0 && t < total) {
+    const long long mn = (long long)M * N, b = t / mn, rem = t - b * mn;
+    const int row = (int)(rem / N), col = (int)(rem - (long long)row * N);
+    C[b * sC + (long long)row * ldc + col] = (T)red[0][ol];
+  }
+}
+
+template <typename T>
+int launch_sum_splits(const T *part, T *C, int M, int N, long long ldc, long long sC, long long total,
+                      int splits) {
+  // 64 consecutive outputs per wave read whole lines; few outputs take more
+  // threads each instead
+  if (total > 4096)
+    hipLaunchKernelGGL((k_sum_splits<T, 4>), dim3((unsigned)mmpi::ceil_div(total, kBlock / 4)),
+                       dim3(kBlock), 0, mmpi::stream(), part, C, M, N, ldc, sC, total, splits);
+  else
+    hipLaunchKernelGGL((k_sum_splits<T, 32>), dim3((unsigned)mmpi::ceil_div(total, kBlock / 32)),
+                       dim3(kBlock), 0, mmpi::stream(), part, C, M, N, ldc, sC, total, splits);
+  return mmpi::check_launch("mmp_matmul(split sum)");
 }
 
 // ------------------------------------------- float32, global -> LDS DMA
@@ -1039,16 +1170,117 @@ int launch16(long long batch, int M, int N, int K, const void *A, long long lda,
   return mmpi::check_launch("mmp_matmul(mfma16)");
 }
 
-template <typename T>
-int launch4(long long batch, int M, int N, int K, const void *A, long long lda, long long sA,
-            const void *B, long long ldb, long long sB, void *C, long long ldc, long long sC) {
+// Tile and K split of the general float kernel.  With few output tiles most
+// CUs would idle, so the tile is made smaller or the K range cut as well; a
+// split pays for its partial products (written once, read once).  The choice
+// is the cheapest by this estimate, in microseconds: rounds of workgroups
+// over the CUs (two 128, four 64 or eight 32 wide tiles fit one), each a
+// start-up plus its slabs, at the matrix cores' rate for the workgroups that
+// share a CU but no faster than one alone hides its loads; and the partials
+// at 6 TB/s plus a launch.  At most 16,384 outputs over a K of 16,384 or more
+// are always cut into ranges of at most 2048, whose sums meet in float64:
+// float32 sums of 10^7 terms then stay within 5e-8 of exact (2e-6 with ranges
+// of 6000).  Measured over tiles and splits, the choice is the
+// fastest or within a tenth of it: float32 1000^3 28 us (32 wide, unsplit; 64
+// wide 30, 128 wide in four splits 34), 2049^3 198 (64 wide; 128 wide 231),
+// 4000 x 70 x 3000 35 (32 wide in two; unsplit 128 wide 94); float64 500 x 500
+// x 100,000 0.84 ms (128 wide in 32; unsplit 15.8).
+struct Plan4 {
+  int tile;    // 128, 64 or 32
+  int splits;  // K ranges
+  double us;
+};
+inline double rounds_us(double wgs, double per_cu, double slabs, double shared, double alone) {
+  const double cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
+  const double full = __builtin_floor(wgs / (cus * per_cu)), rest = wgs - full * cus * per_cu;
+  const double share = __builtin_ceil(rest / cus);
+  const double step = shared * share > alone ? shared * share : alone;
+  return full * (2.0 + slabs * shared * per_cu) + (rest > 0 ? 2.0 + slabs * step : 0.0);
+}
+inline Plan4 plan4(long long batch, int M, int N, int K, int elem, bool may_split) {
+  const int nk = (int)(((long long)K * elem + 127) / 128);
+  const double cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
+  Plan4 best{128, 1, 1e30};
+  const bool long_sum = may_split && batch == 1 && (double)M * N <= 16384 && K >= 16384;
+  const int s0 = !long_sum ? 1 : K < 2048 * 65535 ? (K + 2047) / 2048 : 65535;  // grid limit
+  for (int tile = 128; tile >= 32; tile /= 2) {
+    const double tiles = (double)((M + tile - 1) / tile) * ((N + tile - 1) / tile) * (double)batch;
+    const double per_cu = tile == 128 ? 2 : tile == 64 ? 4 : 8;
+    // a slab of one workgroup: of several sharing a CU, and alone on it
+    const double shared = tile == 128 ? 1.85 : tile == 64 ? 0.5 : 0.15;
+    const double alone = tile == 128 ? 2.2 : tile == 64 ? 0.65 : 0.25;
+    for (int s = s0; s <= 65535; s *= 2) {
+      const double wgs = tiles * s;
+      if (s > s0 && (!may_split || nk / s < 4 || wgs > 2 * cus * per_cu)) break;
+      double t = rounds_us(wgs, per_cu, (nk + s - 1) / s, shared, alone);
+      if (s > 1) t += 4.0 + 2e-6 * s * (double)batch * M * N * elem / 6.0;
+      if (t < best.us * 0.98) best = Plan4{tile, s, t};
+    }
+  }
+  return best;
+}
+
+template <typename T, bool TA, bool TB>
+int launch_general(long long batch, int M, int N, int K, const T *A, long long lda, long long sA,
+                   const T *B, long long ldb, long long sB, T *C, long long ldc, long long sC,
+                   bool sub) {
   constexpr int V = 16 / sizeof(T), BK = 128 / sizeof(T);
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const bool fast = M % BM == 0 && N % BN == 0 && K % BK == 0 && lda % V == 0 && ldb % V == 0 &&
-                    sA % V == 0 && sB % V == 0 && al(A, 16) && al(B, 16);
-  dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
+  // partial products need scratch memory: none while the stream is captured
+  // (a graph's replays would outlive it)
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const bool may_split = !sub && hipStreamIsCapturing(mmpi::stream(), &cap) == hipSuccess &&
+                         cap == hipStreamCaptureStatusNone;
+  Plan4 pl = plan4(batch, M, N, K, (int)sizeof(T), may_split);
+  const int nk = (K + BK - 1) / BK;
+  const int kspan = (nk + pl.splits - 1) / pl.splits;
+  const int splits = (nk + kspan - 1) / kspan;
+  const long long total = (long long)M * N * batch;
+  const int tile = pl.tile;
+  const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
+  // see the kernel: short rows a vector could run past, or offsets past 32 bits
+  const bool guard_all = lda < V - 1 || ldb < V - 1 || lda >= (1LL << 24) || ldb >= (1LL << 24);
+  const bool guard_last = K % BK || (TA && M % tile) || (!TB && N % tile);
+  const int edge = (guard_last ? 1 : 0) | (guard_all ? 2 : 0);
+  void *part = nullptr;
+  T *out = C;
+  long long oldc = ldc, osC = sC, osZ = 0;
+  if (splits > 1) {
+    if (int st = mmp_alloc((size_t)splits * (size_t)total * sizeof(T), &part)) return st;
+    out = (T *)part;
+    oldc = N;
+    osC = (long long)M * N;
+    osZ = total;
+  }
+  dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch, (unsigned)splits);
+  if (tile == 128)
+    hipLaunchKernelGGL((k_gemm4<T, TA, TB, 4, 4>), grid, dim3(kBlock), 0, mmpi::stream(), A, B, out,
+                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0);
+  else if (tile == 64)
+    hipLaunchKernelGGL((k_gemm4<T, TA, TB, 2, 2>), grid, dim3(kBlock), 0, mmpi::stream(), A, B, out,
+                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0);
+  else
+    hipLaunchKernelGGL((k_gemm4<T, TA, TB, 1, 1>), grid, dim3(kBlock), 0, mmpi::stream(), A, B, out,
+                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0);
+  int st = mmpi::check_launch("mmp_matmul(mfma4)");
+  if (part) {
+    if (st == MMP_OK) st = launch_sum_splits<T>((const T *)part, C, M, N, ldc, sC, total, splits);
+    const int fs = mmp_free(part);  // stream-ordered
+    if (st == MMP_OK) st = fs;
+  }
+  return st;
+}
+
+template <typename T>
+int launch4(int ta, int tb, long long batch, int M, int N, int K, const void *A, long long lda,
+            long long sA, const void *B, long long ldb, long long sB, void *C, long long ldc,
+            long long sC, bool sub) {
   if constexpr (__is_same(T, float)) {
-    // the DMA kernel's per-lane copy offsets are 32-bit (7 lda + 28 floats)
+    constexpr int V = 4, BK = 32;
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const bool fast = !ta && !tb && !sub && M % BM == 0 && N % BN == 0 && K % BK == 0 &&
+                      lda % V == 0 && ldb % V == 0 && sA % V == 0 && sB % V == 0 && al(A, 16) &&
+                      al(B, 16);
+    // the DMA kernels' per-lane copy offsets are 32-bit (7 lda + 28 floats)
     if (fast && lda < (1LL << 28) && ldb < (1LL << 28)) {
       // 256 x 128 tiles (one persistent workgroup per CU) when the tiles fill
       // whole rounds of the CUs, or nearly; otherwise 128 x 128 tiles, whose
@@ -1064,21 +1296,27 @@ int launch4(long long batch, int M, int N, int K, const void *A, long long lda, 
         hipLaunchKernelGGL(k_gemm4_dma3, dim3((unsigned)P), dim3(512), 0, mmpi::stream(),
                            (const float *)A, (const float *)B, (float *)C, K, lda, ldb, ldc, sA,
                            sB, sC, tiles_n, (int)((M / 256) * tiles_n), (int)wide_tiles);
-      } else {
-        hipLaunchKernelGGL(k_gemm4_dma, grid, dim3(kBlock), 0, mmpi::stream(),
-                           (const float *)A, (const float *)B, (float *)C, M, N, K, lda, ldb, ldc,
-                           sA, sB, sC, tiles_n);
+        return mmpi::check_launch("mmp_matmul(mfma4 dma)");
       }
-      return mmpi::check_launch("mmp_matmul(mfma4 dma)");
+      // few tiles: the general kernel's smaller tiles or K ranges reach more CUs
+      if (rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 1.6, 2.2) <=
+          plan4(batch, M, N, K, 4, true).us) {
+        hipLaunchKernelGGL(k_gemm4_dma, dim3((unsigned)(tiles_m * tiles_n), (unsigned)batch),
+                           dim3(kBlock), 0, mmpi::stream(), (const float *)A, (const float *)B,
+                           (float *)C, M, N, K, lda, ldb, ldc, sA, sB, sC, tiles_n);
+        return mmpi::check_launch("mmp_matmul(mfma4 dma)");
+      }
     }
   }
-  if (fast)
-    hipLaunchKernelGGL((k_gemm4<T, false>), grid, dim3(kBlock), 0, mmpi::stream(), (const T *)A,
-                       (const T *)B, (T *)C, M, N, K, lda, ldb, ldc, sA, sB, sC, tiles_n);
-  else
-    hipLaunchKernelGGL((k_gemm4<T, true>), grid, dim3(kBlock), 0, mmpi::stream(), (const T *)A,
-                       (const T *)B, (T *)C, M, N, K, lda, ldb, ldc, sA, sB, sC, tiles_n);
-  return mmpi::check_launch("mmp_matmul(mfma4)");
+  const T *a = (const T *)A, *b = (const T *)B;
+  T *c = (T *)C;
+  if (ta && tb)
+    return launch_general<T, true, true>(batch, M, N, K, a, lda, sA, b, ldb, sB, c, ldc, sC, sub);
+  if (ta)
+    return launch_general<T, true, false>(batch, M, N, K, a, lda, sA, b, ldb, sB, c, ldc, sC, sub);
+  if (tb)
+    return launch_general<T, false, true>(batch, M, N, K, a, lda, sA, b, ldb, sB, c, ldc, sC, sub);
+  return launch_general<T, false, false>(batch, M, N, K, a, lda, sA, b, ldb, sB, c, ldc, sC, sub);
 }
 
 template <typename T>
@@ -1093,9 +1331,13 @@ int launch_int(long long batch, int M, int N, int K, const void *A, long long ld
 
 }  // namespace
 
-extern "C" int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, const void *A,
-                          int64_t lda, int64_t sA, const void *B, int64_t ldb, int64_t sB, void *C,
-                          int64_t ldc, int64_t sC) {
+namespace {
+
+// Argument checks and dispatch of both entry points.  Transposed operands:
+// float32 and float64 only (ta: A holds (K, M), tb: B holds (N, K)).
+int matmul(int dtype, int ta, int tb, int64_t batch, int64_t M, int64_t N, int64_t K, const void *A,
+           int64_t lda, int64_t sA, const void *B, int64_t ldb, int64_t sB, void *C, int64_t ldc,
+           int64_t sC) {
   if (int st = mmpi::ensure_init()) return st;
   if (batch < 0 || M < 0 || N < 0 || K < 0) return mmpi::fail(MMP_E_ARG, "negative extent");
   if (batch == 0 || M == 0 || N == 0) return MMP_OK;
@@ -1104,15 +1346,20 @@ extern "C" int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_
     return mmpi::fail(MMP_E_ARG, "matmul extent exceeds 2^31 - 1");
   if (batch > 65535) return mmpi::fail(MMP_E_ARG, "batch %lld > 65535", (long long)batch);
   if (!A || !B || !C) return mmpi::fail(MMP_E_ARG, "null pointer");
-  if (lda < K || ldb < N || ldc < N) return mmpi::fail(MMP_E_ARG, "leading dimension too small");
+  if (lda < (ta ? M : K) || ldb < (tb ? K : N) || ldc < N)
+    return mmpi::fail(MMP_E_ARG, "leading dimension too small");
   const long long tiles = ((M + 127) / 128) * ((N + 127) / 128);
   if (tiles > 0x7fffffffLL) return mmpi::fail(MMP_E_ARG, "matmul grid too large");
   const int m = (int)M, n = (int)N, k = (int)K;
+  if (dtype == MMP_F32)
+    return launch4<float>(ta, tb, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, false);
+  if (dtype == MMP_F64)
+    return launch4<double>(ta, tb, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, false);
+  if (ta || tb)
+    return mmpi::fail(MMP_E_UNSUPPORTED, "transposed operands of matmul dtype %d", dtype);
   switch (dtype) {
     case MMP_F16: return launch16<mmp_half>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
     case MMP_BF16: return launch16<__bf16>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
-    case MMP_F32: return launch4<float>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
-    case MMP_F64: return launch4<double>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
     case MMP_I16: return launch_int<mmp_i16>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
     case MMP_U16: return launch_int<mmp_u16>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
     case MMP_I32: return launch_int<mmp_i32>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
@@ -1121,4 +1368,19 @@ extern "C" int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_
     case MMP_U64: return launch_int<mmp_u64>(batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC);
     default: return mmpi::fail(MMP_E_UNSUPPORTED, "matmul dtype %d", dtype);
   }
+}
+
+}  // namespace
+
+extern "C" int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, const void *A,
+                          int64_t lda, int64_t sA, const void *B, int64_t ldb, int64_t sB, void *C,
+                          int64_t ldc, int64_t sC) {
+  return matmul(dtype, 0, 0, batch, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC);
+}
+
+extern "C" int mmp_matmul_t(int dtype, int trans_a, int trans_b, int64_t batch, int64_t M, int64_t N,
+                            int64_t K, const void *A, int64_t lda, int64_t sA, const void *B,
+                            int64_t ldb, int64_t sB, void *C, int64_t ldc, int64_t sC) {
+  return matmul(dtype, trans_a != 0, trans_b != 0, batch, M, N, K, A, lda, sA, B, ldb, sB, C, ldc,
+                sC);
 }

@@ -36,28 +36,40 @@ def _batch_operand(x, batch_shape, mat_shape):
     return x._broadcast_copy(tuple(batch_shape) + tuple(mat_shape), x._dtype), _prod(mat_shape)
 
 
-_SPLITK_MAX_OUT = 128 * 128   # outputs too few to fill the device with tiles
-_SPLITK_MIN_K = 16384
-_SPLITK_CHUNK = 2048
+def _in_place(x, batch_shape):
+    """(transposed, row stride, batch stride) of a device view that the
+    general kernel can read where it lies, or None.  Its matrices have one
+    unit stride and rows (columns) that do not overlap, and its batch is one
+    stride: the batch dimensions nest, or all have one entry, or are
+    ``batch_shape`` broadcast from a single matrix (batch stride 0)."""
+    rows, cols = x._shape[-2:]
+    rs, cs = x._strides[-2:]
+    if cs == 1 and rs >= cols:
+        ta, ld = False, rs
+    elif rs == 1 and cs >= rows:
+        ta, ld = True, cs
+    else:
+        return None
+    batch = [(n, st) for n, st in zip(x._shape[:-2], x._strides[:-2]) if n != 1]
+    if not batch:
+        return ta, ld, 0
+    if x._shape[:-2] != tuple(batch_shape):
+        return None
+    for (_, outer), (n, inner) in zip(batch, batch[1:]):
+        if outer != n * inner:
+            return None
+    if batch[-1][1] < 0:
+        return None
+    return ta, ld, batch[-1][1]
 
 
-def _matmul_split_k(rdt, M, N, K, A, B, res):
-    """A small output with a long sum (e.g. X @ X.T of a wide X): the K
-    range is cut into chunks that run as one batched matmul, so that every
-    chunk gets its own workgroups, and the partial products are summed
-    (float64 accumulation) into the result."""
-    from .reductions import sum as _sum
-    kc = _SPLITK_CHUNK
-    nb = K // kc
-    rem = K - nb * kc
-    isz = rdt.itemsize
-    part = ndarray._empty_device((nb + (1 if rem else 0), M, N), rdt)
-    be = HipBackend()
-    be.matmul(dtype_code(rdt), nb, M, N, kc, A._ptr, K, kc, B._ptr, N, kc * N, part._ptr, N, M * N)
-    if rem:
-        be.matmul(dtype_code(rdt), 1, M, N, rem, A._ptr + nb * kc * isz, K, 0,
-                  B._ptr + nb * kc * N * isz, N, 0, part._ptr + nb * M * N * isz, N, M * N)
-    res[...] = _sum(part, axis=0)
+def _copy_kernel_shape(M, N, K, batch):
+    """Whether a float32 product of contiguous operands takes the kernels
+    that copy global -> LDS, with enough tiles to fill the device: those gain
+    more over the general kernel than transposing an operand first costs
+    (4096^3 with a transposed operand: 1.00 ms against 1.11)."""
+    return (M % 128 == 0 and N % 128 == 0 and K % 32 == 0
+            and M * N * batch >= 256 * 128 * 128)
 
 
 def matmul(x1, x2, out=None, **kwargs):
@@ -84,18 +96,24 @@ def matmul(x1, x2, out=None, **kwargs):
         A = A.astype(rdt)
     if B._dtype != rdt:
         B = B.astype(rdt)
-    A, sA = _batch_operand(A, batch_shape, (M, K))
-    B, sB = _batch_operand(B, batch_shape, (K, N))
+    A._ensure_gpu()
+    B._ensure_gpu()
+    pa = pb = None
+    if rdt == np.float64 or (rdt == np.float32 and not _copy_kernel_shape(M, N, K, batch)):
+        pa, pb = _in_place(A, batch_shape), _in_place(B, batch_shape)
+    if pa is None:
+        A, sA = _batch_operand(A, batch_shape, (M, K))
+        pa = False, K, sA
+    if pb is None:
+        B, sB = _batch_operand(B, batch_shape, (K, N))
+        pb = False, N, sB
     res = ndarray._empty_device(tuple(batch_shape) + (M, N), rdt)
     if res.size:
         if K == 0:
             res.fill(0)
-        elif (batch == 1 and M * N <= _SPLITK_MAX_OUT and K >= _SPLITK_MIN_K
-              and rdt in (np.float32, np.float64)):
-            _matmul_split_k(rdt, M, N, K, A, B, res)
         else:
-            HipBackend().matmul(dtype_code(rdt), batch, M, N, K, A._ptr, K, sA, B._ptr, N, sB,
-                                res._ptr, N, M * N)
+            HipBackend().matmul_t(dtype_code(rdt), pa[0], pb[0], batch, M, N, K, A._ptr, pa[1], pa[2],
+                                  B._ptr, pb[1], pb[2], res._ptr, N, M * N)
     if a1:
         res = res.reshape(tuple(batch_shape) + (N,))
     elif b1:

@@ -1,0 +1,132 @@
+"""Which operands matmul reads where they lie (CPU), and the general float32 /
+float64 kernel on extents around its tiles, K splits, transposed, strided and
+misaligned operands against exact integer products (GPU)."""
+import numpy as np
+import pytest
+
+import macmetalpy_amd as cp
+from macmetalpy_amd import linalg_top
+
+
+class _Strided:
+    """Shape and element strides of a view, as the rule reads them."""
+
+    def __init__(self, view):
+        self._shape = view.shape
+        self._strides = tuple(s // view.itemsize for s in view.strides)
+
+
+def _views():
+    x = np.arange(2 * 3 * 6 * 8, dtype=np.float32).reshape(2, 3, 6, 8)
+    yield from (x, x.swapaxes(-1, -2), x[..., 1:], x[..., ::2], x[..., ::-1], x[:, ::2], x[::-1],
+                x.transpose(1, 0, 2, 3), x.transpose(2, 0, 1, 3), x.transpose(3, 2, 1, 0),
+                x[:1, :1], x[:1], x[:, :1, 2:, 3:], x[..., :1], x[..., :1, :], x[0, 0], x[0, 0].T,
+                x[0, 0][::2], x[0, 0][:, 2:5].T, x[0].swapaxes(0, 1), x[..., 3:4].swapaxes(-1, -2))
+    yield np.broadcast_to(x[0, 0], (2, 3, 6, 8))
+    yield np.broadcast_to(x[0, 0, :1], (6, 8))
+    yield np.broadcast_to(x[0, 0, :, :1], (6, 8))
+
+
+def test_in_place_rule_addresses_every_element():
+    """Wherever the rule accepts a view, (transposed, row stride, batch
+    stride) gives the address of every element that the view's own strides
+    give; what it refuses is copied as before."""
+    taken = 0
+    for v in _views():
+        s = _Strided(v)
+        got = linalg_top._in_place(s, v.shape[:-2])
+        if got is None:
+            continue
+        taken += 1
+        ta, ld, bs = got
+        rows, cols = v.shape[-2:]
+        assert ld >= (rows if ta else cols) and bs >= 0
+        for b, idx in enumerate(np.ndindex(*v.shape[:-2])):
+            for r in range(rows):
+                for c in range(cols):
+                    want = sum(i * t for i, t in zip(idx + (r, c), s._strides))
+                    assert b * bs + (c * ld + r if ta else r * ld + c) == want
+    assert taken >= 12
+
+
+def test_in_place_rule_refuses():
+    x = np.zeros((6, 8), np.float32)
+    for v in (x[:, ::2], x[::-1], x[:, ::-1], np.broadcast_to(x[:1], (6, 8)),
+              np.broadcast_to(x[:, :1], (6, 8))):
+        assert linalg_top._in_place(_Strided(v), ()) is None
+    y = np.zeros((4, 2, 6, 8), np.float32)
+    assert linalg_top._in_place(_Strided(y.swapaxes(0, 1)), (2, 4)) is None
+    assert linalg_top._in_place(_Strided(y[:, :1]), (4, 3)) is None  # broadcast batch
+
+
+def _exact(a, b, got):
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+    assert got.shape == want.shape and np.array_equal(got.astype(np.float64), want)
+
+
+def _ints(g, shape, dtype):
+    return g.integers(-3, 4, shape).astype(dtype)
+
+
+# Tile edges (32, 64, 128), slab edges (32 floats, 16 doubles), rows shorter
+# than a vector, K splits (one long sum, uneven last range) and batches.
+_SHAPES = [(1, 1, 2, 1), (1, 2, 2, 3), (1, 3, 5, 33), (1, 31, 33, 31), (1, 32, 32, 32),
+           (1, 65, 63, 17), (1, 127, 129, 64), (1, 129, 257, 65), (1, 200, 130, 1000),
+           (1, 2, 3, 40001), (1, 50, 70, 20000), (3, 33, 2, 35), (70, 20, 30, 40),
+           (1, 1030, 700, 100), (1, 4100, 60, 50), (5, 128, 128, 64)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("batch,m,n,k", _SHAPES)
+def test_general_kernel_exact(batch, m, n, k, dtype):
+    """Every combination of stored and transposed operands.  Integer values
+    keep each sum exact, so the result equals the float64 product."""
+    g = np.random.default_rng(m * 1000 + n + k)
+    lead = (batch,) if batch > 1 else ()
+    a, b = _ints(g, lead + (m, k), dtype), _ints(g, lead + (k, n), dtype)
+    at, bt = np.ascontiguousarray(a.swapaxes(-1, -2)), np.ascontiguousarray(b.swapaxes(-1, -2))
+    print("general", batch, m, n, k, np.dtype(dtype), flush=True)
+    for x in (cp.array(a), cp.array(at).swapaxes(-1, -2)):
+        for y in (cp.array(b), cp.array(bt).swapaxes(-1, -2)):
+            _exact(a, b, cp.matmul(x, y).get())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_general_kernel_views(dtype):
+    """Row slices, column slices (misaligned rows), steps, reversed and
+    broadcast operands, and batches that do and do not nest.  The memory
+    round the views holds NaN, which must not reach a result."""
+    g = np.random.default_rng(7)
+    big = np.full((4, 3, 70, 90), np.nan, dtype)
+    big[:, :, 3:67, 5:82] = _ints(g, (4, 3, 64, 77), dtype)
+    w = np.full((90, 50), np.nan, dtype)
+    w[2:79, 1:42] = _ints(g, (77, 41), dtype)
+    dbig, dw = cp.array(big), cp.array(w)
+    pick = [lambda x: x[0, 0], lambda x: x[:, 0], lambda x: x[0], lambda x: x,
+            lambda x: x.transpose(1, 0, 2, 3), lambda x: x[::2, 1:]]
+    for f in pick:
+        a, da = f(big)[..., 3:67, 5:82], f(dbig)[..., 3:67, 5:82]
+        b, db = w[2:79, 1:42], dw[2:79, 1:42]
+        _exact(a, b, cp.matmul(da, db).get())
+        at, dat = a.swapaxes(-1, -2), da.swapaxes(-1, -2)
+        _exact(b.T, at, cp.matmul(db.T, dat).get())
+        _exact(at, a, cp.matmul(dat, da).get())
+    a, da = big[0, 0, 3:67, 5:82], dbig[0, 0, 3:67, 5:82]
+    _exact(a[::2], w[2:79, 1:42], cp.matmul(da[::2], dw[2:79, 1:42]).get())
+    _exact(a[:, ::-1], w[2:79, 1:42], cp.matmul(da[:, ::-1], dw[2:79, 1:42]).get())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(40, 30, 60000), (4, 4, 2_000_003), (128, 128, 16384)])
+def test_long_sums_are_cut(m, n, k):
+    """At most 128 x 128 outputs over 16,384 terms or more: ranges of at most
+    2048 terms, added in float64, so a float32 sum's error stays below 2049
+    roundings of |A| |B| plus the result's own."""
+    g = np.random.default_rng(3)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    got = cp.matmul(cp.array(a), cp.array(b)).get().astype(np.float64)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(got - a @ b) <= 2050 * 2.0 ** -24 * (np.abs(a) @ np.abs(b)))
