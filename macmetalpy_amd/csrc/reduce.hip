@@ -621,78 +621,43 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_rows(const T *__restrict__
     out[row] = total.i;
 }
 
-// Strided axis: grid (ceil(inner / 256), outer, S); thread = column.
-template <int OP, typename T, typename To>
-__global__ __launch_bounds__(kBlock) void k_reduce_cols(const T *__restrict__ x, To *__restrict__ out,
-                                                       long long len, long long inner, int S,
-                                                       ReduceScratch sc) {
-  typedef Red<OP, T> R;
-  typedef typename R::A A;
-  constexpr int W = words_of<A>();
-  const long long o = blockIdx.y;
-  const int s = blockIdx.z;
-  const long long c = (long long)blockIdx.x * kBlock + threadIdx.x;
-  const long long per = (len + S - 1) / S;
-  const long long b0 = s * per;
-  const long long b1 = b0 + per < len ? b0 + per : len;
-  A v = R::ident();
-  if (c < inner) {
-    const T *p = x + o * len * inner + c;
-    long long l = b0;
-    for (; l + kColUnroll <= b1; l += kColUnroll) {  // loads first: kColUnroll in flight
-      T q[kColUnroll];
-#pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) q[u] = p[(l + u) * inner];
-#pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) v = R::comb(v, R::map(q[u]));
-    }
-    for (; l < b1; ++l) v = R::comb(v, R::map(p[l * inner]));
-  }
-  if (S == 1) {
-    if (c < inner) out[o * inner + c] = finalize<OP, T, To>(v, len);
-    return;
-  }
-  // one tagged partial per (o, column block, s, thread); ticket per (o, cb)
-  const long long cb = blockIdx.x, ncb = gridDim.x;
-  unsigned long long *grp = sc.words + (o * ncb + cb) * (long long)S * kBlock * W;
-  put_tagged(grp + ((long long)s * kBlock + threadIdx.x) * W, v, sc.tag);
-  __shared__ int is_last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned t = __hip_atomic_fetch_add(sc.tickets + o * ncb + cb, 1u, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-    is_last = (t == (unsigned)(S - 1));
-  }
-  __syncthreads();
-  if (!is_last) return;
-  const A acc = combine_tagged<R>(grp + (long long)threadIdx.x * W, (long long)kBlock * W, S, sc);
-  if (c < inner) out[o * inner + c] = finalize<OP, T, To>(acc, len);
-  if (threadIdx.x == 0)
-    __hip_atomic_store(sc.tickets + o * ncb + cb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// Partials of a strided reduction: up to kTaggedSplits are combined by the
+// last workgroup to arrive; more are left in the scratch words as they are,
+// (outer, split, column), for a second kernel (k_cols_finish) whose many
+// workgroups read them side by side.  One workgroup alone reading 256
+// partials a column took longer than the reduction of a 2,000,000 x 50 matrix
+// (float32 sum over axis 0 98 us, against 76 with the second kernel); of 31,
+// it is faster than a second launch (2000 x 300 8.6 us against 11.7).
+constexpr int kTaggedSplits = 64;
 
-// Strided arg-reduction: grid (ceil(inner / 256), outer, S); thread =
-// column, the reduced axis split over S workgroups combined in index order
-// by the last to arrive (as k_reduce_cols).
-template <int OP, typename T>
+// Strided arg-reduction: grid (ceil(inner / 2^lc), outer, S); 2^lc threads
+// side by side on the columns (as many as there are, up to the workgroup) and
+// the others on the rows below, whose results meet in LDS; the reduced axis
+// split over S workgroups, combined in index order.  float32 argmax over
+// axis 0: 2,000,000 x 50 648 -> 88 us, 10,000 x 10,001 109 -> 75, against a
+// thread per column and one workgroup combining.
+template <int OP, typename T, bool WIDE>  // WIDE: lc == 8, known at compile time
 __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__ x,
                                                           long long *__restrict__ out,
                                                           long long len, long long inner, int S,
-                                                          ReduceScratch sc) {
+                                                          int lc, ReduceScratch sc) {
   typedef Arg<OP, T> R;
   typedef typename R::A A;
   typedef typename mmp_t<T>::C C;
   constexpr int W = words_of<A>();
+  __shared__ A part[kBlock];
   const long long o = blockIdx.y;
   const int s = blockIdx.z;
-  const long long c = (long long)blockIdx.x * kBlock + threadIdx.x;
+  const int CT = WIDE ? kBlock : 1 << lc, RT = WIDE ? 1 : kBlock >> lc;
+  const int ct = threadIdx.x & (CT - 1), rt = WIDE ? 0 : threadIdx.x >> lc;
+  const long long c = (long long)blockIdx.x * CT + ct;
   const long long per = (len + S - 1) / S;
   const long long b0 = s * per;
   const long long b1 = b0 + per < len ? b0 + per : len;
   A v = R::ident();
   if (c < inner) {
     const T *p = x + o * len * inner + c;
-    long long l = b0;
+    long long l = b0 + rt;
     if (b1 - b0 < 0xffffffffLL) {
       // rows are visited in order: the sequential update rule with 32-bit
       // offsets from b0 (as slice_argreduce) instead of the index-comparing
@@ -705,33 +670,40 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__
         bv = upd ? e : bv;
         bi = upd ? off : bi;
       };
-      for (; l + kColUnroll <= b1; l += kColUnroll) {
+      for (; l + (long long)RT * (kColUnroll - 1) < b1; l += (long long)RT * kColUnroll) {
         T q[kColUnroll];
 #pragma unroll
-        for (int u = 0; u < kColUnroll; ++u) q[u] = p[(l + u) * inner];
+        for (int u = 0; u < kColUnroll; ++u) q[u] = p[(l + (long long)RT * u) * inner];
 #pragma unroll
-        for (int u = 0; u < kColUnroll; ++u) visit((C)q[u], (unsigned)(l + u - b0));
+        for (int u = 0; u < kColUnroll; ++u) visit((C)q[u], (unsigned)(l + (long long)RT * u - b0));
       }
-      for (; l < b1; ++l) visit((C)p[l * inner], (unsigned)(l - b0));
+      for (; l < b1; l += RT) visit((C)p[l * inner], (unsigned)(l - b0));
       if (bi != kNone) v = A{bv, b0 + (long long)bi};
     } else {
-      for (; l + kColUnroll <= b1; l += kColUnroll) {
-        T q[kColUnroll];
-#pragma unroll
-        for (int u = 0; u < kColUnroll; ++u) q[u] = p[(l + u) * inner];
-#pragma unroll
-        for (int u = 0; u < kColUnroll; ++u) v = R::comb(v, A{(C)q[u], l + u});
-      }
-      for (; l < b1; ++l) v = R::comb(v, A{(C)p[l * inner], l});
+      for (; l < b1; l += RT) v = R::comb(v, A{(C)p[l * inner], l});
     }
   }
+  if (RT > 1) {
+    part[threadIdx.x] = v;
+    for (int h = RT / 2; h > 0; h >>= 1) {
+      __syncthreads();
+      if (rt < h) part[threadIdx.x] = R::comb(part[threadIdx.x], part[threadIdx.x + h * CT]);
+    }
+    if (rt == 0) v = part[threadIdx.x];
+  }
+  const bool owner = rt == 0 && c < inner;
   if (S == 1) {
-    if (c < inner) out[o * inner + c] = v.i;
+    if (owner) out[o * inner + c] = v.i;
     return;
   }
+  if (S > kTaggedSplits) {
+    if (owner) reinterpret_cast<A *>(sc.words)[(o * S + s) * inner + c] = v;
+    return;
+  }
+  // one tagged partial per (o, column block, s, column); ticket per (o, cb)
   const long long cb = blockIdx.x, ncb = gridDim.x;
-  unsigned long long *grp = sc.words + (o * ncb + cb) * (long long)S * kBlock * W;
-  put_tagged(grp + ((long long)s * kBlock + threadIdx.x) * W, v, sc.tag);
+  unsigned long long *grp = sc.words + (o * ncb + cb) * (long long)S * CT * W;
+  if (rt == 0) put_tagged(grp + ((long long)s * CT + ct) * W, v, sc.tag);
   __shared__ int is_last;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -741,78 +713,156 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__
   }
   __syncthreads();
   if (!is_last) return;
-  const A acc = combine_tagged<R>(grp + (long long)threadIdx.x * W, (long long)kBlock * W, S, sc);
-  if (c < inner) out[o * inner + c] = acc.i;
+  if (rt == 0) {
+    const A acc = combine_tagged<R>(grp + (long long)ct * W, (long long)CT * W, S, sc);
+    if (owner) out[o * inner + c] = acc.i;
+  }
   if (threadIdx.x == 0)
     __hip_atomic_store(sc.tickets + o * ncb + cb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Strided axis with 16-byte column vectors (element size 2, 4 or 8 bytes,
-// inner extent a multiple of the vector, 16-byte aligned base): grid
-// (ceil(inner / CW), outer, S) with CW = 64 x VI columns per workgroup.
-// A lane owns VI adjacent columns and each wave takes every fourth row of
-// the split (one 1 KiB row segment per wave load, kColUnroll loads in
-// flight); the four waves' partials meet in LDS in wave order, then one
-// partial per (split, column) is combined in split order by the last
-// workgroup to arrive, as in k_reduce_cols.  Sums accumulate in the same
-// types; only the order of additions inside a split differs.
-template <typename T> constexpr int col_vec() { return 16 / (int)sizeof(T); }
-template <typename T> constexpr int col_width() { return 64 * col_vec<T>(); }
+// out[o][c] from the S partials P[o][s][c]: 16 columns x 16 threads each per
+// workgroup, a thread taking every sixteenth partial, then a tree in LDS.
+template <typename R, typename To, typename FinF>
+__device__ __forceinline__ void cols_finish_body(const typename R::A *__restrict__ P,
+                                                 To *__restrict__ out, long long inner, int S,
+                                                 FinF fin) {
+  typedef typename R::A A;
+  constexpr int CT = 16, RT = kBlock / CT;
+  __shared__ A part[kBlock];
+  const int ct = threadIdx.x & (CT - 1), rt = threadIdx.x / CT;
+  const long long c = (long long)blockIdx.x * CT + ct, o = blockIdx.y;
+  A v = R::ident();
+  if (c < inner) {
+    const A *p = P + o * S * inner + c;
+    for (int j0 = rt; j0 < S; j0 += RT * kColUnroll) {
+      A q[kColUnroll];
+#pragma unroll
+      for (int u = 0; u < kColUnroll; ++u) {  // past the end: the first one again, not combined
+        const int j = j0 + RT * u;
+        q[u] = p[(long long)(j < S ? j : rt) * inner];
+      }
+#pragma unroll
+      for (int u = 0; u < kColUnroll; ++u)
+        if (j0 + RT * u < S) v = R::comb(v, q[u]);
+    }
+  }
+  part[threadIdx.x] = v;
+  for (int h = RT / 2; h > 0; h >>= 1) {
+    __syncthreads();
+    if (rt < h) part[threadIdx.x] = R::comb(part[threadIdx.x], part[threadIdx.x + h * CT]);
+  }
+  if (rt == 0 && c < inner) out[o * inner + c] = fin(part[threadIdx.x]);
+}
 
-template <typename R, typename T, typename MapF, typename StoreF>
-__device__ __forceinline__ void cols_vec_body(const T *__restrict__ x, long long len,
-                                              long long inner, int S, const ReduceScratch &sc,
-                                              MapF map, StoreF store) {
+template <int OP, typename T, typename To>
+__global__ __launch_bounds__(kBlock) void k_cols_finish(const typename Red<OP, T>::A *__restrict__ P,
+                                                       To *__restrict__ out, long long len,
+                                                       long long inner, int S) {
+  typedef Red<OP, T> R;
+  cols_finish_body<R, To>(P, out, inner, S,
+                          [&](const typename R::A &a) { return finalize<OP, T, To>(a, len); });
+}
+
+template <int OP, typename T>
+__global__ __launch_bounds__(kBlock) void k_argcols_finish(const typename Arg<OP, T>::A *__restrict__ P,
+                                                          long long *__restrict__ out,
+                                                          long long inner, int S) {
+  typedef Arg<OP, T> R;
+  cols_finish_body<R, long long>(P, out, inner, S, [](const typename R::A &a) { return a.i; });
+}
+
+// Strided axis: grid (column blocks, outer, S).  A lane owns VI adjacent
+// columns, one load: 16 bytes (4 of one-byte elements) at element alignment,
+// so rows need not be 16-byte aligned, or one element where the rows are
+// shorter than that.  2^lg lanes lie side by side on a row, as many as the
+// columns fill, and the wave's other lanes on the rows below, so that a wave
+// load covers 64 vectors also where a row has few; a column block is
+// 2^lg x VI columns.  The last lane of a row that VI does not divide reads
+// the row's last VI columns and drops those its neighbour has.  Each wave
+// takes every fourth group of rows of the split, kColUnroll loads in flight;
+// the lanes of a column meet by shuffles, the four waves in LDS in wave
+// order, then the splits' partials are combined in split order.
+// HBM-bound.  float32 sums over axis 0, before (a thread per column unless
+// rows were whole aligned vectors) and now: 2,000,000 x 50 299 -> 76 us
+// (5.3 TB/s), 12,000,000 x 8 1031 -> 69, 100,000 x 999 111 -> 72, 10,000 x
+// 10,001 88 -> 69; float16 300,000 x 333 109 -> 34; 16384^2 unchanged (174,
+// 6.2 TB/s).
+template <typename T> constexpr int col_vec() { return sizeof(T) == 1 ? 4 : 16 / (int)sizeof(T); }
+template <typename T, int VI> struct ColVec {
+  T e[VI];
+};
+
+template <typename R, typename T, int VI, typename MapF, typename StoreF>
+__device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len, long long inner,
+                                          int S, int lg, const ReduceScratch &sc, MapF map,
+                                          StoreF store) {
   typedef typename R::A A;
   constexpr int W = words_of<A>();
-  constexpr int VI = col_vec<T>();
-  constexpr int CW = col_width<T>();
-  constexpr int KC = (CW + kBlock - 1) / kBlock;  // columns per thread in the combine
-  __shared__ A part[kWaves][CW];
+  constexpr int MW = 64 * VI;                     // most columns of a block
+  constexpr int KC = (MW + kBlock - 1) / kBlock;  // columns per thread in the combine
+  __shared__ A part[kWaves][MW];
   __shared__ int is_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int G = 1 << lg, CW = G * VI;
+  const int lc = lane & (G - 1);
   const long long o = blockIdx.y;
   const int s = blockIdx.z;
   const long long c0 = (long long)blockIdx.x * CW;
-  const long long c = c0 + (long long)lane * VI;
+  const long long cn = c0 + (long long)lc * VI;              // first column of this lane
+  const long long c = cn + VI <= inner ? cn : inner - VI;    // first column it loads
   const long long per = (len + S - 1) / S;
   const long long b0 = s * per;
   const long long b1 = b0 + per < len ? b0 + per : len;
+  const long long step = (long long)kWaves << (6 - lg);      // rows per load of the workgroup
   A v[VI];
 #pragma unroll
   for (int e = 0; e < VI; ++e) v[e] = R::ident();
-  if (c < inner) {
+  if (cn < inner) {
     const T *p = x + o * len * inner + c;
-    long long l = b0 + wave;
-    for (; l + (long long)kWaves * (kColUnroll - 1) < b1; l += (long long)kWaves * kColUnroll) {
-      u32x4 q[kColUnroll];
+    long long l = b0 + ((long long)wave << (6 - lg)) + (lane >> lg);
+    if constexpr (VI > 1) {
+      for (; l + step * (kColUnroll - 1) < b1; l += step * kColUnroll) {
+        ColVec<T, VI> q[kColUnroll];
 #pragma unroll
-      for (int u = 0; u < kColUnroll; ++u)
-        q[u] = *reinterpret_cast<const u32x4 *>(p + (l + (long long)kWaves * u) * inner);
+        for (int u = 0; u < kColUnroll; ++u)
+          __builtin_memcpy(&q[u], p + (l + step * u) * inner, sizeof(q[u]));
 #pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) {
-        Pack<T> pk;
-        pk.v = q[u];
+        for (int u = 0; u < kColUnroll; ++u)
 #pragma unroll
-        for (int e = 0; e < VI; ++e) v[e] = R::comb(v[e], map(pk.e[e], l + (long long)kWaves * u));
+          for (int e = 0; e < VI; ++e) v[e] = R::comb(v[e], map(q[u].e[e]));
       }
-    }
-    for (; l < b1; l += kWaves) {
-      Pack<T> pk;
-      pk.v = *reinterpret_cast<const u32x4 *>(p + l * inner);
+      for (; l < b1; l += step) {
+        ColVec<T, VI> q;
+        __builtin_memcpy(&q, p + l * inner, sizeof(q));
 #pragma unroll
-      for (int e = 0; e < VI; ++e) v[e] = R::comb(v[e], map(pk.e[e], l));
+        for (int e = 0; e < VI; ++e) v[e] = R::comb(v[e], map(q.e[e]));
+      }
+    } else {
+      for (; l + step * (kColUnroll - 1) < b1; l += step * kColUnroll) {
+        T q[kColUnroll];
+#pragma unroll
+        for (int u = 0; u < kColUnroll; ++u) q[u] = p[(l + step * u) * inner];
+#pragma unroll
+        for (int u = 0; u < kColUnroll; ++u) v[0] = R::comb(v[0], map(q[u]));
+      }
+      for (; l < b1; l += step) v[0] = R::comb(v[0], map(p[l * inner]));
     }
   }
+  for (int m = G; m < 64; m <<= 1)
 #pragma unroll
-  for (int e = 0; e < VI; ++e) part[wave][lane * VI + e] = v[e];
+    for (int e = 0; e < VI; ++e) v[e] = R::comb(v[e], shfl_xor(v[e], m));
+  if (lane < G && cn < inner)
+#pragma unroll
+    for (int e = 0; e < VI; ++e)
+      if (c + e >= cn) part[wave][c + e - c0] = v[e];
   __syncthreads();
   A acc[KC];
 #pragma unroll
   for (int k = 0; k < KC; ++k) {
     const int cc = threadIdx.x + k * kBlock;
     acc[k] = R::ident();
-    if (cc < CW) {
+    if (cc < CW && c0 + cc < inner) {
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) acc[k] = R::comb(acc[k], part[w][cc]);
     }
@@ -822,6 +872,15 @@ __device__ __forceinline__ void cols_vec_body(const T *__restrict__ x, long long
     for (int k = 0; k < KC; ++k) {
       const int cc = threadIdx.x + k * kBlock;
       if (cc < CW && c0 + cc < inner) store(o * inner + c0 + cc, acc[k]);
+    }
+    return;
+  }
+  if (S > kTaggedSplits) {
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+      const int cc = threadIdx.x + k * kBlock;
+      if (cc < CW && c0 + cc < inner)
+        reinterpret_cast<A *>(sc.words)[(o * S + s) * inner + c0 + cc] = acc[k];
     }
     return;
   }
@@ -852,42 +911,54 @@ __device__ __forceinline__ void cols_vec_body(const T *__restrict__ x, long long
     __hip_atomic_store(sc.tickets + o * ncb + cb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int OP, typename T, typename To>
-__global__ __launch_bounds__(kBlock) void k_reduce_cols_vec(const T *__restrict__ x,
-                                                           To *__restrict__ out, long long len,
-                                                           long long inner, int S,
-                                                           ReduceScratch sc) {
+template <int OP, typename T, typename To, int VI>
+__global__ __launch_bounds__(kBlock) void k_reduce_cols(const T *__restrict__ x, To *__restrict__ out,
+                                                       long long len, long long inner, int S, int lg,
+                                                       ReduceScratch sc) {
   typedef Red<OP, T> R;
-  cols_vec_body<R, T>(
-      x, len, inner, S, sc, [](T q, long long) { return R::map(q); },
+  cols_body<R, T, VI>(
+      x, len, inner, S, lg, sc, [](T q) { return R::map(q); },
       [&](long long i, const typename R::A &a) { out[i] = finalize<OP, T, To>(a, len); });
 }
 
-// Whether a strided reduction can take the column-vector kernel.
-template <typename T> bool cols_vec_ok(long long inner, const void *x) {
-  if (sizeof(T) < 2) return false;  // one-byte types keep the column-per-thread kernels
-  return inner % col_vec<T>() == 0 && ((uintptr_t)x & 15) == 0;
-}
-
 // ------------------------------------------------------------ launch
-// Strided layouts: split the reduced axis so that the launch has about
-// `target` workgroups, each reading at least 64 rows.  Measured on 16384^2
-// float32 over axis 0 (the splits' partials combined in batched loads):
-// the column-vector sum runs best with one workgroup per CU (256: 6.2 TB/s;
-// 128: 5.3, 512: 5.8, 1024: 5.4, 2048: 5.3), the column-per-thread
-// kernels with 1024 (argmax 4.76 TB/s; 512: 3.2, 2048: 4.45).
-#ifndef MMP_COL_TARGET_BLOCKS
-#define MMP_COL_TARGET_BLOCKS 1024
-#endif
-constexpr long long kColVecTargetBlocks = 256;
-constexpr long long kColTargetBlocks = MMP_COL_TARGET_BLOCKS;
-int col_splits(long long col_blocks, long long len, long long target) {
-  long long want = (target + col_blocks - 1) / col_blocks;
-  long long maxs = len / 64 > 0 ? len / 64 : 1;
-  long long s = want < maxs ? want : maxs;
-  if (s < 1) s = 1;
-  if (s > 1024) s = 1024;
-  return (int)s;
+// Strided layouts: the split of the reduced axis that leaves the CUs most
+// evenly loaded, up to `per_cu` workgroups each and at least 64 steps of rows
+// (`steps`: rows over the rows a workgroup's lanes lie on side by side) to a
+// split.  Workgroups of a launch of this size all run together, so what
+// counts is that each CU gets as many: 40 column blocks x 6 splits (240
+// workgroups on 256 CUs) sum 10,000 x 10,001 float32 in 69 us, x 7 (280)
+// in 91.  Measured on 16384^2 float32 over axis 0: the column-vector sum runs
+// best with one workgroup per CU (256: 6.2 TB/s; 128: 5.3, 512: 5.8, 1024:
+// 5.4, 2048: 5.3), the arg kernel with four (argmax 4.76 TB/s; 512: 3.2,
+// 2048: 4.45).
+constexpr int kColVecPerCu = 1, kColPerCu = 4;
+int col_splits(long long col_blocks, long long steps, int per_cu) {
+  const long long cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
+  long long most = steps / 64;
+  if (most > 1024) most = 1024;
+  // enough workgroups already without splitting, or too few rows to split
+  if (col_blocks >= 4 * cus * per_cu || most <= 1) return 1;
+  // up to per_cu per CU; where the column blocks alone are about that many,
+  // a few more, which fill the CUs better
+  long long top = cus * per_cu / col_blocks;
+  if (top < 4) top = 4;
+  if (top > most) top = most;
+  int best = 1;
+  double best_fill = 0.0;
+  for (long long s = top; s >= 1; --s) {
+    const long long wgs = col_blocks * s, per = (wgs + cus - 1) / cus;
+    // the CUs' even share of the busiest one's load, less a little for every
+    // workgroup on it beyond the wanted number
+    double fill = (double)wgs / (double)(per * cus);
+    if (per > per_cu) fill -= 0.02 * (double)(per - per_cu);
+    if (per < per_cu) fill *= 0.5 + 0.5 * (double)per / per_cu;
+    if (fill > best_fill + 1e-9) {
+      best_fill = fill;
+      best = (int)s;
+    }
+  }
+  return best;
 }
 
 int choose_splits(long long rows, long long len) {
@@ -960,10 +1031,13 @@ int launch_reduce(long long outer, long long len, long long inner, const void *x
     return mmpi::check_launch("mmp_reduce(rows)");
   }
   if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided reduction: outer extent %lld > 65535", outer);
-  const bool vec = cols_vec_ok<T>(inner, x);
-  const int cw = vec ? col_width<T>() : kBlock;  // columns per workgroup
+  const bool vec = inner >= col_vec<T>();
+  const int vi = vec ? col_vec<T>() : 1;
+  int lg = 0;  // lanes side by side on a row
+  while (lg < 6 && ((long long)vi << lg) < inner) ++lg;
+  const int cw = vi << lg;  // columns per workgroup
   const long long ncb = mmpi::ceil_div(inner, cw);
-  int S = col_splits(outer * ncb, len, vec ? kColVecTargetBlocks : kColTargetBlocks);
+  int S = col_splits(outer * ncb, len >> (6 - lg), kColVecPerCu);
   if (noalloc) S = noalloc_col_splits<A>(S, outer * ncb, cw);
   if (S > 1) {
     if (int st = noalloc ? noalloc_scratch<A>(outer * ncb * S * cw, outer * ncb, &sc)
@@ -971,16 +1045,18 @@ int launch_reduce(long long outer, long long len, long long inner, const void *x
       return st;
   }
   const dim3 grid((unsigned)ncb, (unsigned)outer, (unsigned)S);
-  if constexpr (sizeof(T) >= 2) {
-    if (vec) {
-      hipLaunchKernelGGL((k_reduce_cols_vec<OP, T, To>), grid, dim3(kBlock), 0, mmpi::stream(),
-                         (const T *)x, (To *)out, len, inner, S, sc);
-      return mmpi::check_launch("mmp_reduce(cols)");
-    }
-  }
-  hipLaunchKernelGGL((k_reduce_cols<OP, T, To>), grid, dim3(kBlock), 0, mmpi::stream(),
-                     (const T *)x, (To *)out, len, inner, S, sc);
-  return mmpi::check_launch("mmp_reduce(cols)");
+  if (vec)
+    hipLaunchKernelGGL((k_reduce_cols<OP, T, To, col_vec<T>()>), grid, dim3(kBlock), 0,
+                       mmpi::stream(), (const T *)x, (To *)out, len, inner, S, lg, sc);
+  else
+    hipLaunchKernelGGL((k_reduce_cols<OP, T, To, 1>), grid, dim3(kBlock), 0, mmpi::stream(),
+                       (const T *)x, (To *)out, len, inner, S, lg, sc);
+  if (int st = mmpi::check_launch("mmp_reduce(cols)")) return st;
+  if (S <= kTaggedSplits) return MMP_OK;
+  hipLaunchKernelGGL((k_cols_finish<OP, T, To>), dim3((unsigned)mmpi::ceil_div(inner, 16),
+                     (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.words,
+                     (To *)out, len, inner, S);
+  return mmpi::check_launch("mmp_reduce(cols finish)");
 }
 
 template <int OP, typename T>
@@ -999,14 +1075,26 @@ int launch_argreduce(long long outer, long long len, long long inner, const void
     return mmpi::check_launch("mmp_argreduce(rows)");
   }
   if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided argreduce: outer extent %lld > 65535", outer);
-  const long long ncb = mmpi::ceil_div(inner, kBlock);
-  const int S = col_splits(outer * ncb, len, kColTargetBlocks);
+  int lc = 0;  // threads side by side on the columns
+  while (lc < 8 && (1LL << lc) < inner) ++lc;
+  const long long ncb = mmpi::ceil_div(inner, 1LL << lc);
+  const int S = col_splits(outer * ncb, len >> (8 - lc), kColPerCu);
   if (S > 1) {
-    if (int st = reduce_scratch<A>(outer * ncb * S * kBlock, outer * ncb, &sc)) return st;
+    if (int st = reduce_scratch<A>((outer * ncb * S) << lc, outer * ncb, &sc)) return st;
   }
-  hipLaunchKernelGGL((k_argreduce_cols<OP, T>), dim3((unsigned)ncb, (unsigned)outer, (unsigned)S),
-                     dim3(kBlock), 0, mmpi::stream(), (const T *)x, out, len, inner, S, sc);
-  return mmpi::check_launch("mmp_argreduce(cols)");
+  const dim3 grid((unsigned)ncb, (unsigned)outer, (unsigned)S);
+  if (lc == 8)
+    hipLaunchKernelGGL((k_argreduce_cols<OP, T, true>), grid, dim3(kBlock), 0, mmpi::stream(),
+                       (const T *)x, out, len, inner, S, lc, sc);
+  else
+    hipLaunchKernelGGL((k_argreduce_cols<OP, T, false>), grid, dim3(kBlock), 0, mmpi::stream(),
+                       (const T *)x, out, len, inner, S, lc, sc);
+  if (int st = mmpi::check_launch("mmp_argreduce(cols)")) return st;
+  if (S <= kTaggedSplits) return MMP_OK;
+  hipLaunchKernelGGL((k_argcols_finish<OP, T>), dim3((unsigned)mmpi::ceil_div(inner, 16),
+                     (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.words, out,
+                     inner, S);
+  return mmpi::check_launch("mmp_argreduce(cols finish)");
 }
 
 // Output dtypes NumPy's rules produce: max/min keep the dtype; sums and
