@@ -398,12 +398,132 @@ def _sign_facts(prog: _Program):
     return facts
 
 
+_FLAT_UNROLL = 4  # 4-element vectors per thread of a flat kernel
+# Outputs a flat launch is worth: smaller ones would be under 16 of its tiles,
+# and the row launch spreads them over more CUs (1000 x 100: 5.6 us a call
+# either way; 30,000 x 8: 14.3 by rows, 5.7 flat).
+_FLAT_MIN = 1 << 16
+
+
+def _flat_kinds(outer, cols, leaf_str, ptrs, itemsizes, out_ptr, out_itemsize, tile):
+    """Leaf classes of a flat launch, or None where the row launch stays.
+
+    The row launch gives every row its own workgroups, so rows shorter than a
+    workgroup's ``tile`` leave most of it idle, and a row length that is no
+    multiple of 4 takes it element by element.  The flat launch cuts the
+    output into tiles whatever its rows: a vector finds its row and column
+    with one 32-bit division (hence fewer than 2^31 elements).  Classes: 'f'
+    follows the output (read as vectors: its pointer and the output's must be
+    aligned); where rows are whole aligned vectors, a row vector repeated down
+    the rows is read as vectors ('q'), so are rows lying further apart ('v'),
+    and a value per row once per vector ('w'); else by element ('p', 'r', and
+    'g' for any other strides, whose loads are spread too wide to take long
+    rows flat).  (x - m) / d of a
+    2,000,000 x 50 float32 x and row vectors m, d: 655 us by rows,
+    134 flat (6 TB/s); 12,000,000 x 8: 4965 and 126; 10,000 x 10,001: 182 and
+    140."""
+    if len(outer) != 1 or (cols >= tile and cols % _ELEMS == 0):
+        return None
+    if not _FLAT_MIN <= outer[0] * cols < 1 << 31 or out_ptr % (_ELEMS * out_itemsize):
+        return None
+    whole = cols % _ELEMS == 0
+    kinds = []
+    for (row_st, col_st), ptr, isz in zip(leaf_str, ptrs, itemsizes):
+        aligned = ptr % (_ELEMS * isz) == 0
+        if row_st == cols and col_st == 1 and aligned:
+            kinds.append("f")
+        elif row_st == 0 and col_st == 1:
+            kinds.append("q" if whole and aligned else "p")
+        elif col_st == 0:
+            kinds.append("w" if whole else "r")
+        elif col_st == 1 and whole and aligned and row_st % _ELEMS == 0:
+            kinds.append("v")
+        elif cols < _BLOCK:
+            kinds.append("g")
+        else:
+            return None
+    return kinds
+
+
+def _flat_body(kinds, ct, vtypes, out_ct, expr_lines, res):
+    """Body of a flat kernel (see _flat_kinds) after the leaf and scalar
+    declarations."""
+    tile = _FLAT_UNROLL * _BLOCK * _ELEMS
+    L = []
+    L.append("  const unsigned n = (unsigned)p.n, cols = (unsigned)p.cols;")
+    for k, kind in enumerate(kinds):
+        if kind in "rwgv":
+            L.append(f"  const long long rs{k} = p.ostride[{k}];")
+        if kind == "g":
+            L.append(f"  const long long cs{k} = p.lstride[{k}];")
+
+    def at(k):
+        """Leaf k at (row, col)."""
+        return {"p": f"in{k}[col]", "q": f"in{k}[col]", "r": f"in{k}[(long long)row * rs{k}]",
+                "w": f"in{k}[(long long)row * rs{k}]",
+                "v": f"in{k}[(long long)row * rs{k} + col]",
+                "g": f"in{k}[(long long)row * rs{k} + (long long)col * cs{k}]"}[kinds[k]]
+
+    L.append(f"  const unsigned i0 = blockIdx.x * {tile}u;")
+    L.append(f"  if (n - i0 >= {tile}u) {{")
+    for k, kind in enumerate(kinds):
+        if kind == "f":
+            L.append(f"    {vtypes[ct[k]]} l{k}[{_FLAT_UNROLL}];")
+    L.append(f"    #pragma unroll\n    for (int u = 0; u < {_FLAT_UNROLL}; ++u) {{")
+    L.append(f"      const unsigned i = i0 + (u * {_BLOCK} + threadIdx.x) * {_ELEMS};")
+    for k, kind in enumerate(kinds):
+        if kind == "f":
+            L.append(f"      l{k}[u] = __builtin_nontemporal_load((const {vtypes[ct[k]]}*)(in{k} + i));")
+    L.append("    }")
+    L.append(f"    #pragma unroll\n    for (int u = 0; u < {_FLAT_UNROLL}; ++u) {{")
+    L.append(f"      const unsigned i = i0 + (u * {_BLOCK} + threadIdx.x) * {_ELEMS};")
+    L.append("      unsigned row = i / cols, col = i - row * cols;")
+    for k, kind in enumerate(kinds):
+        if kind in "qv":
+            L.append(f"      const {vtypes[ct[k]]} l{k} = *(const {vtypes[ct[k]]}*)&{at(k)};")
+        elif kind == "w":
+            L.append(f"      const {ct[k]} l{k} = {at(k)};")
+        elif kind != "f":
+            L.append(f"      {ct[k]} l{k}[{_ELEMS}];")
+    if any(kind in "prg" for kind in kinds):
+        # the elements' loads ahead of the arithmetic
+        L.append(f"      #pragma unroll\n      for (int e = 0; e < {_ELEMS}; ++e) {{")
+        for k, kind in enumerate(kinds):
+            if kind in "prg":
+                L.append(f"        l{k}[e] = {at(k)};")
+        L.append("        if (++col == cols) { col = 0; ++row; }")
+        L.append("      }")
+    L.append(f"      {vtypes[out_ct]} o;")
+    L.append(f"      #pragma unroll\n      for (int e = 0; e < {_ELEMS}; ++e) {{")
+
+    def elem(k):
+        if kinds[k] == "f":
+            return f"({ct[k]})l{k}[u][e]"
+        return f"l{k}" if kinds[k] == "w" else f"({ct[k]})l{k}[e]"
+    L.extend(expr_lines(elem, "        "))
+    L.append(f"        o[e] = {res};")
+    L.append("      }")
+    L.append(f"      __builtin_nontemporal_store(o, ({vtypes[out_ct]}*)(({out_ct}*)p.outp + i));")
+    L.append("    }")
+    L.append("    return;")
+    L.append("  }")
+    L.append(f"  for (unsigned i = i0 + threadIdx.x; i < n; i += {_BLOCK}) {{")
+    L.append("    const unsigned row = i / cols, col = i - row * cols;")
+    L.extend(expr_lines(lambda k: f"in{k}[i]" if kinds[k] == "f" else at(k), "    "))
+    L.append(f"    (({out_ct}*)p.outp)[i] = {res};")
+    L.append("  }")
+    L.append("}")
+    return L
+
+
 def generate_source(prog: _Program, kinds, nouter, out_dtype, vec, mode, fast=False):
     """HIP source for ``prog``.
 
     kinds[k]: last-dim stride class of array leaf k ('c' unit, 'b' zero,
     's' general).  nouter: number of outer (row) dims (0 = 1-D launch).
-    mode: 'map' (elementwise, contiguous output), 'sum' (row-sum epilogue).
+    mode: 'map' (elementwise, contiguous output), 'flat' (the same over the
+    flat index, for rows too short or too odd to be a workgroup's: kinds as
+    _flat_kinds gives them), 'sum' (row-sum epilogue).
     fast: use the fast_math forms of the transcendentals.
     """
     nin, nsc = len(prog.arrays), len(prog.scalars)
@@ -418,7 +538,7 @@ def generate_source(prog: _Program, kinds, nouter, out_dtype, vec, mode, fast=Fa
     # vector types for the vectorised path
     vtypes = {}
     if vec:
-        for t in set(ct + ([out_ct] if mode == "map" else [])):
+        for t in set(ct + ([out_ct] if mode != "sum" else [])):
             vt = "v4_" + t.replace(" ", "_")
             st = "unsigned char" if t == "bool" else t
             vtypes[t] = vt
@@ -465,6 +585,9 @@ def generate_source(prog: _Program, kinds, nouter, out_dtype, vec, mode, fast=Fa
             L.append(f"  const bool s{j} = (p.sbits[{j}] & 1ull) != 0;")
         else:
             L.append(f"  const {t} s{j} = __builtin_bit_cast({t}, ({bt})p.sbits[{j}]);")
+    if mode == "flat":
+        L.extend(_flat_body(kinds, ct, vtypes, out_ct, expr_lines, f"t{prog.result}"))
+        return "\n".join(L) + "\n"
     # row setup
     if nouter == 0:
         L.append("  const long long row = 0; const long long cb = blockIdx.x;")
@@ -725,9 +848,19 @@ def run_map(root: FusionNode, out_buffer, out_ptr: int) -> None:
     shape = root._shape
     cshape, outer, cols, leaf_str, kinds = _plan(prog, shape, keep_last=False)
     out_dtype = root._dtype
+    tile = _map_tile(kinds)
+    flat = _flat_kinds(outer, cols, leaf_str, [_leaf_ptr(a) for a in prog.arrays],
+                       [a._dtype.itemsize for a in prog.arrays], out_ptr, out_dtype.itemsize, tile)
+    if flat is not None:
+        kern = _kernel_for_program(prog, flat, 1, out_dtype, True, "flat")
+        P = _param_struct(len(prog.arrays), len(prog.scalars), 1)
+        p, rows = _fill_params(prog, P, outer, cols, leaf_str, out_ptr, 1, 1.0)
+        nblocks = -(-rows * cols // (_FLAT_UNROLL * _BLOCK * _ELEMS))
+        if nblocks:
+            HipBackend().launch(kern, (nblocks, 1, 1), (_BLOCK, 1, 1), [p])
+        return
     vec = _vec_ok(prog, kinds, leaf_str, outer, cols, out_ptr, out_dtype.itemsize, "map")
     kern = _kernel_for_program(prog, kinds, len(outer), out_dtype, vec, "map")
-    tile = _map_tile(kinds)
     colblocks = -(-cols // tile)
     P = _param_struct(len(prog.arrays), len(prog.scalars), len(outer))
     p, rows = _fill_params(prog, P, outer, cols, leaf_str, out_ptr, colblocks, 1.0)
@@ -833,8 +966,8 @@ def materialize_node(node: FusionNode, out_ptr: int) -> None:
 
 
 def compile_for_native(root, kinds, nouter, out_dtype, vec, mode="map") -> int:
-    """Kernel handle of the generated kernel for ``root`` ('map' or 'sum'
-    mode) with the iteration plan the native gate computed (leaf stride
+    """Kernel handle of the generated kernel for ``root`` ('map', 'flat' or
+    'sum' mode) with the iteration plan the native gate computed (leaf stride
     classes ``kinds``, ``nouter`` outer dims, output dtype, vector flag);
     the DAG is linearised here in the same order as there."""
     prog = _Program(root)

@@ -1118,6 +1118,11 @@ long long map_tile(const std::string &kinds) {
   return kinds == "c" ? 256 * 4 * 1 : 256 * 4 * 4;
 }
 
+// The flat launch's leaf classes (the Python _flat_kinds, which says what they
+// are and when a launch is flat), or false where the row launch stays.
+constexpr long long kFlatTile = 256 * 4 * 4, kFlatMin = 1 << 16;
+bool flat_kinds(const Plan &pl, unsigned long long outp, int out_dt, std::string *kinds);
+
 // 1 = planned, 0 = not handled here (fall back), -1 = error set.
 int make_plan(PyObject *root, PyObject *shape, bool keep_last, Plan *pl) {
   Prog &p = pl->p;
@@ -1180,8 +1185,27 @@ bool vec_ok(const Plan &pl, bool out_ok) {
   return true;
 }
 
-// Kernel for the plan (mode 'm' map, 's' row sum), by structure; compiled
-// through the Python code generator the first time.
+bool flat_kinds(const Plan &pl, unsigned long long outp, int out_dt, std::string *kinds) {
+  if (pl.nouter != 1 || (pl.cols >= map_tile(pl.kinds) && pl.cols % 4 == 0)) return false;
+  const long long n = pl.rows * pl.cols;
+  if (n < kFlatMin || n >= (1LL << 31) || outp % (4ull * itemsize[out_dt])) return false;
+  const bool whole = pl.cols % 4 == 0;
+  kinds->clear();
+  for (size_t k = 0; k < pl.p.leaves.size(); ++k) {
+    const long long row = pl.cst[k][0], col = pl.cst[k][1];
+    const bool aligned = pl.p.leaves[k].ptr % (4ull * itemsize[pl.p.leaves[k].dt]) == 0;
+    if (row == pl.cols && col == 1 && aligned) kinds->push_back('f');
+    else if (row == 0 && col == 1) kinds->push_back(whole && aligned ? 'q' : 'p');
+    else if (col == 0) kinds->push_back(whole ? 'w' : 'r');
+    else if (col == 1 && whole && aligned && row % 4 == 0) kinds->push_back('v');
+    else if (pl.cols < kBlock) kinds->push_back('g');
+    else return false;
+  }
+  return true;
+}
+
+// Kernel for the plan (mode 'm' map, 'f' flat map, 's' row sum), by structure;
+// compiled through the Python code generator the first time.
 void *kernel_for(const Plan &pl, PyObject *root, int out_dt, bool vec, char mode, bool fast) {
   std::string key = pl.p.key;
   key.push_back('|');
@@ -1197,7 +1221,7 @@ void *kernel_for(const Plan &pl, PyObject *root, int out_dt, bool vec, char mode
   PyObject *kt = PyUnicode_FromStringAndSize(pl.kinds.data(), (Py_ssize_t)pl.kinds.size());
   PyObject *r = kt ? PyObject_CallFunction(py_compile_map, "OOiOOs", root, kt, (int)pl.nouter,
                                            dtypes[out_dt], vec ? Py_True : Py_False,
-                                           mode == 'm' ? "map" : "sum")
+                                           mode == 'm' ? "map" : mode == 'f' ? "flat" : "sum")
                    : nullptr;
   Py_XDECREF(kt);
   if (!r) return nullptr;
@@ -1214,10 +1238,10 @@ void *kernel_for(const Plan &pl, PyObject *root, int out_dt, bool vec, char mode
 
 // Pack the generated kernel's parameter block (struct P: 8-byte fields
 // ptr[nin], outp, sbits[nsc], n, rows, cols, colblocks, oshape[nouter],
-// ostride[nin * nouter], lstride[nin], scale) and launch rows * colblocks
-// workgroups of kBlock threads.  0 or -1 with an exception set.
+// ostride[nin * nouter], lstride[nin], scale) and launch `blocks` workgroups
+// of kBlock threads.  0 or -1 with an exception set.
 int launch_plan(const Plan &pl, void *kern, unsigned long long outp, long long colblocks,
-                double scale) {
+                double scale, long long blocks) {
   const size_t nin = pl.p.leaves.size(), nsc = pl.p.sbits.size(), nouter = pl.nouter;
   const size_t nin1 = nin ? nin : 1, nsc1 = nsc ? nsc : 1, nout1 = nouter ? nouter : 1,
                nio1 = (nin * nouter) != 0 ? nin * nouter : 1;
@@ -1244,7 +1268,7 @@ int launch_plan(const Plan &pl, void *kern, unsigned long long outp, long long c
   P[o_n + 2] = (unsigned long long)pl.cols;
   P[o_n + 3] = (unsigned long long)colblocks;
   std::memcpy(&P[o_scale], &scale, 8);
-  const unsigned long long nblocks = (unsigned long long)(pl.rows * colblocks);
+  const unsigned long long nblocks = (unsigned long long)blocks;
   if (nblocks * kBlock > 0xffffffffull) {  // HIP's limit on work-items per grid dimension
     PyErr_SetString(PyExc_ValueError, "fused launch too large");
     return -1;
@@ -1351,12 +1375,20 @@ PyObject *gate_materialize(PyObject *, PyObject *arr) {
     buf = new_devbuf(n * itemsize[odt]);
     if (!buf) goto fail;
     const unsigned long long outp = ((DevBuf *)buf)->ptr;
-    const bool vec = vec_ok(pl, outp % (4ull * itemsize[odt]) == 0);
-    void *kern = kernel_for(pl, node, odt, vec, 'm', fast);
-    if (!kern) goto fail;
     const long long tile = map_tile(pl.kinds);
-    const long long colblocks = (pl.cols + tile - 1) / tile;
-    if (launch_plan(pl, kern, outp, colblocks, 1.0)) goto fail;
+    std::string flat;
+    if (flat_kinds(pl, outp, odt, &flat)) {
+      pl.kinds = flat;
+      void *kern = kernel_for(pl, node, odt, true, 'f', fast);
+      if (!kern) goto fail;
+      if (launch_plan(pl, kern, outp, 1, 1.0, (pl.rows * pl.cols + kFlatTile - 1) / kFlatTile)) goto fail;
+    } else {
+      const bool vec = vec_ok(pl, outp % (4ull * itemsize[odt]) == 0);
+      void *kern = kernel_for(pl, node, odt, vec, 'm', fast);
+      if (!kern) goto fail;
+      const long long colblocks = (pl.cols + tile - 1) / tile;
+      if (launch_plan(pl, kern, outp, colblocks, 1.0, pl.rows * colblocks)) goto fail;
+    }
     result = Py_None;
   }
   if (finish(arr, arrd, buf, shape)) goto fail;
@@ -1426,14 +1458,14 @@ PyObject *gate_run_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   void *kern = kernel_for(pl, root, final_direct ? odt : acc, vec, 's', cfg_flag(s_fast_math));
   if (!kern) return nullptr;
   if (final_direct) {
-    if (launch_plan(pl, kern, out_ptr, 1, scale)) return nullptr;
+    if (launch_plan(pl, kern, out_ptr, 1, scale, pl.rows)) return nullptr;
     ++stat_native_mat;
     Py_RETURN_NONE;
   }
   PyObject *part = new_devbuf(pl.rows * colblocks * 8);
   if (!part) return nullptr;
   const unsigned long long pp = ((DevBuf *)part)->ptr;
-  if (launch_plan(pl, kern, pp, colblocks, scale)) {
+  if (launch_plan(pl, kern, pp, colblocks, scale, pl.rows * colblocks)) {
     Py_DECREF(part);
     return nullptr;
   }

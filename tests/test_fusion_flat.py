@@ -1,0 +1,133 @@
+"""The flat launch of fused expressions (rows too short or too odd to be a
+workgroup's): its leaf classes and generated source on the CPU, and its
+results on the GPU against NumPy and the op-by-op evaluation."""
+import itertools
+
+import numpy as np
+import pytest
+
+import macmetalpy_amd as cp
+from macmetalpy_amd import _fusion as F
+from macmetalpy_amd._backend import DeviceBuffer, rtc_build
+
+
+def _leaf(shape, dtype, strides, ptr):
+    return F.InputNode(DeviceBuffer(ptr, 0, owned=False), shape, dtype, strides)
+
+
+def _plan(leaves, shape, dtype=np.float32):
+    root = leaves[0]
+    for x in leaves[1:]:
+        root = F.BinaryOpNode("add_op", root, x, shape, dtype)
+    prog = F._Program(root)
+    cshape, outer, cols, leaf_str, kinds = F._plan(prog, shape, False)
+    flat = F._flat_kinds(outer, cols, leaf_str, [F._leaf_ptr(a) for a in prog.arrays],
+                         [a._dtype.itemsize for a in prog.arrays], 0x20000, 4, F._map_tile(kinds))
+    return prog, outer, cols, leaf_str, flat
+
+
+# (strides of a leaf over (rows, cols), rows x cols -> its class or None)
+def _strides(cols):
+    return {"full": (cols, 1), "row": (0, 1), "column": (1, 0), "columns": (5, 0),
+            "padded": (cols + 4, 1), "odd pad": (cols + 3, 1), "transposed": (1, 7),
+            "stepped": (2 * cols, 2), "reversed": (cols, -1), "one": (0, 0)}
+
+
+@pytest.mark.parametrize("cols", [1, 2, 3, 4, 7, 50, 64, 255, 256, 257, 1000, 4095, 4096, 4097, 8192])
+def test_leaf_classes_address_every_element(cols):
+    """Each class stands for the leaf's own strides, vectors are aligned, and
+    rows of whole tiles (or too long for spread loads) stay with the row
+    launch."""
+    rows = 70000
+    for name, st in _strides(cols).items():
+        for ptr in (0x10000, 0x10004):
+            x = _leaf((rows, cols), np.float32, (cols, 1), 0x40000)
+            y = _leaf((rows, cols), np.float32, st, ptr)
+            _, outer, c, leaf_str, flat = _plan([x, y], (rows, cols))
+            if len(outer) != 1:
+                assert flat is None  # both contiguous: one flat row already
+                continue
+            if c % 4 == 0 and c >= 4096:
+                assert flat is None
+                continue
+            if flat is None:
+                assert c >= 256
+                continue
+            (rs, cs), kind = leaf_str[1], flat[1]
+            want = {"f": (c, 1), "q": (0, 1), "p": (0, 1), "w": (rs, 0), "r": (rs, 0),
+                    "v": (rs, 1), "g": (rs, cs)}[kind]
+            assert (rs, cs) == want, (name, kind)
+            if kind in "fqv":
+                assert ptr % 16 == 0
+            if kind in "qwv":
+                assert c % 4 == 0
+            if kind == "v":
+                assert rs % 4 == 0
+    big = _leaf((1 << 21, 1024), np.float32, (1024, 1), 0x40000)
+    row = _leaf((1 << 21, 1024), np.float32, (0, 1), 0x10000)
+    assert _plan([big, row], (1 << 21, 1024))[-1] is None  # 2^31 elements
+    small = _leaf((600, 100), np.float32, (100, 1), 0x40000)
+    srow = _leaf((600, 100), np.float32, (0, 1), 0x10000)
+    assert _plan([small, srow], (600, 100))[-1] is None  # under 2^16 elements
+
+
+@pytest.mark.parametrize("out", [np.float32, np.float16, np.float64, np.bool_, np.int64])
+def test_flat_source_compiles(out):
+    kinds = ["f", "p", "q", "r", "w", "v", "g"]
+    leaves = [_leaf((9, 8), out, (8, 1), 0x1000 * (k + 1)) for k in range(7)]
+    root = leaves[0]
+    for x in leaves[1:]:
+        root = F.BinaryOpNode("max_op" if out != np.bool_ else "bit_or_op", root, x, (9, 8), out)
+    src = F.generate_source(F._Program(root), kinds, 1, np.dtype(out), True, "flat")
+    assert rtc_build(src, F.RTC_OPTIONS)[:4] == b"\x7fELF"
+
+
+def _same(got, want):
+    assert got.dtype == want.dtype and got.shape == want.shape
+    assert np.array_equal(got, want, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("cols", [1, 2, 3, 4, 5, 8, 50, 63, 255, 257, 1000, 1001, 4097])
+def test_flat_matches_numpy(cols, native):
+    """Row vectors, one value per row, padded and odd rows, transposed and
+    reversed leaves; few rows (row launch), and outputs that end inside, at
+    and past a tile (flat launch)."""
+    g = np.random.default_rng(cols)
+    cp.set_config(native_dispatch=native)
+    try:
+        for rows in (1, 5, 65535 // cols + 1, 69632 // cols + 1, 90000 // cols + 3):
+            x = g.standard_normal((rows, cols), dtype=np.float32)
+            wide = g.standard_normal((rows, cols + 4), dtype=np.float32)
+            r, c = g.standard_normal(cols, dtype=np.float32), g.standard_normal((rows, 1),
+                                                                                dtype=np.float32)
+            t = g.standard_normal((cols, rows), dtype=np.float32)
+            i = g.integers(-9, 9, (rows, cols)).astype(np.int32)
+            dx, dwide, dr, dc, dt, di = (cp.array(a) for a in (x, wide, r, c, t, i))
+            print("flat", rows, cols, flush=True)
+            _same(((dx - dr) / dr).get(), (x - r) / r)
+            _same(((dx - dc) * dr).get(), (x - c) * r)
+            _same((dx * dwide[:, :cols] - dr).get(), x * wide[:, :cols] - r)
+            _same((dx * dwide[:, 3:3 + cols] - dc).get(), x * wide[:, 3:3 + cols] - c)
+            _same((dx + dt.T - dr).get(), x + t.T - r)
+            _same((dx[:, ::-1] * dr + dc).get(), x[:, ::-1] * r + c)
+            _same((dr + dc).get(), r + c)
+            _same((di * di[:1] + dc).get(), i * i[:1] + c)
+            _same((dx > dr).get(), x > r)
+            _same(cp.where(di > di[:, :1], dx, dr).get(), np.where(i > i[:, :1], x, r))
+    finally:
+        cp.set_config(native_dispatch=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float16, np.float64, np.int16, np.int64, np.bool_])
+def test_flat_element_types(dtype):
+    g = np.random.default_rng(5)
+    for rows, cols in itertools.product((3, 20001), (6, 33, 48)):
+        x, r, c = ((g.integers(0, 2, s) if dtype == np.bool_ else g.integers(-50, 50, s)).astype(dtype)
+                   for s in ((rows, cols), (cols,), (rows, 1)))
+        dx, dr, dc = cp.array(x), cp.array(r), cp.array(c)
+        _same(cp.maximum(cp.maximum(dx, dr), dc).get() if dtype != np.bool_ else ((dx | dr) & dc).get(),
+              np.maximum(np.maximum(x, r), c) if dtype != np.bool_ else (x | r) & c)
+        _same((dx == dr).get(), x == r)
