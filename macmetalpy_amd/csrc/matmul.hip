@@ -1227,10 +1227,12 @@ int launch_general(long long batch, int M, int N, int K, const T *A, long long l
   constexpr int V = 16 / sizeof(T), BK = 128 / sizeof(T);
   // partial products need scratch memory: none while the stream is captured
   // (a graph's replays would outlive it)
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const bool may_split = !sub && hipStreamIsCapturing(mmpi::stream(), &cap) == hipSuccess &&
-                         cap == hipStreamCaptureStatusNone;
-  Plan4 pl = plan4(batch, M, N, K, (int)sizeof(T), may_split);
+  Plan4 pl = plan4(batch, M, N, K, (int)sizeof(T), !sub);
+  if (pl.splits > 1) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(mmpi::stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+      pl = plan4(batch, M, N, K, (int)sizeof(T), false);
+  }
   const int nk = (K + BK - 1) / BK;
   const int kspan = (nk + pl.splits - 1) / pl.splits;
   const int splits = (nk + kspan - 1) / kspan;

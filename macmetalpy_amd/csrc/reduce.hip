@@ -621,14 +621,15 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_rows(const T *__restrict__
     out[row] = total.i;
 }
 
-// Partials of a strided reduction: up to kTaggedSplits are combined by the
-// last workgroup to arrive; more are left in the scratch words as they are,
-// (outer, split, column), for a second kernel (k_cols_finish) whose many
-// workgroups read them side by side.  One workgroup alone reading 256
+// Partials of a strided reduction: few are combined by the last workgroup to
+// arrive; more (`plain`) are left in the scratch words as they are, (outer,
+// split, column), for a second kernel (k_cols_finish) whose many workgroups
+// read them side by side.  One workgroup alone reading 256
 // partials a column took longer than the reduction of a 2,000,000 x 50 matrix
-// (float32 sum over axis 0 98 us, against 76 with the second kernel); of 31,
-// it is faster than a second launch (2000 x 300 8.6 us against 11.7).
-constexpr int kTaggedSplits = 64;
+// (float32 sum over axis 0 98 us, against 76 with the second kernel), and 25
+// a column cost a 10,000 x 10,001 argmax 20 us more; but 31 of a 2000 x 300
+// matrix are done sooner than a second launch (8.6 us against 11.7).
+bool plain_partials(int S, long long bytes) { return S > 64 || (S > 16 && bytes >= (32LL << 20)); }
 
 // Strided arg-reduction: grid (ceil(inner / 2^lc), outer, S); 2^lc threads
 // side by side on the columns (as many as there are, up to the workgroup) and
@@ -640,7 +641,7 @@ template <int OP, typename T, bool WIDE>  // WIDE: lc == 8, known at compile tim
 __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__ x,
                                                           long long *__restrict__ out,
                                                           long long len, long long inner, int S,
-                                                          int lc, ReduceScratch sc) {
+                                                          int lc, bool plain, ReduceScratch sc) {
   typedef Arg<OP, T> R;
   typedef typename R::A A;
   typedef typename mmp_t<T>::C C;
@@ -696,7 +697,7 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__
     if (owner) out[o * inner + c] = v.i;
     return;
   }
-  if (S > kTaggedSplits) {
+  if (plain) {
     if (owner) reinterpret_cast<A *>(sc.words)[(o * S + s) * inner + c] = v;
     return;
   }
@@ -795,7 +796,7 @@ template <typename T, int VI> struct ColVec {
 
 template <typename R, typename T, int VI, typename MapF, typename StoreF>
 __device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len, long long inner,
-                                          int S, int lg, const ReduceScratch &sc, MapF map,
+                                          int S, int lg, bool plain, const ReduceScratch &sc, MapF map,
                                           StoreF store) {
   typedef typename R::A A;
   constexpr int W = words_of<A>();
@@ -875,7 +876,7 @@ __device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len
     }
     return;
   }
-  if (S > kTaggedSplits) {
+  if (plain) {
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
       const int cc = threadIdx.x + k * kBlock;
@@ -914,10 +915,10 @@ __device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len
 template <int OP, typename T, typename To, int VI>
 __global__ __launch_bounds__(kBlock) void k_reduce_cols(const T *__restrict__ x, To *__restrict__ out,
                                                        long long len, long long inner, int S, int lg,
-                                                       ReduceScratch sc) {
+                                                       bool plain, ReduceScratch sc) {
   typedef Red<OP, T> R;
   cols_body<R, T, VI>(
-      x, len, inner, S, lg, sc, [](T q) { return R::map(q); },
+      x, len, inner, S, lg, plain, sc, [](T q) { return R::map(q); },
       [&](long long i, const typename R::A &a) { out[i] = finalize<OP, T, To>(a, len); });
 }
 
@@ -1044,15 +1045,16 @@ int launch_reduce(long long outer, long long len, long long inner, const void *x
                          : reduce_scratch<A>(outer * ncb * S * cw, outer * ncb, &sc))
       return st;
   }
+  const bool plain = plain_partials(S, outer * len * inner * (long long)sizeof(T));
   const dim3 grid((unsigned)ncb, (unsigned)outer, (unsigned)S);
   if (vec)
     hipLaunchKernelGGL((k_reduce_cols<OP, T, To, col_vec<T>()>), grid, dim3(kBlock), 0,
-                       mmpi::stream(), (const T *)x, (To *)out, len, inner, S, lg, sc);
+                       mmpi::stream(), (const T *)x, (To *)out, len, inner, S, lg, plain, sc);
   else
     hipLaunchKernelGGL((k_reduce_cols<OP, T, To, 1>), grid, dim3(kBlock), 0, mmpi::stream(),
-                       (const T *)x, (To *)out, len, inner, S, lg, sc);
+                       (const T *)x, (To *)out, len, inner, S, lg, plain, sc);
   if (int st = mmpi::check_launch("mmp_reduce(cols)")) return st;
-  if (S <= kTaggedSplits) return MMP_OK;
+  if (!plain) return MMP_OK;
   hipLaunchKernelGGL((k_cols_finish<OP, T, To>), dim3((unsigned)mmpi::ceil_div(inner, 16),
                      (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.words,
                      (To *)out, len, inner, S);
@@ -1082,15 +1084,16 @@ int launch_argreduce(long long outer, long long len, long long inner, const void
   if (S > 1) {
     if (int st = reduce_scratch<A>((outer * ncb * S) << lc, outer * ncb, &sc)) return st;
   }
+  const bool plain = plain_partials(S, outer * len * inner * (long long)sizeof(T));
   const dim3 grid((unsigned)ncb, (unsigned)outer, (unsigned)S);
   if (lc == 8)
     hipLaunchKernelGGL((k_argreduce_cols<OP, T, true>), grid, dim3(kBlock), 0, mmpi::stream(),
-                       (const T *)x, out, len, inner, S, lc, sc);
+                       (const T *)x, out, len, inner, S, lc, plain, sc);
   else
     hipLaunchKernelGGL((k_argreduce_cols<OP, T, false>), grid, dim3(kBlock), 0, mmpi::stream(),
-                       (const T *)x, out, len, inner, S, lc, sc);
+                       (const T *)x, out, len, inner, S, lc, plain, sc);
   if (int st = mmpi::check_launch("mmp_argreduce(cols)")) return st;
-  if (S <= kTaggedSplits) return MMP_OK;
+  if (!plain) return MMP_OK;
   hipLaunchKernelGGL((k_argcols_finish<OP, T>), dim3((unsigned)mmpi::ceil_div(inner, 16),
                      (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.words, out,
                      inner, S);

@@ -96,11 +96,13 @@ def matmul(x1, x2, out=None, **kwargs):
         A = A.astype(rdt)
     if B._dtype != rdt:
         B = B.astype(rdt)
-    A._ensure_gpu()
-    B._ensure_gpu()
     pa = pb = None
-    if rdt == np.float64 or (rdt == np.float32 and not _copy_kernel_shape(M, N, K, batch)):
-        pa, pb = _in_place(A, batch_shape), _in_place(B, batch_shape)
+    if rdt.kind == "f" and rdt.itemsize > 2 and not (A._is_device_contiguous()
+                                                     and B._is_device_contiguous()):
+        A._ensure_gpu()
+        B._ensure_gpu()
+        if rdt.itemsize == 8 or not _copy_kernel_shape(M, N, K, batch):
+            pa, pb = _in_place(A, batch_shape), _in_place(B, batch_shape)
     if pa is None:
         A, sA = _batch_operand(A, batch_shape, (M, K))
         pa = False, K, sA
