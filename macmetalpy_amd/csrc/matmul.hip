@@ -1374,6 +1374,16 @@ int matmul(int dtype, int ta, int tb, int64_t batch, int64_t M, int64_t N, int64
 
 }  // namespace
 
+namespace mmpi {
+int matmul_sub(int dtype, long long batch, int M, int N, int K, const void *A, long long lda,
+               long long sA, const void *B, long long ldb, long long sB, void *C, long long ldc,
+               long long sC) {
+  if (dtype == MMP_F32)
+    return launch4<float>(0, 0, batch, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, true);
+  return launch4<double>(0, 0, batch, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, true);
+}
+}  // namespace mmpi
+
 extern "C" int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, const void *A,
                           int64_t lda, int64_t sA, const void *B, int64_t ldb, int64_t sB, void *C,
                           int64_t ldc, int64_t sC) {

@@ -75,6 +75,11 @@ struct WaitParams {
 };
 WaitParams wait_params();
 
+// C[b] -= A[b] @ B[b] in place (float32, float64; row-major as mmp_matmul).
+int matmul_sub(int dtype, long long batch, int M, int N, int K, const void *A, long long lda,
+               long long sA, const void *B, long long ldb, long long sB, void *C, long long ldc,
+               long long sC);
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 }  // namespace mmpi
