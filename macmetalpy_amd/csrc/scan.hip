@@ -352,8 +352,8 @@ __device__ typename S::A look_back(const ScanScratch &sc, long long tile, long l
   return prefix;
 }
 
-// Prefix for a row's tail (MODE 2): the inclusive descriptor of the row's
-// last whole tile, published by the preceding launch on the same stream.
+// Prefix for a row's tail: the inclusive descriptor of the row's last whole
+// tile, published by the preceding launch on the same stream.
 template <typename S>
 __device__ typename S::A tail_prefix(const ScanScratch &sc, long long pred, unsigned gen) {
   const unsigned long long w0 = __hip_atomic_load(sc.desc + 2 * pred, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -368,9 +368,6 @@ __device__ typename S::A tail_prefix(const ScanScratch &sc, long long pred, unsi
 //         row), guard-free streaming body, look-back.
 // MODE 1: any layout (grid = rows x ceil tiles per row), guarded body,
 //         look-back.
-// MODE 2: the partial last tile of each row after a MODE 0 launch (grid =
-//         rows); its prefix is the inclusive descriptor MODE 0 published for
-//         the row's last whole tile.
 // MODE 0 is compiled for at least two workgroups per CU (measured best:
 // more concurrent tiles lengthen every look-back); keeping the guarded
 // paths out of it keeps its registers down.
@@ -393,11 +390,9 @@ __global__ __launch_bounds__(kBlock, MODE == 0 ? 2 : 1) void k_scan_rows(
   To *sy = reinterpret_cast<To *>(stage);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
-  // tile = workgroup id (rows x tiles per row, row-major); MODE 2: the
-  // row's tail, one past its last whole tile
-  const long long tile = MODE == 2 ? (long long)blockIdx.x * tiles_per_row + tiles_per_row
-                                   : (long long)blockIdx.x;
-  const long long row = MODE == 2 ? (long long)blockIdx.x : tile / tiles_per_row;
+  // tile = workgroup id (rows x tiles per row, row-major)
+  const long long tile = blockIdx.x;
+  const long long row = tile / tiles_per_row;
   const long long t = tile - row * tiles_per_row;
   const long long base = t * kTile;
   const long long rem = len - base;
@@ -493,9 +488,7 @@ __global__ __launch_bounds__(kBlock, MODE == 0 ? 2 : 1) void k_scan_rows(
     }
 
     // 3. look-back (wave 0), prefix to every thread through LDS
-    if constexpr (MODE == 2) {
-      if (tid == 0) s_prefix = t > 0 ? tail_prefix<S>(sc, tile - 1, gen) : S::ident();
-    } else if (wave == 0) {
+    if (wave == 0) {
       const A prefix = look_back<S, scan_look<Ti, To>(), Q>(sc, tile, t, total, gen, lane,
                                                             x + row * len, s_own, s_win);
       if (lane == 0) s_prefix = prefix;
@@ -538,6 +531,133 @@ __global__ __launch_bounds__(kBlock, MODE == 0 ? 2 : 1) void k_scan_rows(
     body(Bool<true>());
   else
     body(Bool<false>());
+}
+
+// Rows shorter than a tile, and the last partial tile of longer ones (prefix:
+// the inclusive descriptor of the row's last whole tile): NW waves walk a row
+// NW x 64 x VPL elements at a time, VPL consecutive ones per lane in 16-byte
+// loads at element alignment, the next step's loads issued before this one's
+// are scanned.  Lanes are scanned by DPP moves, waves through LDS (one barrier
+// a step), steps by a running carry.  NW = 1 puts four rows in a workgroup and
+// needs no barrier.  The order of every addition is fixed, so floating rows
+// repeat bit for bit.  HBM-bound.  float32 rows (read and written)
+// 10,000 x 5000 196 -> 90 us (4.5 TB/s), 100,000 x 700 834 -> 106, 50,000 x
+// 1001 484 -> 75, int32 -> int64 10,000 x 5000 272 -> 150, against a guarded
+// 16,384-element tile per row; the tail of 50,000,000 elements 22 -> 5 us.
+template <typename A, int CTRL, int ROWS> __device__ __forceinline__ A dpp_or(A v, A ident) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned long long i = __builtin_bit_cast(unsigned long long, ident);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp((int)(unsigned)i, (int)(unsigned)u, CTRL, ROWS, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp((int)(unsigned)(i >> 32), (int)(unsigned)(u >> 32), CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(A, ((unsigned long long)hi << 32) | lo);
+}
+// Elements per lane: 32 bytes of the wider of input and output.
+template <typename Ti, typename To> constexpr int scan_vpl() {
+  return 32 / (int)(sizeof(Ti) > sizeof(To) ? sizeof(Ti) : sizeof(To));
+}
+// Inclusive scan over a wave's lanes; lanes without a source take the identity.
+template <typename S> __device__ __forceinline__ typename S::A wave_scan(typename S::A v) {
+  typedef typename S::A A;
+  const A id = S::ident();
+  v = S::comb(dpp_or<A, 0x111, 0xf>(v, id), v);  // row_shr:1
+  v = S::comb(dpp_or<A, 0x112, 0xf>(v, id), v);  // row_shr:2
+  v = S::comb(dpp_or<A, 0x114, 0xf>(v, id), v);  // row_shr:4
+  v = S::comb(dpp_or<A, 0x118, 0xf>(v, id), v);  // row_shr:8
+  v = S::comb(dpp_or<A, 0x142, 0xa>(v, id), v);  // row_bcast:15
+  v = S::comb(dpp_or<A, 0x143, 0xc>(v, id), v);  // row_bcast:31
+  return v;
+}
+
+template <int OP, typename Ti, typename To, int NW>
+__global__ __launch_bounds__(NW == 1 ? kBlock : NW * 64) void k_scan_short(
+    const Ti *__restrict__ x, To *__restrict__ y, long long rows, long long len, long long start,
+    long long tiles_per_row, ScanScratch sc, unsigned gen) {
+  typedef ScanOp<OP, Ti> S;
+  typedef typename S::A A;
+  constexpr int VPL = scan_vpl<Ti, To>();
+  constexpr int STEP = NW * 64 * VPL;
+  __shared__ A wtot[2][NW];
+  const int lane = threadIdx.x & 63, wave = NW == 1 ? 0 : threadIdx.x >> 6;
+  const long long row = NW == 1 ? (long long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)
+                                : (long long)blockIdx.x;
+  if (row >= rows) return;  // whole waves (NW == 1: no barrier below)
+  const Ti *xr = x + row * len + start;
+  To *yr = y + row * len + start;
+  const long long n = len - start;
+  A carry = S::ident();
+  if (start > 0) carry = tail_prefix<S>(sc, row * tiles_per_row + tiles_per_row - 1, gen);
+  const long long mine = (long long)(wave * 64 + lane) * VPL;
+  auto load = [&](Ti (&q)[VPL], long long b) {
+    if (b + VPL <= n) {
+      __builtin_memcpy(q, xr + b, sizeof(q));
+    } else {
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) q[j] = b + j < n ? xr[b + j] : Ti(0);
+    }
+  };
+  Ti cur[VPL], nxt[VPL];
+  load(cur, mine);
+  int par = 0;
+  for (long long s0 = 0; s0 < n; s0 += STEP, par ^= 1) {
+    const long long b = s0 + mine;
+    if (s0 + STEP < n) load(nxt, b + STEP);
+    A tot = S::ident();
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+      if (b + j < n) tot = S::comb(tot, S::map(cur[j]));
+    const A inc = wave_scan<S>(tot);
+    A run = dpp_or<A, 0x138, 0xf>(inc, S::ident());  // wave_shr:1: the lanes before
+    if constexpr (NW > 1) {
+      if (lane == 63) wtot[par][wave] = inc;
+      __syncthreads();
+      A pre = carry;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        if (w == wave) run = S::comb(pre, run);
+        pre = S::comb(pre, wtot[par][w]);
+      }
+      carry = pre;
+    } else {
+      run = S::comb(carry, run);
+      carry = S::comb(carry, readlane64(inc, 63));
+    }
+    To out[VPL];
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      run = S::comb(run, S::map(cur[j]));
+      out[j] = mmp_convert<To, A>(run);
+    }
+    if (b + VPL <= n) {
+      __builtin_memcpy(yr + b, out, sizeof(out));
+    } else {
+#pragma unroll
+      for (int j = 0; j < VPL; ++j)
+        if (b + j < n) yr[b + j] = out[j];
+    }
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) cur[j] = nxt[j];
+  }
+}
+
+// Waves per row: enough rows for eight waves a CU take one each; fewer take
+// four or sixteen, where the row has work for them.
+template <int OP, typename Ti, typename To>
+int launch_scan_short(long long rows, long long len, long long start, long long tpr, const void *x,
+                      void *y, const ScanScratch &sc, unsigned gen) {
+  constexpr int VPL = scan_vpl<Ti, To>();
+  const long long cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
+  const long long n = len - start;
+  if (rows >= 8 * cus || n <= 64 * VPL)
+    hipLaunchKernelGGL((k_scan_short<OP, Ti, To, 1>), dim3((unsigned)mmpi::ceil_div(rows, kBlock / 64)),
+                       dim3(kBlock), 0, mmpi::stream(), (const Ti *)x, (To *)y, rows, len, start, tpr,
+                       sc, gen);
+  else if (rows >= 2 * cus || n <= 4 * 64 * VPL)
+    hipLaunchKernelGGL((k_scan_short<OP, Ti, To, 4>), dim3((unsigned)rows), dim3(256), 0,
+                       mmpi::stream(), (const Ti *)x, (To *)y, rows, len, start, tpr, sc, gen);
+  else
+    hipLaunchKernelGGL((k_scan_short<OP, Ti, To, 16>), dim3((unsigned)rows), dim3(1024), 0,
+                       mmpi::stream(), (const Ti *)x, (To *)y, rows, len, start, tpr, sc, gen);
+  return mmpi::check_launch("mmp_scan(short rows)");
 }
 
 // Strided axis: one thread per column; the axis is cut into S chunks so
@@ -606,13 +726,17 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols(const Ti *__restrict__ x, 
 }
 
 // Strided axis with 16-byte column vectors (input element of 2, 4 or 8
-// bytes, inner extent a multiple of the vector, 16-byte aligned input and
-// output): a thread owns VI = 16 / sizeof(Ti) adjacent columns, so a
+// bytes, at least a vector of columns; accesses at element alignment, so rows
+// may start anywhere): a thread owns VI = 16 / sizeof(Ti) adjacent columns
+// (the last one of a row that VI does not divide the row's last VI, of which
+// it shares some with its neighbour: both write the same values), so a
 // workgroup reads 256 x 16 bytes of every row and each lane keeps 16 bytes
 // in flight per row.  Phase 1 writes the VI chunk totals, a carry pass turns
 // each column's totals into exclusive prefixes in place, phase 2 rescans
 // each chunk from its prefix.
 template <typename Ti> constexpr int scan_col_vec() { return 16 / (int)sizeof(Ti); }
+// 16 bytes at element alignment (2 bytes and up): one global access all the same
+typedef unsigned int u32x4u __attribute__((ext_vector_type(4), aligned(2)));
 
 template <int OP, typename Ti>
 __global__ __launch_bounds__(kBlock) void k_scan_cols_part_vec(
@@ -623,8 +747,9 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_part_vec(
   constexpr int VI = scan_col_vec<Ti>();
   const long long o = blockIdx.y;
   const int s = blockIdx.z;
-  const long long c = ((long long)blockIdx.x * kBlock + threadIdx.x) * VI;
-  if (c >= inner) return;
+  const long long cv = ((long long)blockIdx.x * kBlock + threadIdx.x) * VI;
+  if (cv >= inner) return;
+  const long long c = cv + VI <= inner ? cv : inner - VI;
   const long long per = (len + S - 1) / S;
   const long long b0 = s * per;
   const long long b1 = b0 + per < len ? b0 + per : len;
@@ -636,7 +761,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_part_vec(
   for (; l + kColUnroll <= b1; l += kColUnroll) {
     u32x4 q[kColUnroll];
 #pragma unroll
-    for (int u = 0; u < kColUnroll; ++u) q[u] = *reinterpret_cast<const u32x4 *>(p + (l + u) * inner);
+    for (int u = 0; u < kColUnroll; ++u) q[u] = *reinterpret_cast<const u32x4u *>(p + (l + u) * inner);
 #pragma unroll
     for (int u = 0; u < kColUnroll; ++u) {
       union { u32x4 v; Ti e[VI]; } w;
@@ -647,7 +772,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_part_vec(
   }
   for (; l < b1; ++l) {
     union { u32x4 v; Ti e[VI]; } w;
-    w.v = *reinterpret_cast<const u32x4 *>(p + l * inner);
+    w.v = *reinterpret_cast<const u32x4u *>(p + l * inner);
 #pragma unroll
     for (int e = 0; e < VI; ++e) acc[e] = Sc::comb(acc[e], Sc::map(w.e[e]));
   }
@@ -696,8 +821,9 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_vec(const Ti *__restrict__
   static_assert(VI % VO == 0, "a lane's outputs fill whole 16-byte stores");
   const long long o = blockIdx.y;
   const int s = blockIdx.z;
-  const long long c = ((long long)blockIdx.x * kBlock + threadIdx.x) * VI;
-  if (c >= inner) return;
+  const long long cv = ((long long)blockIdx.x * kBlock + threadIdx.x) * VI;
+  if (cv >= inner) return;
+  const long long c = cv + VI <= inner ? cv : inner - VI;
   const long long per = (len + S - 1) / S;
   const long long b0 = s * per;
   const long long b1 = b0 + per < len ? b0 + per : len;
@@ -705,7 +831,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_vec(const Ti *__restrict__
 #pragma unroll
   for (int e = 0; e < VI; ++e) acc[e] = pre ? pre[((long long)o * S + s) * inner + c + e] : Sc::ident();
   const long long off = o * len * inner + c;
-  auto row = [&](const u32x4 &v, long long l) {
+  auto row = [&](u32x4 v, long long l) {
     union { u32x4 v; Ti e[VI]; } w;
     w.v = v;
     union { u32x4 v[VI / VO]; To e[VI]; } r;
@@ -714,7 +840,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_vec(const Ti *__restrict__
       acc[e] = Sc::comb(acc[e], Sc::map(w.e[e]));
       r.e[e] = mmp_convert<To, A>(acc[e]);
     }
-    u32x4 *dst = reinterpret_cast<u32x4 *>(y + off + l * inner);
+    u32x4u *dst = reinterpret_cast<u32x4u *>(y + off + l * inner);
 #pragma unroll
     for (int k = 0; k < VI / VO; ++k) dst[k] = r.v[k];
   };
@@ -722,11 +848,11 @@ __global__ __launch_bounds__(kBlock) void k_scan_cols_vec(const Ti *__restrict__
   for (; l + kColUnroll <= b1; l += kColUnroll) {
     u32x4 q[kColUnroll];
 #pragma unroll
-    for (int u = 0; u < kColUnroll; ++u) q[u] = *reinterpret_cast<const u32x4 *>(x + off + (l + u) * inner);
+    for (int u = 0; u < kColUnroll; ++u) q[u] = *reinterpret_cast<const u32x4u *>(x + off + (l + u) * inner);
 #pragma unroll
     for (int u = 0; u < kColUnroll; ++u) row(q[u], l + u);
   }
-  for (; l < b1; ++l) row(*reinterpret_cast<const u32x4 *>(x + off + l * inner), l);
+  for (; l < b1; ++l) row(*reinterpret_cast<const u32x4u *>(x + off + l * inner), l);
 }
 
 template <int OP, typename Ti, typename To> constexpr bool scan_out_ok() {
@@ -744,7 +870,7 @@ template <int OP, typename Ti, typename To>
 int launch_scan_cols_vec(long long outer, long long len, long long inner, const void *x, void *y) {
   typedef typename ScanOp<OP, Ti>::A A;
   constexpr int VI = scan_col_vec<Ti>();
-  const long long ncb = mmpi::ceil_div(inner / VI, kBlock);
+  const long long ncb = mmpi::ceil_div(mmpi::ceil_div(inner, VI), kBlock);
   const long long want = (MMP_SCAN_COL_TARGET + outer * ncb - 1) / (outer * ncb);
   const long long maxs = len / 64 > 0 ? len / 64 : 1;
   long long S = want < maxs ? want : maxs;
@@ -792,9 +918,12 @@ int launch_scan(long long outer, long long len, long long inner, const void *x, 
       constexpr long long kTile = (long long)sub_tiles<Ti>() * kSubTile;
       // streaming layout: every row starts 16-byte aligned in input and output
       const bool vec = ((uintptr_t)x & 15u) == 0 && ((uintptr_t)y & 15u) == 0 &&
-                       (len * (long long)sizeof(Ti)) % 16 == 0 &&
-                       (len * (long long)sizeof(To)) % 16 == 0;
-      const long long tpr = vec ? len / kTile : mmpi::ceil_div(len, kTile);
+                       (outer == 1 || ((len * (long long)sizeof(Ti)) % 16 == 0 &&
+                                       (len * (long long)sizeof(To)) % 16 == 0));
+      // rows for the short-row kernel alone: under a tile, or unaligned and
+      // enough of them to fill the device
+      const bool by_rows = len < kTile || (!vec && outer >= 256);
+      const long long tpr = by_rows ? 0 : vec ? len / kTile : mmpi::ceil_div(len, kTile);
       const long long ntiles = outer * tpr;
       if (ntiles > 0x7fffffffLL || outer > 0x7fffffffLL)
         return mmpi::fail(MMP_E_ARG, "scan too large");
@@ -810,6 +939,7 @@ int launch_scan(long long outer, long long len, long long inner, const void *x, 
       // polls of a missing predecessor before summing it here: it normally
       // publishes within a few (its loads are in flight when we start)
       sc.spin_limit = wp.spin_limit < kPollsBeforeSum ? wp.spin_limit : kPollsBeforeSum;
+      if (by_rows) return launch_scan_short<OP, Ti, To>(outer, len, 0, 0, x, y, sc, gen);
       if (!vec) {
         hipLaunchKernelGGL((k_scan_rows<OP, Ti, To, 1>), dim3((unsigned)ntiles), dim3(kBlock), 0,
                            mmpi::stream(), (const Ti *)x, (To *)y, len, tpr, ntiles, sc, gen);
@@ -820,17 +950,18 @@ int launch_scan(long long outer, long long len, long long inner, const void *x, 
                            mmpi::stream(), (const Ti *)x, (To *)y, len, tpr, ntiles, sc, gen);
         if (int e = mmpi::check_launch("mmp_scan(rows)")) return e;
       }
-      if (len % kTile) {
-        hipLaunchKernelGGL((k_scan_rows<OP, Ti, To, 2>), dim3((unsigned)outer), dim3(kBlock), 0,
-                           mmpi::stream(), (const Ti *)x, (To *)y, len, tpr, ntiles, sc, gen);
-        return mmpi::check_launch("mmp_scan(row tails)");
-      }
+      if (len % kTile)
+        return launch_scan_short<OP, Ti, To>(outer, len, len / kTile * kTile, tpr, x, y, sc, gen);
       return MMP_OK;
     }
     if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided scan: outer extent %lld > 65535", outer);
     if constexpr (sizeof(Ti) >= 2) {
       constexpr int VI = scan_col_vec<Ti>();
-      if (inner % VI == 0 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)y & 15u) == 0)
+      // whole aligned vectors; or four or more columns a vector and enough rows
+      // to split (float32 50,000 x 1001 155 -> 126 us; float64 3000 x 3001 is
+      // quicker by column, 36 against 42, and so is 100 x 300,001)
+      if ((inner % VI == 0 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)y & 15u) == 0) ||
+          (VI >= 4 && inner >= VI && len >= 128))
         return launch_scan_cols_vec<OP, Ti, To>(outer, len, inner, x, y);
     }
     const long long ncb = mmpi::ceil_div(inner, kBlock);
