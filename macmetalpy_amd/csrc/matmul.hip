@@ -20,7 +20,9 @@
 //    Accumulation in fp32 (the reference accumulates float16 in half).
 //    Products with 256-divisible extents, 16-byte aligned rows and at least
 //    128 output tiles of 256 x 256 use k_gemm16_dma instead (256 x 256
-//    tiles, operands copied global -> LDS without passing through VGPRs).
+//    tiles, operands copied global -> LDS without passing through VGPRs);
+//    other whole tiles of aligned rows k_gemm16_aligned, where there are
+//    enough of them; everything else k_gemm16, as k_gemm4 below.
 //  * float32 / float64: v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64.  The
 //    k slot a lane feeds is permuted (MFMA step t, lane group g consumes
 //    k = KG*g + t), so a lane's A values for a whole slab are contiguous in
@@ -32,9 +34,10 @@
 //    Everything else of these types is k_gemm4: any extents and alignment,
 //    operands as they are or transposed, the K range split over workgroups
 //    where the output has few tiles.
-// Partial tiles and unaligned operands of the 16-bit kernels use guarded
-// scalar loads (zero fill) and guarded stores.  Integer matmul: LDS-tiled exact kernel with
+// Integer matmul: LDS-tiled exact kernel with
 // wrap-around arithmetic (NumPy's integer matmul wraps).
+#include <type_traits>
+
 #include "mmp_ops.h"
 #include "mmp_internal.h"
 
@@ -73,12 +76,13 @@ template <typename T> __device__ __forceinline__ T from_f32(float v) {
   }
 }
 
-template <typename T, bool EDGE>
-__global__ __launch_bounds__(kBlock, 2) void k_gemm16(const T *__restrict__ A,
-                                                     const T *__restrict__ B, T *__restrict__ C,
-                                                     int M, int N, int K, long long lda,
-                                                     long long ldb, long long ldc, long long sA,
-                                                     long long sB, long long sC, int tiles_n) {
+// 128 x 128 tiles for whole tiles and slabs of aligned rows, where the general
+// kernel below takes 5 % longer (2304^3 54.6 us here, 57.2 there).
+template <typename T>
+__global__ __launch_bounds__(kBlock, 2) void k_gemm16_aligned(
+    const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int M, int N, int K,
+    long long lda, long long ldb, long long ldc, long long sA, long long sB, long long sC,
+    int tiles_n) {
   constexpr int BK = 64, LDK = BK + 8;
   typedef typename Half16<T>::vec V;
   __shared__ __attribute__((aligned(16))) unsigned short As[2][BM * LDK];
@@ -103,29 +107,12 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm16(const T *__restrict__ A,
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int r = m0 + a_row + 32 * p, k = k0 + a_kv * 8;
-      if constexpr (!EDGE) {
-        ra[p] = *reinterpret_cast<const u32x4 *>(Ag + (long long)r * lda + k);
-      } else {
-        unsigned short h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          h[e] = (r < M && k + e < K) ? Ag[(long long)r * lda + k + e] : (unsigned short)0;
-        ra[p] = u32x4{h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16),
-                      h[4] | ((unsigned)h[5] << 16), h[6] | ((unsigned)h[7] << 16)};
-      }
+      ra[p] = *reinterpret_cast<const u32x4 *>(Ag + (long long)r * lda + k);
     }
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) {
       const int k = k0 + b_k8 * 8 + kk, n = n0 + b_n4 * 4;
-      if constexpr (!EDGE) {
-        rb[kk] = *reinterpret_cast<const u32x2 *>(Bg + (long long)k * ldb + n);
-      } else {
-        unsigned short h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          h[e] = (k < K && n + e < N) ? Bg[(long long)k * ldb + n + e] : (unsigned short)0;
-        rb[kk] = u32x2{h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16)};
-      }
+      rb[kk] = *reinterpret_cast<const u32x2 *>(Bg + (long long)k * ldb + n);
     }
   };
   auto store = [&](int buf) {
@@ -152,7 +139,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm16(const T *__restrict__ A,
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
 
-  const int nk = (K + BK - 1) / BK;
+  const int nk = K / BK;
   load(0);
   store(0);
   __syncthreads();
@@ -188,8 +175,174 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm16(const T *__restrict__ A,
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm * 64 + i * 16 + (lane >> 4) * 4 + r;
         const int col = n0 + wn * 64 + j * 16 + fr;
-        if (!EDGE || (row < M && col < N)) Cb[(long long)row * ldc + col] = from_f32<T>(acc[i][j][r]);
+        Cb[(long long)row * ldc + col] = from_f32<T>(acc[i][j][r]);
       }
+}
+
+// General 16-bit product: any extents, alignment and row strides, 32 I x 32 J
+// outputs per workgroup (four waves, 2 x 2), 64 deep slabs.  Loads, `edge`,
+// K ranges (blockIdx.z) and end checks as in k_gemm4 below.  A thread brings
+// I 16-byte vectors of A and a 2 J (k) x 4 (n) block of B per slab; the block
+// is transposed in registers on its way to LDS.  The MFMA is issued as
+// C^T = B^T A^T, so that a lane's four accumulators are four consecutive
+// columns of a row.  To: T, or float for the partial products of K ranges.
+// float16 3000 x 2500 x 2001 175 -> 60 us (500 TFLOP/s), 5000 x 4999 x 5000 1408
+// -> 425 (588), 64 x 64 x 5000 208 -> 12, 1000^3 52 -> 13, against guarded
+// element loads in 128 wide tiles.
+template <typename T, typename To, int I, int J>
+__global__ __launch_bounds__(kBlock, 2) void k_gemm16(const T *__restrict__ A,
+                                                     const T *__restrict__ B, To *__restrict__ C,
+                                                     int M, int N, int K, long long lda,
+                                                     long long ldb, long long ldc, long long sA,
+                                                     long long sB, long long sC, long long sZ,
+                                                     int tiles_n, int kspan, int edge,
+                                                     const T *Aend, const T *Bend) {
+  constexpr int BK = 64, LDK = BK + 8, TM = 32 * I, TN = 32 * J;
+  constexpr int NG = 8 * J, KB = 2 * J;  // threads along n; k rows per thread of B
+  typedef typename Half16<T>::vec V;
+  typedef unsigned short u16;
+  typedef u16 a8 __attribute__((ext_vector_type(8)));
+  typedef u16 a8u __attribute__((ext_vector_type(8), aligned(2)));
+  typedef u16 b4 __attribute__((ext_vector_type(4)));
+  typedef u16 b4u __attribute__((ext_vector_type(4), aligned(2)));
+  __shared__ __attribute__((aligned(16))) u16 As[2][TM * LDK];
+  __shared__ __attribute__((aligned(16))) u16 Bs[2][TN * LDK];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+  const long long bz = blockIdx.y;
+  const int m0 = tm * TM, n0 = tn * TN;
+  const u16 *Ag = reinterpret_cast<const u16 *>(A + bz * sA) + (long long)m0 * lda;
+  const u16 *Bg = reinterpret_cast<const u16 *>(B + bz * sB) + n0;
+  const u16 *Ae = reinterpret_cast<const u16 *>(Aend), *Be = reinterpret_cast<const u16 *>(Bend);
+
+  const int a_row = tid >> 3, a_k = (tid & 7) * 8;
+  const int b_n = (tid % NG) * 4, b_k = (tid / NG) * KB;
+  unsigned ao[I];
+#pragma unroll
+  for (int p = 0; p < I; ++p)
+    ao[p] = (unsigned)min(a_row + 32 * p, M - 1 - m0) * (unsigned)lda + (unsigned)a_k;
+  const int bn = n0 + b_n < N ? b_n : 0;
+  const unsigned bo = (unsigned)b_k * (unsigned)ldb + (unsigned)bn;
+  a8 ra[I];
+  b4 rb[KB];
+  const int nk = (K + BK - 1) / BK;
+  const int kb = blockIdx.z * kspan, ke = min(nk, kb + kspan);
+
+  auto load = [&](int kt) {
+    const int k0 = kt * BK;
+    if (!((edge & 6) || ((edge & 1) && kt == nk - 1))) {
+      const u16 *ga = Ag + k0, *gb = Bg + (long long)k0 * ldb;
+#pragma unroll
+      for (int p = 0; p < I; ++p) ra[p] = *reinterpret_cast<const a8u *>(ga + ao[p]);
+#pragma unroll
+      for (int kk = 0; kk < KB; ++kk)
+        rb[kk] = *reinterpret_cast<const b4u *>(gb + bo + (unsigned)kk * (unsigned)ldb);
+      return;
+    }
+    const bool vec_a = !(edge & 2), vec_b = !(edge & 4);
+#pragma unroll
+    for (int p = 0; p < I; ++p) {
+      const int k = k0 + a_k;
+      const u16 *g = Ag + (long long)min(a_row + 32 * p, M - 1 - m0) * lda + min(k, K - 1);
+      if (vec_a && g + 8 <= Ae) {
+        ra[p] = *reinterpret_cast<const a8u *>(g);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ra[p][e] = k + e < K ? g[e] : (u16)0;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (k + e >= K) ra[p][e] = 0;
+    }
+#pragma unroll
+    for (int kk = 0; kk < KB; ++kk) {
+      const int k = k0 + b_k + kk;
+      const u16 *g = Bg + (long long)min(k, K - 1) * ldb + bn;
+      if (vec_b && g + 4 <= Be) {
+        rb[kk] = *reinterpret_cast<const b4u *>(g);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rb[kk][e] = n0 + bn + e < N ? g[e] : (u16)0;
+      }
+      if (k >= K) rb[kk] = b4{0, 0, 0, 0};
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < I; ++p)
+      *reinterpret_cast<a8 *>(&As[buf][(a_row + 32 * p) * LDK + a_k]) = ra[p];
+    // column c of the block, its KB consecutive k: halves of word pairs
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      typedef unsigned kv __attribute__((ext_vector_type(KB / 2)));
+      kv h;
+#pragma unroll
+      for (int d = 0; d < KB / 2; ++d) {
+        const unsigned lo = __builtin_bit_cast(u32x2, rb[2 * d])[c >> 1];
+        const unsigned hi = __builtin_bit_cast(u32x2, rb[2 * d + 1])[c >> 1];
+        h[d] = (c & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
+      }
+      *reinterpret_cast<kv *>(&Bs[buf][(b_n + c) * LDK + b_k]) = h;
+    }
+  };
+
+  f4 acc[I][J];
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+
+  load(kb);
+  store(0);
+  __syncthreads();
+  const int fr = lane & 15, fk = (lane >> 4) * 8;
+  for (int kt = kb; kt < ke; ++kt) {
+    const int cur = (kt - kb) & 1;
+    if (kt + 1 < ke) load(kt + 1);
+#pragma unroll
+    for (int s = 0; s < BK / 32; ++s) {
+      V af[I], bf[J];
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+        af[i] = *reinterpret_cast<const V *>(&As[cur][(wm * 16 * I + i * 16 + fr) * LDK + s * 32 + fk]);
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        bf[j] = *reinterpret_cast<const V *>(&Bs[cur][(wn * 16 * J + j * 16 + fr) * LDK + s * 32 + fk]);
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i][j] = Half16<T>::mfma(bf[j], af[i], acc[i][j]);
+    }
+    if (kt + 1 < ke) store(cur ^ 1);
+    __syncthreads();
+  }
+
+  // lane: row lane % 16 and columns 4 (lane / 16) .. + 3 of each 16 x 16 tile
+  To *Cb = C + bz * sC + (long long)blockIdx.z * sZ;
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int row = m0 + wm * 16 * I + i * 16 + fr;
+      const int col = n0 + wn * 16 * J + j * 16 + (lane >> 4) * 4;
+      if (row >= M || col >= N) continue;
+      To h[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (sizeof(To) == 4) h[r] = acc[i][j][r];
+        else h[r] = from_f32<To>(acc[i][j][r]);
+      }
+      To *o = Cb + (long long)row * ldc + col;
+      if (col + 4 <= N) {
+        __builtin_memcpy(o, h, sizeof(h));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < N) o[r] = h[r];
+      }
+    }
 }
 
 // ---------------------------- 16-bit inputs, large tiles, global -> LDS DMA
@@ -446,10 +599,11 @@ template <> struct Mfma4<double> {
 // enough for a global load).  Rows (columns) past the edge re-read the last
 // one, or the next row's start: such values only reach outputs that are not
 // stored.  `edge` says when even that could leave the operand: bit 0, the
-// last slab is guarded element by element and zero filled (it is a partial
-// one, or a vector at the end of the operand's last row would run over it);
-// bit 1, every slab is (rows shorter than a vector, or so long that the
-// 32-bit lane offsets do not reach).
+// last slab is checked vector by vector against the operand's end, and zero
+// beyond K (it is a partial one, or a vector at the end of the operand's last
+// row would run over it); bits 1 and 2, every slab of A, of B, goes element
+// by element (rows shorter than a vector, or so long that the 32-bit lane
+// offsets do not reach).
 //
 // blockIdx.z takes slabs [z * kspan, (z + 1) * kspan) and writes its own
 // partial product sZ elements further on (k_sum_splits adds them).  `sub`:
@@ -465,7 +619,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, co
                                                     long long lda, long long ldb, long long ldc,
                                                     long long sA, long long sB, long long sC,
                                                     long long sZ, int tiles_n, int kspan, int edge,
-                                                    int sub) {
+                                                    int sub, const T *Aend, const T *Bend) {
   constexpr int V = 16 / sizeof(T);        // elements per 16-byte vector
   constexpr int BK = 128 / sizeof(T);      // 32 floats / 16 doubles per slab
   constexpr int KG = BK / 4;               // k per lane group per slab
@@ -514,7 +668,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, co
 
   auto load = [&](int kt) {
     const int k0 = kt * BK;
-    if (!((edge & 2) || ((edge & 1) && kt == nk - 1))) {
+    if (!((edge & 6) || ((edge & 1) && kt == nk - 1))) {
       const T *ga = Ag + (TA ? (long long)k0 * lda : (long long)k0);
       const T *gb = Bg + (TB ? (long long)k0 : (long long)k0 * ldb);
 #pragma unroll
@@ -523,25 +677,39 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, co
       for (int p = 0; p < BV; ++p) rb[p] = *reinterpret_cast<const VU *>(gb + bo[p]);
       return;
     }
+    // A slab that K cuts off, or whose last rows may end the operand: vectors
+    // wherever they stay inside it (as above they may reach over a row's end),
+    // element by element where not; k beyond K is zero.
+    auto fetch = [&](VL &q, const T *g, long long off, const T *end, bool vec, int have) {
+      if (vec && g + off + V <= end) {
+        q = *reinterpret_cast<const VU *>(g + off);
+      } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e) q[e] = e < have ? g[off + e] : (T)0;
+      }
+    };
+    const bool vec_a = !(edge & 2), vec_b = !(edge & 4);
 #pragma unroll
     for (int p = 0; p < AV; ++p) {
       const int idx = tid + p * kBlock, r = idx / A_VPR, v = (idx % A_VPR) * V;
+      const int k = k0 + (TA ? r : v), m = TA ? v : min(r, M - 1 - m0);
+      const int have = k >= K ? 0 : TA ? M - m0 - m : K - k;
+      fetch(ra[p], Ag, TA ? (long long)min(k, K - 1) * lda + (m0 + m < M ? m : 0)
+                          : (long long)m * lda + min(k, K - 1), Aend, vec_a, have);
 #pragma unroll
-      for (int e = 0; e < V; ++e) {
-        const int m = TA ? v + e : r, k = k0 + (TA ? r : v + e);
-        ra[p][e] = (m0 + m < M && k < K)
-                       ? Ag[TA ? (long long)k * lda + m : (long long)m * lda + k] : (T)0;
-      }
+      for (int e = 0; e < V; ++e)
+        if ((TA ? k : k + e) >= K) ra[p][e] = (T)0;
     }
 #pragma unroll
     for (int p = 0; p < BV; ++p) {
       const int idx = tid + p * kBlock, r = idx / B_VPR, v = (idx % B_VPR) * V;
+      const int k = k0 + (TB ? v : r), n = TB ? min(r, N - 1 - n0) : v;
+      const int have = k >= K ? 0 : TB ? K - k : N - n0 - n;
+      fetch(rb[p], Bg, TB ? (long long)n * ldb + min(k, K - 1)
+                          : (long long)min(k, K - 1) * ldb + (n0 + n < N ? n : 0), Bend, vec_b, have);
 #pragma unroll
-      for (int e = 0; e < V; ++e) {
-        const int n = TB ? r : v + e, k = k0 + (TB ? v + e : r);
-        rb[p][e] = (n0 + n < N && k < K)
-                       ? Bg[TB ? (long long)n * ldb + k : (long long)k * ldb + n] : (T)0;
-      }
+      for (int e = 0; e < V; ++e)
+        if ((TB ? k + e : k) >= K) rb[p][e] = (T)0;
     }
   };
   auto store = [&](int buf) {
@@ -621,9 +789,16 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, co
         const int col = n0 + wn * 16 * J + j * 16 + fr;
         if (row < M && col < N) {
           T *o = Cb + (long long)row * ldc + col;
-          *o = sub ? *o - acc[i][j][r] : acc[i][j][r];
+          if (sub) acc[i][j][r] = *o - acc[i][j][r];
+          *o = acc[i][j][r];
         }
       }
+}
+
+// The 16-bit types round from float (as the unsplit kernels do).
+template <typename To> __device__ __forceinline__ To mmp_round(double v) {
+  if constexpr (sizeof(To) == 2) return from_f32<To>((float)v);
+  else return (To)v;
 }
 
 // C[b][row][col] = sum over z of P[z][b][row][col] in float64, the partial
@@ -631,8 +806,8 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm4(const T *__restrict__ A, co
 // each adds its z = zl, zl + ZL, ... in eight running sums, and the sums meet
 // in a tree (a fixed order, and short chains: thousands of partials cost no
 // accuracy or time that one thread's long chain would).
-template <typename T, int ZL>
-__global__ __launch_bounds__(kBlock) void k_sum_splits(const T *__restrict__ P, T *__restrict__ C,
+template <typename T, typename To, int ZL>
+__global__ __launch_bounds__(kBlock) void k_sum_splits(const T *__restrict__ P, To *__restrict__ C,
                                                        int M, int N, long long ldc, long long sC,
                                                        long long total, int splits) {
   constexpr int OL = kBlock / ZL;  // outputs per workgroup
@@ -661,20 +836,20 @@ __global__ __launch_bounds__(kBlock) void k_sum_splits(const T *__restrict__ P, 
   if (zl == 0 && t < total) {
     const long long mn = (long long)M * N, b = t / mn, rem = t - b * mn;
     const int row = (int)(rem / N), col = (int)(rem - (long long)row * N);
-    C[b * sC + (long long)row * ldc + col] = (T)red[0][ol];
+    C[b * sC + (long long)row * ldc + col] = mmp_round<To>(red[0][ol]);
   }
 }
 
-template <typename T>
-int launch_sum_splits(const T *part, T *C, int M, int N, long long ldc, long long sC, long long total,
+template <typename T, typename To>
+int launch_sum_splits(const T *part, To *C, int M, int N, long long ldc, long long sC, long long total,
                       int splits) {
   // 64 consecutive outputs per wave read whole lines; few outputs take more
   // threads each instead
   if (total > 4096)
-    hipLaunchKernelGGL((k_sum_splits<T, 4>), dim3((unsigned)mmpi::ceil_div(total, kBlock / 4)),
+    hipLaunchKernelGGL((k_sum_splits<T, To, 4>), dim3((unsigned)mmpi::ceil_div(total, kBlock / 4)),
                        dim3(kBlock), 0, mmpi::stream(), part, C, M, N, ldc, sC, total, splits);
   else
-    hipLaunchKernelGGL((k_sum_splits<T, 32>), dim3((unsigned)mmpi::ceil_div(total, kBlock / 32)),
+    hipLaunchKernelGGL((k_sum_splits<T, To, 32>), dim3((unsigned)mmpi::ceil_div(total, kBlock / 32)),
                        dim3(kBlock), 0, mmpi::stream(), part, C, M, N, ldc, sC, total, splits);
   return mmpi::check_launch("mmp_matmul(split sum)");
 }
@@ -1138,39 +1313,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm_int(const T *__restrict__ A, co
 // -------------------------------------------------------------- launch
 inline bool al(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
-// The 256 x 256 kernel is used once the product has at least
-// MMP_GEMM16_BIG_MIN_TILES tiles (fewer leave CUs idle).
-#ifndef MMP_GEMM16_BIG_MIN_TILES
-#define MMP_GEMM16_BIG_MIN_TILES 128
-#endif
-
-template <typename T>
-int launch16(long long batch, int M, int N, int K, const void *A, long long lda, long long sA,
-             const void *B, long long ldb, long long sB, void *C, long long ldc, long long sC) {
-  if (M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
-      lda < (1ll << 28) && ldb < (1ll << 28) &&
-      ldc % 4 == 0 && sA % 8 == 0 && sB % 8 == 0 && sC % 4 == 0 && al(A, 16) && al(B, 16) &&
-      al(C, 8) && (long long)(M / 256) * (N / 256) * batch >= MMP_GEMM16_BIG_MIN_TILES) {
-    const int tm = M / 256, tn = N / 256;
-    hipLaunchKernelGGL((k_gemm16_dma<T>), dim3((unsigned)(tm * tn), (unsigned)batch), dim3(512), 0,
-                       mmpi::stream(), (const T *)A, (const T *)B, (T *)C, M, N, K, lda, ldb,
-                       ldc, sA, sB, sC, tm, tn);
-    return mmpi::check_launch("mmp_matmul(mfma16 256x256)");
-  }
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const bool fast = M % BM == 0 && N % BN == 0 && K % 64 == 0 && lda % 8 == 0 && ldb % 4 == 0 &&
-                    sA % 8 == 0 && sB % 4 == 0 && al(A, 16) && al(B, 8);
-  dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
-  if (fast)
-    hipLaunchKernelGGL((k_gemm16<T, false>), grid, dim3(kBlock), 0, mmpi::stream(), (const T *)A,
-                       (const T *)B, (T *)C, M, N, K, lda, ldb, ldc, sA, sB, sC, tiles_n);
-  else
-    hipLaunchKernelGGL((k_gemm16<T, true>), grid, dim3(kBlock), 0, mmpi::stream(), (const T *)A,
-                       (const T *)B, (T *)C, M, N, K, lda, ldb, ldc, sA, sB, sC, tiles_n);
-  return mmpi::check_launch("mmp_matmul(mfma16)");
-}
-
-// Tile and K split of the general float kernel.  With few output tiles most
+// Tile and K split of the general kernels.  With few output tiles most
 // CUs would idle, so the tile is made smaller or the K range cut as well; a
 // split pays for its partial products (written once, read once).  The choice
 // is the cheapest by this estimate, in microseconds: rounds of workgroups
@@ -1190,12 +1333,13 @@ struct Plan4 {
   int splits;  // K ranges
   double us;
 };
-inline double rounds_us(double wgs, double per_cu, double slabs, double shared, double alone) {
+inline double rounds_us(double wgs, double per_cu, double slabs, double start, double shared,
+                        double alone) {
   const double cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
   const double full = __builtin_floor(wgs / (cus * per_cu)), rest = wgs - full * cus * per_cu;
   const double share = __builtin_ceil(rest / cus);
   const double step = shared * share > alone ? shared * share : alone;
-  return full * (2.0 + slabs * shared * per_cu) + (rest > 0 ? 2.0 + slabs * step : 0.0);
+  return full * (start + slabs * shared * per_cu) + (rest > 0 ? start + slabs * step : 0.0);
 }
 inline Plan4 plan4(long long batch, int M, int N, int K, int elem, bool may_split) {
   const int nk = (int)(((long long)K * elem + 127) / 128);
@@ -1206,18 +1350,88 @@ inline Plan4 plan4(long long batch, int M, int N, int K, int elem, bool may_spli
   for (int tile = 128; tile >= 32; tile /= 2) {
     const double tiles = (double)((M + tile - 1) / tile) * ((N + tile - 1) / tile) * (double)batch;
     const double per_cu = tile == 128 ? 2 : tile == 64 ? 4 : 8;
-    // a slab of one workgroup: of several sharing a CU, and alone on it
-    const double shared = tile == 128 ? 1.85 : tile == 64 ? 0.5 : 0.15;
-    const double alone = tile == 128 ? 2.2 : tile == 64 ? 0.65 : 0.25;
+    const double start = tile == 128 ? 6.0 : tile == 64 ? 3.0 : 1.5;  // and the result's stores
+    // a slab of one workgroup: of several sharing a CU, and alone on it (the
+    // 16-bit matrix rate leaves a slab to its loads and LDS traffic)
+    const double shared = elem == 2 ? (tile == 128 ? 0.85 : tile == 64 ? 0.4 : 0.18)
+                                    : (tile == 128 ? 1.85 : tile == 64 ? 0.5 : 0.15);
+    const double alone = elem == 2 ? (tile == 128 ? 1.05 : tile == 64 ? 0.55 : 0.35)
+                                   : (tile == 128 ? 2.2 : tile == 64 ? 0.65 : 0.25);
     for (int s = s0; s <= 65535; s *= 2) {
       const double wgs = tiles * s;
       if (s > s0 && (!may_split || nk / s < 4 || wgs > 2 * cus * per_cu)) break;
-      double t = rounds_us(wgs, per_cu, (nk + s - 1) / s, shared, alone);
-      if (s > 1) t += 4.0 + 2e-6 * s * (double)batch * M * N * elem / 6.0;
+      double t = rounds_us(wgs, per_cu, (nk + s - 1) / s, start, shared, alone);
+      if (s > 1) t += 4.0 + 2e-6 * s * (double)batch * M * N * (elem == 2 ? 4 : elem) / 6.0;
       if (t < best.us * 0.98) best = Plan4{tile, s, t};
     }
   }
   return best;
+}
+
+// The 256 x 256 kernel is used once the product has at least
+// MMP_GEMM16_BIG_MIN_TILES tiles (fewer leave CUs idle).
+#ifndef MMP_GEMM16_BIG_MIN_TILES
+#define MMP_GEMM16_BIG_MIN_TILES 128
+#endif
+
+template <typename T>
+int launch16(long long batch, int M, int N, int K, const void *A, long long lda, long long sA,
+             const void *B, long long ldb, long long sB, void *C, long long ldc, long long sC) {
+  if (M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
+      lda < (1ll << 28) && ldb < (1ll << 28) &&
+      ldc % 4 == 0 && sA % 8 == 0 && sB % 8 == 0 && sC % 4 == 0 && al(A, 16) && al(B, 16) &&
+      al(C, 8) && (long long)(M / 256) * (N / 256) * batch >= MMP_GEMM16_BIG_MIN_TILES) {
+    const int tm = M / 256, tn = N / 256;
+    hipLaunchKernelGGL((k_gemm16_dma<T>), dim3((unsigned)(tm * tn), (unsigned)batch), dim3(512), 0,
+                       mmpi::stream(), (const T *)A, (const T *)B, (T *)C, M, N, K, lda, ldb,
+                       ldc, sA, sB, sC, tm, tn);
+    return mmpi::check_launch("mmp_matmul(mfma16 256x256)");
+  }
+  Plan4 pl = plan4(batch, M, N, K, 2, true);
+  if (pl.splits > 1) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(mmpi::stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+      pl = plan4(batch, M, N, K, 2, false);
+  }
+  constexpr int BK = 64;
+  if (pl.tile == 128 && pl.splits == 1 && M % 128 == 0 && N % 128 == 0 && K % BK == 0 &&
+      lda % 8 == 0 && ldb % 4 == 0 && sA % 8 == 0 && sB % 4 == 0 && al(A, 16) && al(B, 8)) {
+    hipLaunchKernelGGL((k_gemm16_aligned<T>), dim3((unsigned)(M / 128 * (N / 128)), (unsigned)batch),
+                       dim3(kBlock), 0, mmpi::stream(), (const T *)A, (const T *)B, (T *)C, M, N, K,
+                       lda, ldb, ldc, sA, sB, sC, N / 128);
+    return mmpi::check_launch("mmp_matmul(mfma16 128x128)");
+  }
+  const int nk = (K + BK - 1) / BK, kspan = (nk + pl.splits - 1) / pl.splits;
+  const int splits = (nk + kspan - 1) / kspan, tile = pl.tile;
+  const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
+  const long long total = (long long)M * N * batch;
+  const int edge = (K % BK || N % tile ? 1 : 0) | (lda < 7 || lda >= (1LL << 24) ? 2 : 0) |
+                   (ldb < 3 || ldb >= (1LL << 24) ? 4 : 0);
+  const T *a = (const T *)A, *b = (const T *)B;
+  const T *Aend = a + (batch - 1) * sA + (M - 1LL) * lda + K;
+  const T *Bend = b + (batch - 1) * sB + (K - 1LL) * ldb + N;
+  dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch, (unsigned)splits);
+  auto go = [&](auto *out, long long oldc, long long osC, long long osZ) {
+    typedef typename std::remove_pointer<decltype(out)>::type To;
+    if (tile == 128)
+      hipLaunchKernelGGL((k_gemm16<T, To, 4, 4>), grid, dim3(kBlock), 0, mmpi::stream(), a, b, out, M,
+                         N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, Aend, Bend);
+    else if (tile == 64)
+      hipLaunchKernelGGL((k_gemm16<T, To, 2, 2>), grid, dim3(kBlock), 0, mmpi::stream(), a, b, out, M,
+                         N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, Aend, Bend);
+    else
+      hipLaunchKernelGGL((k_gemm16<T, To, 1, 1>), grid, dim3(kBlock), 0, mmpi::stream(), a, b, out, M,
+                         N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, Aend, Bend);
+    return mmpi::check_launch("mmp_matmul(mfma16)");
+  };
+  if (splits == 1) return go((T *)C, ldc, sC, 0);
+  void *part = nullptr;
+  if (int st = mmp_alloc((size_t)splits * (size_t)total * 4, &part)) return st;
+  int st = go((float *)part, N, (long long)M * N, total);
+  if (st == MMP_OK)
+    st = launch_sum_splits<float, T>((const float *)part, (T *)C, M, N, ldc, sC, total, splits);
+  const int fs = mmp_free(part);  // stream-ordered
+  return st ? st : fs;
 }
 
 template <typename T, bool TA, bool TB>
@@ -1240,9 +1454,13 @@ int launch_general(long long batch, int M, int N, int K, const T *A, long long l
   const int tile = pl.tile;
   const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
   // see the kernel: short rows a vector could run past, or offsets past 32 bits
-  const bool guard_all = lda < V - 1 || ldb < V - 1 || lda >= (1LL << 24) || ldb >= (1LL << 24);
+  const bool guard_a = lda < V - 1 || lda >= (1LL << 24);
+  const bool guard_b = ldb < V - 1 || ldb >= (1LL << 24);
   const bool guard_last = K % BK || (TA && M % tile) || (!TB && N % tile);
-  const int edge = (guard_last ? 1 : 0) | (guard_all ? 2 : 0);
+  const int edge = (guard_last ? 1 : 0) | (guard_a ? 2 : 0) | (guard_b ? 4 : 0);
+  // one past each operand's last element
+  const T *Aend = A + (batch - 1) * sA + (TA ? (K - 1LL) * lda + M : (M - 1LL) * lda + K);
+  const T *Bend = B + (batch - 1) * sB + (TB ? (N - 1LL) * ldb + K : (K - 1LL) * ldb + N);
   void *part = nullptr;
   T *out = C;
   long long oldc = ldc, osC = sC, osZ = 0;
@@ -1256,16 +1474,16 @@ int launch_general(long long batch, int M, int N, int K, const T *A, long long l
   dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch, (unsigned)splits);
   if (tile == 128)
     hipLaunchKernelGGL((k_gemm4<T, TA, TB, 4, 4>), grid, dim3(kBlock), 0, mmpi::stream(), A, B, out,
-                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0);
+                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0, Aend, Bend);
   else if (tile == 64)
     hipLaunchKernelGGL((k_gemm4<T, TA, TB, 2, 2>), grid, dim3(kBlock), 0, mmpi::stream(), A, B, out,
-                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0);
+                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0, Aend, Bend);
   else
     hipLaunchKernelGGL((k_gemm4<T, TA, TB, 1, 1>), grid, dim3(kBlock), 0, mmpi::stream(), A, B, out,
-                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0);
+                       M, N, K, lda, ldb, oldc, sA, sB, osC, osZ, tiles_n, kspan, edge, sub ? 1 : 0, Aend, Bend);
   int st = mmpi::check_launch("mmp_matmul(mfma4)");
   if (part) {
-    if (st == MMP_OK) st = launch_sum_splits<T>((const T *)part, C, M, N, ldc, sC, total, splits);
+    if (st == MMP_OK) st = launch_sum_splits<T, T>((const T *)part, C, M, N, ldc, sC, total, splits);
     const int fs = mmp_free(part);  // stream-ordered
     if (st == MMP_OK) st = fs;
   }
@@ -1301,7 +1519,7 @@ int launch4(int ta, int tb, long long batch, int M, int N, int K, const void *A,
         return mmpi::check_launch("mmp_matmul(mfma4 dma)");
       }
       // few tiles: the general kernel's smaller tiles or K ranges reach more CUs
-      if (rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 1.6, 2.2) <=
+      if (rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 6.0, 1.6, 2.2) <=
           plan4(batch, M, N, K, 4, true).us) {
         hipLaunchKernelGGL(k_gemm4_dma, dim3((unsigned)(tiles_m * tiles_n), (unsigned)batch),
                            dim3(kBlock), 0, mmpi::stream(), (const float *)A, (const float *)B,

@@ -93,6 +93,34 @@ def test_general_kernel_exact(batch, m, n, k, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,n,k", _SHAPES + [(1, 64, 64, 5000), (1, 300, 1, 4000),
+                                                   (1, 1, 300, 4000), (2, 640, 384, 448)])
+def test_general_half_kernel_exact(batch, m, n, k):
+    """float16: the same edges (slabs of 64, vectors of 8 and 4), contiguous
+    and with row strides that leave rows on odd elements, NaN round the view.
+    Sums of products of -1, 0 and 1 stay below 2048 here and so are exact."""
+    g = np.random.default_rng(m * 1000 + n + k)
+    lead = (batch,) if batch > 1 else ()
+    a, b = (g.integers(-1, 2, lead + s).astype(np.float16) for s in ((m, k), (k, n)))
+    print("half", batch, m, n, k, flush=True)
+    want = np.matmul(a.astype(np.float32), b.astype(np.float32))
+    assert np.abs(want).max() <= 2048
+    got = cp.matmul(cp.array(a), cp.array(b)).get()
+    assert got.dtype == np.float16 and np.array_equal(got.astype(np.float32), want)
+    if batch == 1:
+        from macmetalpy_amd._backend import HipBackend
+        from macmetalpy_amd._dtypes import dtype_code
+        pa, pb = np.full((m, k + 3), np.nan, np.float16), np.full((k, n + 5), np.nan, np.float16)
+        pa[:, :k], pb[:, :n] = a, b
+        c = np.full((m, n + 1), 7.0, np.float16)
+        da, db, dc = (cp.array(x)._ensure_gpu() for x in (pa, pb, c))
+        HipBackend().matmul(dtype_code(np.dtype(np.float16)), 1, m, n, k, da._ptr, k + 3, 0, db._ptr,
+                            n + 5, 0, dc._ptr, n + 1, 0)
+        out = dc.get()
+        assert np.array_equal(out[:, :n].astype(np.float32), want) and np.all(out[:, n:] == 7.0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_general_kernel_views(dtype):
     """Row slices, column slices (misaligned rows), steps, reversed and
