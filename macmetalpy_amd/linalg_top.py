@@ -96,19 +96,22 @@ def matmul(x1, x2, out=None, **kwargs):
         A = A.astype(rdt)
     if B._dtype != rdt:
         B = B.astype(rdt)
-    pa = pb = None
-    if rdt.kind == "f" and rdt.itemsize > 2 and not (A._is_device_contiguous()
-                                                     and B._is_device_contiguous()):
-        A._ensure_gpu()
-        B._ensure_gpu()
-        if rdt.itemsize == 8 or not _copy_kernel_shape(M, N, K, batch):
-            pa, pb = _in_place(A, batch_shape), _in_place(B, batch_shape)
-    if pa is None:
-        A, sA = _batch_operand(A, batch_shape, (M, K))
-        pa = False, K, sA
-    if pb is None:
-        B, sB = _batch_operand(B, batch_shape, (K, N))
-        pb = False, N, sB
+    if (A._is_device_contiguous() and B._is_device_contiguous()
+            and A._shape[:-2] == B._shape[:-2]):
+        pa, pb = (False, K, M * K), (False, N, K * N)
+    else:
+        pa = pb = None
+        if rdt.kind == "f" and rdt.itemsize > 2:
+            A._ensure_gpu()
+            B._ensure_gpu()
+            if rdt.itemsize == 8 or not _copy_kernel_shape(M, N, K, batch):
+                pa, pb = _in_place(A, batch_shape), _in_place(B, batch_shape)
+        if pa is None:
+            A, sA = _batch_operand(A, batch_shape, (M, K))
+            pa = False, K, sA
+        if pb is None:
+            B, sB = _batch_operand(B, batch_shape, (K, N))
+            pb = False, N, sB
     res = ndarray._empty_device(tuple(batch_shape) + (M, N), rdt)
     if res.size:
         if K == 0:

@@ -157,6 +157,18 @@ def _reduce(a, kind, axis=None, dtype=None, out=None, keepdims=False):
         run_sum(node, axes is not None, odt, res._ptr, kind == "mean")
         return _finish(res, out)
 
+    if (a._fusion_node is not None and kind in ("sum", "mean") and dtype is None and a.ndim == 2
+            and axes == (0,) and a._dtype.kind == "f" and get_config().fusion):
+        from ._fusion import COL_SUM_MIN, run_col_sum
+        # a float64 mean divides afterwards, as its own reduction does: a
+        # reciprocal's rounding would show there
+        wide = kind == "mean" and odt == np.float64
+        res = ndarray._empty_device(oshape, odt)
+        if a.size >= COL_SUM_MIN and run_col_sum(a._fusion_node, odt, res._ptr,
+                                                 1.0 / red_len if kind == "mean" and not wide
+                                                 else 1.0):
+            return _finish(res / float(red_len) if wide else res, out)
+
     x = a._ensure_contiguous()
     lay = _layout(x._shape, axes)
     if lay is None:

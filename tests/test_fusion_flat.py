@@ -131,3 +131,49 @@ def test_flat_element_types(dtype):
         _same(cp.maximum(cp.maximum(dx, dr), dc).get() if dtype != np.bool_ else ((dx | dr) & dc).get(),
               np.maximum(np.maximum(x, r), c) if dtype != np.bool_ else (x | r) & c)
         _same((dx == dr).get(), x == r)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16, np.float64])
+def test_column_sum_source_compiles(dtype):
+    leaves = [_leaf((9, 8), dtype, (8, 1), 0x1000 * (k + 1)) for k in range(3)]
+    root = F.BinaryOpNode("mul_op", F.BinaryOpNode("sub_op", leaves[0], leaves[1], (9, 8), dtype),
+                          leaves[2], (9, 8), dtype)
+    src = F.generate_source(F._Program(root), ["v", "p", "r"], 1, np.dtype(dtype), False, "colsum")
+    assert rtc_build(src, F.RTC_OPTIONS)[:4] == b"\x7fELF"
+
+
+def test_column_sum_leaf_classes():
+    """A class stands for the strides it is read with; others are refused."""
+    for st, want in (((8, 1), "v"), ((13, 1), "v"), ((-8, 1), "v"), ((0, 1), "p"), ((3, 0), "r"),
+                     ((0, 0), "r"), ((1, 9), None), ((16, 2), None), ((8, -1), None)):
+        assert F._col_kinds([9], 8, [(8, 1), st]) == (want and ["v", want])
+    assert F._col_kinds([9], 3, [(3, 1)]) is None and F._col_kinds([], 8, [(1,)]) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.float16])
+@pytest.mark.parametrize("rows,cols", [(1_200_000, 4), (700_000, 7), (90_000, 50), (20_000, 255),
+                                       (20_000, 257), (5000, 1001), (40, 110_000)])
+def test_column_sums_of_expressions(rows, cols, dtype, monkeypatch):
+    """sum / mean / var / std of lazy expressions down the columns, with row
+    vectors, one value per row, padded and transposed leaves: NumPy's values
+    of the same expression, accumulated in float64."""
+    monkeypatch.setattr(F, "COL_SUM_MIN", 1 << 22)  # smaller than calls are sent there
+    g = np.random.default_rng(cols)
+    wide = (g.integers(-8, 9, (rows, cols + 3)) / 4).astype(dtype)
+    x, r, c = wide[:, 1:cols + 1], (g.integers(1, 5, cols) / 2).astype(dtype), \
+        g.integers(-3, 4, (rows, 1)).astype(dtype)
+    dw, dr, dc = cp.array(wide), cp.array(r), cp.array(c)
+    dx = dw[:, 1:cols + 1]
+    print("colsum", rows, cols, np.dtype(dtype), flush=True)
+    for got, e in ((cp.sum((dx - dr) * dc, axis=0), (x - r) * c),
+                   (cp.sum(dx * dx.copy() + dc, axis=0, keepdims=True), x * x + c)):
+        want = np.sum(e.astype(np.float64), axis=0, keepdims=got.ndim == 2).astype(dtype)
+        assert got.dtype == want.dtype and np.array_equal(got.get(), want, equal_nan=True)
+    got, e = cp.mean(dx * dr, axis=0), (x * r).astype(np.float64)
+    want = e.mean(axis=0)
+    tol = 2 * np.finfo(dtype).eps * np.abs(e).mean(axis=0) + np.finfo(dtype).tiny
+    assert got.dtype == dtype and np.all(np.abs(got.get().astype(np.float64) - want) <= tol)
+    if dtype != np.float16:
+        v = x.astype(np.float64)
+        assert np.allclose(cp.std(dx, axis=0).get(), v.std(axis=0), rtol=8 * np.finfo(dtype).eps)
