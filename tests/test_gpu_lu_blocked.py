@@ -71,7 +71,8 @@ def test_zero_and_nan_columns():
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("batch,n,nrhs", [(1, 1, 1), (3, 31, 2), (2, 32, 9), (40, 33, 1), (1, 64, 100),
-                                          (1, 300, 1), (2, 500, 8), (1, 1000, 20), (1, 2100, 3),
+                                          (1, 300, 1), (2, 500, 8), (1, 1000, 20), (1, 2048, 8),
+                                          (1, 2100, 8),
                                           (1, 4200, 5)])
 def test_solve(batch, n, nrhs, dtype):
     """Residual within the substitution's backward error: n u (|A| + |L| |U|)
