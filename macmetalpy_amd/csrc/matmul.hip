@@ -1518,9 +1518,12 @@ int launch4(int ta, int tb, long long batch, int M, int N, int K, const void *A,
                            sB, sC, tiles_n, (int)((M / 256) * tiles_n), (int)wide_tiles);
         return mmpi::check_launch("mmp_matmul(mfma4 dma)");
       }
-      // few tiles: the general kernel's smaller tiles or K ranges reach more CUs
-      if (rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 6.0, 1.6, 2.2) <=
-          plan4(batch, M, N, K, 4, true).us) {
+      // few tiles: the general kernel's smaller tiles or K ranges reach more
+      // CUs (32 of 384^3 53 -> 43 us); near the line
+      // the copies win (256 of 128^3 14.5 us against 16.3, 16 of 512^3 38
+      // against 42)
+      if (rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 4.0, 1.6, 1.9) <=
+          1.07 * plan4(batch, M, N, K, 4, true).us) {
         hipLaunchKernelGGL(k_gemm4_dma, dim3((unsigned)(tiles_m * tiles_n), (unsigned)batch),
                            dim3(kBlock), 0, mmpi::stream(), (const float *)A, (const float *)B,
                            (float *)C, M, N, K, lda, ldb, ldc, sA, sB, sC, tiles_n);
