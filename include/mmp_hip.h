@@ -531,7 +531,8 @@ int mmp_wait_status(uint32_t *flags);
 /* ---- test hooks -------------------------------------------------------- */
 /* Make the next `count`-th call of kind (1 = mmp_alloc, 2 = mmp_rtc_compile,
  * 3 = kernel launch) fail with MMP_E_INJECTED.  Kind 4: the `count`-th next
- * split reduction or scan waits for a tag that its writers never write,
+ * split reduction (one whose last workgroup combines the partials) or scan
+ * waits for a tag that its writers never write,
  * with a spin limit of 64: a reduction's bounded wait runs out at once (the
  * kernel still finishes) and the next mmp_sync / mmp_d2h returns
  * MMP_E_WAIT; a scan's tiles find no predecessor descriptor and sum their

@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "mmp_hip.h"
+#include "mmp_plan.h"
 
 namespace mmpi {
 
@@ -34,11 +35,8 @@ bool inject(int kind);
 // Per-device scratch memory owned by the library (grown on demand, never
 // shrunk).  Used for reduction partials, completion tickets and scan tile
 // descriptors.  The memory is zero-filled when first allocated; kernels
-// that use counters leave them at zero when they finish.
+// that use counters leave them at zero when they finish.  Slots: mmp_plan.h.
 void *scratch(int slot, size_t bytes, int *status);
-enum { SCRATCH_REDUCE_PARTIALS = 0, SCRATCH_REDUCE_TICKETS = 1,
-       SCRATCH_SCAN_FLAGS = 2, SCRATCH_SCAN_VALUES = 3,
-       SCRATCH_SCAN_COUNTER = 4, SCRATCH_NSLOTS = 5 };
 // Monotone call counter used to tag scan tile flags with a generation, so
 // the flag array never needs clearing between calls (atomic: concurrent
 // callers never share a generation).

@@ -414,7 +414,9 @@ __device__ __forceinline__ To finalize(A a, long long len) {
 // RELAXED agent-scope atomics.  The reader spins until the tag matches the
 // current call.  No release/acquire fence is needed -- on multi-XCD CDNA an
 // agent-scope fence writes back / invalidates the whole L2 of the XCD, which
-// costs far more than the partial itself.
+// costs far more than the partial itself.  Since the tag is all that tells
+// this call's word from an earlier call's, nothing untagged but zeros may be
+// written to such words: raw partials have memory of their own.
 template <typename A> constexpr int words_of() { return (int)((sizeof(A) + 3) / 4); }
 
 template <typename A>
@@ -454,7 +456,8 @@ __device__ __forceinline__ A get_tagged(const unsigned long long *slot, unsigned
 }
 
 struct ReduceScratch {
-  unsigned long long *words;  // tagged partial words
+  unsigned long long *words;  // tagged partial words; never a raw value
+  void *plain;                // raw partials for a second kernel (then no words), or null
   unsigned *tickets;          // arrival counters (left at 0)
   unsigned *timeout;          // pinned host word, set to 1 if a wait ran out
   unsigned tag;               // this call's generation (written)
@@ -621,16 +624,6 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_rows(const T *__restrict__
     out[row] = total.i;
 }
 
-// Partials of a strided reduction: few are combined by the last workgroup to
-// arrive; more (`plain`) are left in the scratch words as they are, (outer,
-// split, column), for a second kernel (k_cols_finish) whose many workgroups
-// read them side by side.  One workgroup alone reading 256
-// partials a column took longer than the reduction of a 2,000,000 x 50 matrix
-// (float32 sum over axis 0 98 us, against 76 with the second kernel), and 25
-// a column cost a 10,000 x 10,001 argmax 20 us more; but 31 of a 2000 x 300
-// matrix are done sooner than a second launch (8.6 us against 11.7).
-bool plain_partials(int S, long long bytes) { return S > 64 || (S > 16 && bytes >= (32LL << 20)); }
-
 // Strided arg-reduction: grid (ceil(inner / 2^lc), outer, S); 2^lc threads
 // side by side on the columns (as many as there are, up to the workgroup) and
 // the others on the rows below, whose results meet in LDS; the reduced axis
@@ -641,7 +634,7 @@ template <int OP, typename T, bool WIDE>  // WIDE: lc == 8, known at compile tim
 __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__ x,
                                                           long long *__restrict__ out,
                                                           long long len, long long inner, int S,
-                                                          int lc, bool plain, ReduceScratch sc) {
+                                                          int lc, ReduceScratch sc) {
   typedef Arg<OP, T> R;
   typedef typename R::A A;
   typedef typename mmp_t<T>::C C;
@@ -697,8 +690,8 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_cols(const T *__restrict__
     if (owner) out[o * inner + c] = v.i;
     return;
   }
-  if (plain) {
-    if (owner) reinterpret_cast<A *>(sc.words)[(o * S + s) * inner + c] = v;
+  if (sc.plain) {
+    if (owner) reinterpret_cast<A *>(sc.plain)[(o * S + s) * inner + c] = v;
     return;
   }
   // one tagged partial per (o, column block, s, column); ticket per (o, cb)
@@ -796,7 +789,7 @@ template <typename T, int VI> struct ColVec {
 
 template <typename R, typename T, int VI, typename MapF, typename StoreF>
 __device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len, long long inner,
-                                          int S, int lg, bool plain, const ReduceScratch &sc, MapF map,
+                                          int S, int lg, const ReduceScratch &sc, MapF map,
                                           StoreF store) {
   typedef typename R::A A;
   constexpr int W = words_of<A>();
@@ -876,12 +869,12 @@ __device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len
     }
     return;
   }
-  if (plain) {
+  if (sc.plain) {
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
       const int cc = threadIdx.x + k * kBlock;
       if (cc < CW && c0 + cc < inner)
-        reinterpret_cast<A *>(sc.words)[(o * S + s) * inner + c0 + cc] = acc[k];
+        reinterpret_cast<A *>(sc.plain)[(o * S + s) * inner + c0 + cc] = acc[k];
     }
     return;
   }
@@ -915,53 +908,14 @@ __device__ __forceinline__ void cols_body(const T *__restrict__ x, long long len
 template <int OP, typename T, typename To, int VI>
 __global__ __launch_bounds__(kBlock) void k_reduce_cols(const T *__restrict__ x, To *__restrict__ out,
                                                        long long len, long long inner, int S, int lg,
-                                                       bool plain, ReduceScratch sc) {
+                                                       ReduceScratch sc) {
   typedef Red<OP, T> R;
   cols_body<R, T, VI>(
-      x, len, inner, S, lg, plain, sc, [](T q) { return R::map(q); },
+      x, len, inner, S, lg, sc, [](T q) { return R::map(q); },
       [&](long long i, const typename R::A &a) { out[i] = finalize<OP, T, To>(a, len); });
 }
 
 // ------------------------------------------------------------ launch
-// Strided layouts: the split of the reduced axis that leaves the CUs most
-// evenly loaded, up to `per_cu` workgroups each and at least 64 steps of rows
-// (`steps`: rows over the rows a workgroup's lanes lie on side by side) to a
-// split.  Workgroups of a launch of this size all run together, so what
-// counts is that each CU gets as many: 40 column blocks x 6 splits (240
-// workgroups on 256 CUs) sum 10,000 x 10,001 float32 in 69 us, x 7 (280)
-// in 91.  Measured on 16384^2 float32 over axis 0: the column-vector sum runs
-// best with one workgroup per CU (256: 6.2 TB/s; 128: 5.3, 512: 5.8, 1024:
-// 5.4, 2048: 5.3), the arg kernel with four (argmax 4.76 TB/s; 512: 3.2,
-// 2048: 4.45).
-constexpr int kColVecPerCu = 1, kColPerCu = 4;
-int col_splits(long long col_blocks, long long steps, int per_cu) {
-  const long long cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
-  long long most = steps / 64;
-  if (most > 1024) most = 1024;
-  // enough workgroups already without splitting, or too few rows to split
-  if (col_blocks >= 4 * cus * per_cu || most <= 1) return 1;
-  // up to per_cu per CU; where the column blocks alone are about that many,
-  // a few more, which fill the CUs better
-  long long top = cus * per_cu / col_blocks;
-  if (top < 4) top = 4;
-  if (top > most) top = most;
-  int best = 1;
-  double best_fill = 0.0;
-  for (long long s = top; s >= 1; --s) {
-    const long long wgs = col_blocks * s, per = (wgs + cus - 1) / cus;
-    // the CUs' even share of the busiest one's load, less a little for every
-    // workgroup on it beyond the wanted number
-    double fill = (double)wgs / (double)(per * cus);
-    if (per > per_cu) fill -= 0.02 * (double)(per - per_cu);
-    if (per < per_cu) fill *= 0.5 + 0.5 * (double)per / per_cu;
-    if (fill > best_fill + 1e-9) {
-      best_fill = fill;
-      best = (int)s;
-    }
-  }
-  return best;
-}
-
 int choose_splits(long long rows, long long len) {
   long long want = (kTargetBlocks + rows - 1) / rows;
   // A single row (axis=None) splits into kTargetBlocksOneRow workgroups:
@@ -978,11 +932,20 @@ int choose_splits(long long rows, long long len) {
   return (int)s;
 }
 
+inline long long cus() { return mmpi::cu_count() > 0 ? mmpi::cu_count() : 256; }
+
+// Scratch for `count` raw partials of type A (a second kernel combines them).
+template <typename A> int plain_scratch(long long count, ReduceScratch *sc) {
+  int st = MMP_OK;
+  sc->plain = mmpi::scratch(mmpi::partials_slot(true), sizeof(A) * (size_t)count, &st);
+  return st;
+}
+
 // Scratch for `count` tagged partials of type A plus `nticket` tickets.
 template <typename A>
 int reduce_scratch(long long count, long long nticket, ReduceScratch *sc) {
   int st = MMP_OK;
-  sc->words = (unsigned long long *)mmpi::scratch(mmpi::SCRATCH_REDUCE_PARTIALS,
+  sc->words = (unsigned long long *)mmpi::scratch(mmpi::partials_slot(false),
                                                   8ull * words_of<A>() * count, &st);
   if (st) return st;
   sc->tickets = (unsigned *)mmpi::scratch(mmpi::SCRATCH_REDUCE_TICKETS, 4ull * nticket, &st);
@@ -1033,30 +996,31 @@ int launch_reduce(long long outer, long long len, long long inner, const void *x
   }
   if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided reduction: outer extent %lld > 65535", outer);
   const bool vec = inner >= col_vec<T>();
-  const int vi = vec ? col_vec<T>() : 1;
-  int lg = 0;  // lanes side by side on a row
-  while (lg < 6 && ((long long)vi << lg) < inner) ++lg;
-  const int cw = vi << lg;  // columns per workgroup
-  const long long ncb = mmpi::ceil_div(inner, cw);
-  int S = col_splits(outer * ncb, len >> (6 - lg), kColVecPerCu);
+  const mmpi::ColPlan pl = mmpi::reduce_cols_plan(outer, len, inner, col_vec<T>(), cus());
+  const int cw = pl.cw, lg = pl.lanes;
+  const long long ncb = pl.ncb;
+  int S = pl.splits;
   if (noalloc) S = noalloc_col_splits<A>(S, outer * ncb, cw);
+  const bool plain = mmpi::second_kernel(S, outer * len * inner * (long long)sizeof(T));
   if (S > 1) {
-    if (int st = noalloc ? noalloc_scratch<A>(outer * ncb * S * cw, outer * ncb, &sc)
+    if (int st = noalloc  ? noalloc_scratch<A>(outer * ncb * S * cw, outer * ncb, &sc)
+                 : plain ? plain_scratch<A>(outer * S * inner, &sc)
                          : reduce_scratch<A>(outer * ncb * S * cw, outer * ncb, &sc))
       return st;
+    // the static words are zeroed before every use, so raw values may lie there
+    if (noalloc && plain) sc.plain = sc.words;
   }
-  const bool plain = plain_partials(S, outer * len * inner * (long long)sizeof(T));
   const dim3 grid((unsigned)ncb, (unsigned)outer, (unsigned)S);
   if (vec)
     hipLaunchKernelGGL((k_reduce_cols<OP, T, To, col_vec<T>()>), grid, dim3(kBlock), 0,
-                       mmpi::stream(), (const T *)x, (To *)out, len, inner, S, lg, plain, sc);
+                       mmpi::stream(), (const T *)x, (To *)out, len, inner, S, lg, sc);
   else
     hipLaunchKernelGGL((k_reduce_cols<OP, T, To, 1>), grid, dim3(kBlock), 0, mmpi::stream(),
-                       (const T *)x, (To *)out, len, inner, S, lg, plain, sc);
+                       (const T *)x, (To *)out, len, inner, S, lg, sc);
   if (int st = mmpi::check_launch("mmp_reduce(cols)")) return st;
   if (!plain) return MMP_OK;
   hipLaunchKernelGGL((k_cols_finish<OP, T, To>), dim3((unsigned)mmpi::ceil_div(inner, 16),
-                     (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.words,
+                     (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.plain,
                      (To *)out, len, inner, S);
   return mmpi::check_launch("mmp_reduce(cols finish)");
 }
@@ -1077,25 +1041,26 @@ int launch_argreduce(long long outer, long long len, long long inner, const void
     return mmpi::check_launch("mmp_argreduce(rows)");
   }
   if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided argreduce: outer extent %lld > 65535", outer);
-  int lc = 0;  // threads side by side on the columns
-  while (lc < 8 && (1LL << lc) < inner) ++lc;
-  const long long ncb = mmpi::ceil_div(inner, 1LL << lc);
-  const int S = col_splits(outer * ncb, len >> (8 - lc), kColPerCu);
+  const mmpi::ColPlan pl = mmpi::argreduce_cols_plan(outer, len, inner, cus());
+  const int lc = pl.lanes, S = pl.splits;
+  const long long ncb = pl.ncb;
+  const bool plain = mmpi::second_kernel(S, outer * len * inner * (long long)sizeof(T));
   if (S > 1) {
-    if (int st = reduce_scratch<A>((outer * ncb * S) << lc, outer * ncb, &sc)) return st;
+    if (int st = plain ? plain_scratch<A>(outer * S * inner, &sc)
+                       : reduce_scratch<A>((outer * ncb * S) << lc, outer * ncb, &sc))
+      return st;
   }
-  const bool plain = plain_partials(S, outer * len * inner * (long long)sizeof(T));
   const dim3 grid((unsigned)ncb, (unsigned)outer, (unsigned)S);
   if (lc == 8)
     hipLaunchKernelGGL((k_argreduce_cols<OP, T, true>), grid, dim3(kBlock), 0, mmpi::stream(),
-                       (const T *)x, out, len, inner, S, lc, plain, sc);
+                       (const T *)x, out, len, inner, S, lc, sc);
   else
     hipLaunchKernelGGL((k_argreduce_cols<OP, T, false>), grid, dim3(kBlock), 0, mmpi::stream(),
-                       (const T *)x, out, len, inner, S, lc, plain, sc);
+                       (const T *)x, out, len, inner, S, lc, sc);
   if (int st = mmpi::check_launch("mmp_argreduce(cols)")) return st;
   if (!plain) return MMP_OK;
   hipLaunchKernelGGL((k_argcols_finish<OP, T>), dim3((unsigned)mmpi::ceil_div(inner, 16),
-                     (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.words, out,
+                     (unsigned)outer), dim3(kBlock), 0, mmpi::stream(), (const A *)sc.plain, out,
                      inner, S);
   return mmpi::check_launch("mmp_argreduce(cols finish)");
 }

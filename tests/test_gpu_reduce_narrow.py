@@ -62,3 +62,22 @@ def test_few_columns_nan(rows, cols):
     inf = h.copy()
     inf[rows // 2] = -np.inf
     assert np.array_equal(cp.sum(cp.array(inf), axis=0).get(), np.sum(inf, axis=0), equal_nan=True)
+
+
+def test_partials_of_one_call_do_not_reach_the_next():
+    """Reductions that leave raw partials for a second kernel, whose values
+    are the numbers that calls are tagged with, between reductions that know
+    their partials by the tag."""
+    rows, cols = 400_000, 48
+    raw = np.empty((rows, cols), np.int32)
+    raw[:] = np.arange(cols * 8).reshape(8, cols)[np.arange(rows) % 8]
+    big = np.random.default_rng(0).integers(-9, 9, (3000, 300)).astype(np.int32)
+    draw, dbig = cp.array(raw), cp.array(big)
+    flat = cp.array(big.ravel())
+    for _ in range(40):
+        assert np.array_equal(cp.max(draw, axis=0).get(), raw[7])
+        assert np.array_equal(cp.argmax(draw, axis=0).get(), np.full(cols, 7))
+        assert np.array_equal(cp.max(dbig, axis=0).get(), big.max(axis=0))
+        assert np.array_equal(cp.sum(dbig, axis=0).get(), big.sum(axis=0))
+        assert np.array_equal(cp.argmin(dbig, axis=0).get(), big.argmin(axis=0))
+        assert int(cp.sum(flat)) == big.sum()
