@@ -1313,59 +1313,9 @@ __global__ __launch_bounds__(kBlock) void k_gemm_int(const T *__restrict__ A, co
 // -------------------------------------------------------------- launch
 inline bool al(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
-// Tile and K split of the general kernels.  With few output tiles most
-// CUs would idle, so the tile is made smaller or the K range cut as well; a
-// split pays for its partial products (written once, read once).  The choice
-// is the cheapest by this estimate, in microseconds: rounds of workgroups
-// over the CUs (two 128, four 64 or eight 32 wide tiles fit one), each a
-// start-up plus its slabs, at the matrix cores' rate for the workgroups that
-// share a CU but no faster than one alone hides its loads; and the partials
-// at 6 TB/s plus a launch.  At most 16,384 outputs over a K of 16,384 or more
-// are always cut into ranges of at most 2048, whose sums meet in float64:
-// float32 sums of 10^7 terms then stay within 5e-8 of exact (2e-6 with ranges
-// of 6000).  Measured over tiles and splits, the choice is the
-// fastest or within a tenth of it: float32 1000^3 28 us (32 wide, unsplit; 64
-// wide 30, 128 wide in four splits 34), 2049^3 198 (64 wide; 128 wide 231),
-// 4000 x 70 x 3000 35 (32 wide in two; unsplit 128 wide 94); float64 500 x 500
-// x 100,000 0.84 ms (128 wide in 32; unsplit 15.8).
-struct Plan4 {
-  int tile;    // 128, 64 or 32
-  int splits;  // K ranges
-  double us;
-};
-inline double rounds_us(double wgs, double per_cu, double slabs, double start, double shared,
-                        double alone) {
-  const double cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
-  const double full = __builtin_floor(wgs / (cus * per_cu)), rest = wgs - full * cus * per_cu;
-  const double share = __builtin_ceil(rest / cus);
-  const double step = shared * share > alone ? shared * share : alone;
-  return full * (start + slabs * shared * per_cu) + (rest > 0 ? start + slabs * step : 0.0);
-}
-inline Plan4 plan4(long long batch, int M, int N, int K, int elem, bool may_split) {
-  const int nk = (int)(((long long)K * elem + 127) / 128);
-  const double cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
-  Plan4 best{128, 1, 1e30};
-  const bool long_sum = may_split && batch == 1 && (double)M * N <= 16384 && K >= 16384;
-  const int s0 = !long_sum ? 1 : K < 2048 * 65535 ? (K + 2047) / 2048 : 65535;  // grid limit
-  for (int tile = 128; tile >= 32; tile /= 2) {
-    const double tiles = (double)((M + tile - 1) / tile) * ((N + tile - 1) / tile) * (double)batch;
-    const double per_cu = tile == 128 ? 2 : tile == 64 ? 4 : 8;
-    const double start = tile == 128 ? 6.0 : tile == 64 ? 3.0 : 1.5;  // and the result's stores
-    // a slab of one workgroup: of several sharing a CU, and alone on it (the
-    // 16-bit matrix rate leaves a slab to its loads and LDS traffic)
-    const double shared = elem == 2 ? (tile == 128 ? 0.85 : tile == 64 ? 0.4 : 0.18)
-                                    : (tile == 128 ? 1.85 : tile == 64 ? 0.5 : 0.15);
-    const double alone = elem == 2 ? (tile == 128 ? 1.05 : tile == 64 ? 0.55 : 0.35)
-                                   : (tile == 128 ? 2.2 : tile == 64 ? 0.65 : 0.25);
-    for (int s = s0; s <= 65535; s *= 2) {
-      const double wgs = tiles * s;
-      if (s > s0 && (!may_split || nk / s < 4 || wgs > 2 * cus * per_cu)) break;
-      double t = rounds_us(wgs, per_cu, (nk + s - 1) / s, start, shared, alone);
-      if (s > 1) t += 4.0 + 2e-6 * s * (double)batch * M * N * (elem == 2 ? 4 : elem) / 6.0;
-      if (t < best.us * 0.98) best = Plan4{tile, s, t};
-    }
-  }
-  return best;
+// The general kernels' plan for this device; tile 0: no grid holds the output.
+inline mmpi::GemmPlan plan4(long long batch, int M, int N, int K, int elem, bool may_split) {
+  return mmpi::gemm_plan(batch, M, N, K, elem, may_split, mmpi::cu_count() > 0 ? mmpi::cu_count() : 256);
 }
 
 // The 256 x 256 kernel is used once the product has at least
@@ -1387,12 +1337,13 @@ int launch16(long long batch, int M, int N, int K, const void *A, long long lda,
                        ldc, sA, sB, sC, tm, tn);
     return mmpi::check_launch("mmp_matmul(mfma16 256x256)");
   }
-  Plan4 pl = plan4(batch, M, N, K, 2, true);
+  mmpi::GemmPlan pl = plan4(batch, M, N, K, 2, true);
   if (pl.splits > 1) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(mmpi::stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
       pl = plan4(batch, M, N, K, 2, false);
   }
+  if (!pl.tile) return mmpi::fail(MMP_E_ARG, "matmul grid too large");
   constexpr int BK = 64;
   if (pl.tile == 128 && pl.splits == 1 && M % 128 == 0 && N % 128 == 0 && K % BK == 0 &&
       lda % 8 == 0 && ldb % 4 == 0 && sA % 8 == 0 && sB % 4 == 0 && al(A, 16) && al(B, 8)) {
@@ -1403,7 +1354,8 @@ int launch16(long long batch, int M, int N, int K, const void *A, long long lda,
   }
   const int nk = (K + BK - 1) / BK, kspan = (nk + pl.splits - 1) / pl.splits;
   const int splits = (nk + kspan - 1) / kspan, tile = pl.tile;
-  const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
+  const int tiles_m = (int)(((long long)M + tile - 1) / tile);
+  const int tiles_n = (int)(((long long)N + tile - 1) / tile);
   const long long total = (long long)M * N * batch;
   const int edge = (K % BK || N % tile ? 1 : 0) | (lda < 7 || lda >= (1LL << 24) ? 2 : 0) |
                    (ldb < 3 || ldb >= (1LL << 24) ? 4 : 0);
@@ -1441,18 +1393,20 @@ int launch_general(long long batch, int M, int N, int K, const T *A, long long l
   constexpr int V = 16 / sizeof(T), BK = 128 / sizeof(T);
   // partial products need scratch memory: none while the stream is captured
   // (a graph's replays would outlive it)
-  Plan4 pl = plan4(batch, M, N, K, (int)sizeof(T), !sub);
+  mmpi::GemmPlan pl = plan4(batch, M, N, K, (int)sizeof(T), !sub);
   if (pl.splits > 1) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(mmpi::stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
       pl = plan4(batch, M, N, K, (int)sizeof(T), false);
   }
+  if (!pl.tile) return mmpi::fail(MMP_E_ARG, "matmul grid too large");
   const int nk = (K + BK - 1) / BK;
   const int kspan = (nk + pl.splits - 1) / pl.splits;
   const int splits = (nk + kspan - 1) / kspan;
   const long long total = (long long)M * N * batch;
   const int tile = pl.tile;
-  const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
+  const int tiles_m = (int)(((long long)M + tile - 1) / tile);
+  const int tiles_n = (int)(((long long)N + tile - 1) / tile);
   // see the kernel: short rows a vector could run past, or offsets past 32 bits
   const bool guard_a = lda < V - 1 || lda >= (1LL << 24);
   const bool guard_b = ldb < V - 1 || ldb >= (1LL << 24);
@@ -1522,7 +1476,8 @@ int launch4(int ta, int tb, long long batch, int M, int N, int K, const void *A,
       // CUs (32 of 384^3 53 -> 43 us); near the line
       // the copies win (256 of 128^3 14.5 us against 16.3, 16 of 512^3 38
       // against 42)
-      if (rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 4.0, 1.6, 1.9) <=
+      if (mmpi::rounds_us((double)tiles_m * tiles_n * (double)batch, 2, K / BK, 4.0, 1.6, 1.9,
+                          mmpi::cu_count() > 0 ? mmpi::cu_count() : 256) <=
           1.07 * plan4(batch, M, N, K, 4, true).us) {
         hipLaunchKernelGGL(k_gemm4_dma, dim3((unsigned)(tiles_m * tiles_n), (unsigned)batch),
                            dim3(kBlock), 0, mmpi::stream(), (const float *)A, (const float *)B,

@@ -13,6 +13,9 @@ enum { SCRATCH_REDUCE_PARTIALS = 0, SCRATCH_REDUCE_TICKETS = 1,
        SCRATCH_SCAN_FLAGS = 2, SCRATCH_SCAN_VALUES = 3,
        SCRATCH_SCAN_COUNTER = 4, SCRATCH_REDUCE_PLAIN = 5, SCRATCH_NSLOTS = 6 };
 
+// HIP counts at most 2^32 - 1 work-items per grid dimension.
+inline bool grid_fits(long long blocks, int threads) { return blocks <= 0xffffffffLL / threads; }
+
 // Strided layouts: the split of the reduced axis that leaves the CUs most
 // evenly loaded, up to `per_cu` workgroups each and at least 64 steps of rows
 // (`steps`: rows over the rows a workgroup's lanes lie on side by side) to a
@@ -97,6 +100,64 @@ inline bool second_kernel(int splits, long long bytes) {
 // Where the partials of a strided reduction lie.
 inline int partials_slot(bool second) {
   return second ? SCRATCH_REDUCE_PLAIN : SCRATCH_REDUCE_PARTIALS;
+}
+
+// Tile and K split of the general kernels.  With few output tiles most
+// CUs would idle, so the tile is made smaller or the K range cut as well; a
+// split pays for its partial products (written once, read once).  The choice
+// is the cheapest by this estimate, in microseconds: rounds of workgroups
+// over the CUs (two 128, four 64 or eight 32 wide tiles fit one), each a
+// start-up plus its slabs, at the matrix cores' rate for the workgroups that
+// share a CU but no faster than one alone hides its loads; and the partials
+// at 6 TB/s plus a launch.  At most 16,384 outputs over a K of 16,384 or more
+// are always cut into ranges of at most 2048, whose sums meet in float64:
+// float32 sums of 10^7 terms then stay within 5e-8 of exact (2e-6 with ranges
+// of 6000).  Measured over tiles and splits, the choice is the
+// fastest or within a tenth of it: float32 1000^3 28 us (32 wide, unsplit; 64
+// wide 30, 128 wide in four splits 34), 2049^3 198 (64 wide; 128 wide 231),
+// 4000 x 70 x 3000 35 (32 wide in two; unsplit 128 wide 94); float64 500 x 500
+// x 100,000 0.84 ms (128 wide in 32; unsplit 15.8).
+// A tile whose workgroups are more than a grid holds is no choice (from 2^29
+// rows of one column on 32 wide ones are).
+struct GemmPlan {
+  int tile;    // 128, 64 or 32; 0: none fits a grid
+  int splits;  // K ranges
+  double us;
+};
+inline double rounds_us(double wgs, double per_cu, double slabs, double start, double shared,
+                        double alone, double cus) {
+  const double full = __builtin_floor(wgs / (cus * per_cu)), rest = wgs - full * cus * per_cu;
+  const double share = __builtin_ceil(rest / cus);
+  const double step = shared * share > alone ? shared * share : alone;
+  return full * (start + slabs * shared * per_cu) + (rest > 0 ? start + slabs * step : 0.0);
+}
+inline GemmPlan gemm_plan(long long batch, int M, int N, int K, int elem, bool may_split,
+                          double cus) {
+  const int nk = (int)(((long long)K * elem + 127) / 128);
+  GemmPlan best{0, 1, 1e30};
+  const bool long_sum = may_split && batch == 1 && (double)M * N <= 16384 && K >= 16384;
+  const int s0 = !long_sum ? 1 : K < 2048 * 65535 ? (K + 2047) / 2048 : 65535;  // grid limit
+  for (int tile = 128; tile >= 32; tile /= 2) {
+    const long long one = (((long long)M + tile - 1) / tile) * (((long long)N + tile - 1) / tile);
+    if (!grid_fits(one, 256)) break;  // nor do smaller tiles
+    const double tiles = (double)one * (double)batch;
+    const double per_cu = tile == 128 ? 2 : tile == 64 ? 4 : 8;
+    const double start = tile == 128 ? 6.0 : tile == 64 ? 3.0 : 1.5;  // and the result's stores
+    // a slab of one workgroup: of several sharing a CU, and alone on it (the
+    // 16-bit matrix rate leaves a slab to its loads and LDS traffic)
+    const double shared = elem == 2 ? (tile == 128 ? 0.85 : tile == 64 ? 0.4 : 0.18)
+                                    : (tile == 128 ? 1.85 : tile == 64 ? 0.5 : 0.15);
+    const double alone = elem == 2 ? (tile == 128 ? 1.05 : tile == 64 ? 0.55 : 0.35)
+                                   : (tile == 128 ? 2.2 : tile == 64 ? 0.65 : 0.25);
+    for (int s = s0; s <= 65535; s *= 2) {
+      const double wgs = tiles * s;
+      if (s > s0 && (!may_split || nk / s < 4 || wgs > 2 * cus * per_cu)) break;
+      double t = rounds_us(wgs, per_cu, (nk + s - 1) / s, start, shared, alone, cus);
+      if (s > 1) t += 4.0 + 2e-6 * s * (double)batch * M * N * (elem == 2 ? 4 : elem) / 6.0;
+      if (t < best.us * 0.98) best = GemmPlan{tile, s, t};
+    }
+  }
+  return best;
 }
 
 }  // namespace mmpi

@@ -1,5 +1,5 @@
 """Launch plans (mmp_plan.h), compiled for the host: where a reduction's
-partials lie."""
+partials lie, and grids that HIP accepts."""
 import ctypes
 import os
 import shutil
@@ -20,6 +20,13 @@ void t_reduce(int arg, int elem, long long outer, long long len, long long inner
   out[0] = p.splits;
   out[1] = mmpi::second_kernel(p.splits, outer * len * inner * elem);
   out[2] = mmpi::partials_slot(out[1]);
+}
+// out: tile, K ranges, workgroups of a matrix
+void t_gemm(long long batch, int m, int n, int k, int elem, int may_split, long long *out) {
+  const mmpi::GemmPlan p = mmpi::gemm_plan(batch, m, n, k, elem, may_split != 0, 256);
+  out[0] = p.tile;
+  out[1] = p.splits;
+  out[2] = p.tile ? ((m + (long long)p.tile - 1) / p.tile) * ((n + (long long)p.tile - 1) / p.tile) : 0;
 }
 int t_tagged_slot() { return mmpi::SCRATCH_REDUCE_PARTIALS; }
 int t_slots() { return mmpi::SCRATCH_NSLOTS; }
@@ -64,3 +71,30 @@ def test_raw_partials_stay_out_of_the_tagged_words(plans):
                         assert (slot == plans.t_tagged_slot()) == (not second)
                         seen.add((splits > 1, second))
     assert seen == {(False, 0), (True, 0), (True, 1)}  # every kind came up
+
+
+MAX_ITEMS = 0xFFFFFFFF  # work-items per grid dimension
+
+
+def _gemm(plans, batch, m, n, k, elem, may_split=True):
+    out = (ctypes.c_longlong * 3)()
+    plans.t_gemm(ctypes.c_longlong(batch), m, n, k, elem, int(may_split), out)
+    return tuple(out)
+
+
+@pytest.mark.parametrize("elem", [2, 4, 8])
+def test_product_grids_fit(plans, elem):
+    """Tall and wide products: no tile whose workgroups pass the limit of a
+    grid is chosen, and wherever 128 wide tiles fit there is a plan."""
+    for rows in (1 << 20, 500_000_000, (1 << 29) - 31, 1 << 29, (1 << 29) + 1, 600_000_000, 1 << 30,
+                 (1 << 31) - 200):
+        for cols in (1, 2, 31, 32, 33, 100, 129):
+            for k in (1, 2, 32, 100):
+                for m, n in ((rows, cols), (cols, rows)):
+                    tile, splits, wgs = _gemm(plans, 1, m, n, k, elem)
+                    wide = -(-m // 128) * -(-n // 128)
+                    assert (tile != 0) == (wide * 256 <= MAX_ITEMS), (m, n, k)
+                    assert wgs * 256 <= MAX_ITEMS and 1 <= splits <= 65535, (m, n, k, tile)
+    assert _gemm(plans, 1, (1 << 31) - 1, 1, 2, elem)[0] == 0  # 2^24 tiles of 128
+    # the largest that 32 wide tiles are laid over
+    assert _gemm(plans, 1, (1 << 29) - 32, 1, 2, elem)[0] == 32
