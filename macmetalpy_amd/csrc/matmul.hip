@@ -1314,8 +1314,31 @@ __global__ __launch_bounds__(kBlock) void k_gemm_int(const T *__restrict__ A, co
 inline bool al(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
 // The general kernels' plan for this device; tile 0: no grid holds the output.
+// K ranges take scratch memory for their partial products, so there are none
+// while the stream is captured (a graph's replays would outlive it).
 inline mmpi::GemmPlan plan4(long long batch, int M, int N, int K, int elem, bool may_split) {
-  return mmpi::gemm_plan(batch, M, N, K, elem, may_split, mmpi::cu_count() > 0 ? mmpi::cu_count() : 256);
+  const double cus = mmpi::cu_count() > 0 ? mmpi::cu_count() : 256;
+  if (may_split) {
+    const mmpi::GemmPlan pl = mmpi::gemm_plan(batch, M, N, K, elem, true, cus);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (pl.splits == 1 || (hipStreamIsCapturing(mmpi::stream(), &cap) == hipSuccess &&
+                           cap == hipStreamCaptureStatusNone))
+      return pl;
+  }
+  return mmpi::gemm_plan(batch, M, N, K, elem, false, cus);
+}
+
+// plan4 with the memory for its partial products of `bytes` each.  The product
+// itself needs none: without it, it runs in one range.
+inline int plan_with_partials(long long batch, int M, int N, int K, int elem, bool may_split,
+                              size_t bytes, mmpi::GemmPlan *pl, void **part) {
+  *part = nullptr;
+  *pl = plan4(batch, M, N, K, elem, may_split);
+  if (pl->splits > 1 && mmp_alloc((size_t)pl->splits * bytes, part) != MMP_OK) {
+    *part = nullptr;
+    *pl = plan4(batch, M, N, K, elem, false);
+  }
+  return pl->tile ? MMP_OK : mmpi::fail(MMP_E_ARG, "matmul grid too large");
 }
 
 // The 256 x 256 kernel is used once the product has at least
@@ -1337,13 +1360,10 @@ int launch16(long long batch, int M, int N, int K, const void *A, long long lda,
                        ldc, sA, sB, sC, tm, tn);
     return mmpi::check_launch("mmp_matmul(mfma16 256x256)");
   }
-  mmpi::GemmPlan pl = plan4(batch, M, N, K, 2, true);
-  if (pl.splits > 1) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(mmpi::stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
-      pl = plan4(batch, M, N, K, 2, false);
-  }
-  if (!pl.tile) return mmpi::fail(MMP_E_ARG, "matmul grid too large");
+  const long long total = (long long)M * N * batch;
+  mmpi::GemmPlan pl;
+  void *part;
+  if (int st = plan_with_partials(batch, M, N, K, 2, true, (size_t)total * 4, &pl, &part)) return st;
   constexpr int BK = 64;
   if (pl.tile == 128 && pl.splits == 1 && M % 128 == 0 && N % 128 == 0 && K % BK == 0 &&
       lda % 8 == 0 && ldb % 4 == 0 && sA % 8 == 0 && sB % 4 == 0 && al(A, 16) && al(B, 8)) {
@@ -1352,11 +1372,9 @@ int launch16(long long batch, int M, int N, int K, const void *A, long long lda,
                        lda, ldb, ldc, sA, sB, sC, N / 128);
     return mmpi::check_launch("mmp_matmul(mfma16 128x128)");
   }
-  const int nk = (K + BK - 1) / BK, kspan = (nk + pl.splits - 1) / pl.splits;
-  const int splits = (nk + kspan - 1) / kspan, tile = pl.tile;
+  const int kspan = pl.kspan, splits = pl.splits, tile = pl.tile;
   const int tiles_m = (int)(((long long)M + tile - 1) / tile);
   const int tiles_n = (int)(((long long)N + tile - 1) / tile);
-  const long long total = (long long)M * N * batch;
   const int edge = (K % BK || N % tile ? 1 : 0) | (lda < 7 || lda >= (1LL << 24) ? 2 : 0) |
                    (ldb < 3 || ldb >= (1LL << 24) ? 4 : 0);
   const T *a = (const T *)A, *b = (const T *)B;
@@ -1377,8 +1395,6 @@ int launch16(long long batch, int M, int N, int K, const void *A, long long lda,
     return mmpi::check_launch("mmp_matmul(mfma16)");
   };
   if (splits == 1) return go((T *)C, ldc, sC, 0);
-  void *part = nullptr;
-  if (int st = mmp_alloc((size_t)splits * (size_t)total * 4, &part)) return st;
   int st = go((float *)part, N, (long long)M * N, total);
   if (st == MMP_OK)
     st = launch_sum_splits<float, T>((const float *)part, (T *)C, M, N, ldc, sC, total, splits);
@@ -1391,19 +1407,13 @@ int launch_general(long long batch, int M, int N, int K, const T *A, long long l
                    const T *B, long long ldb, long long sB, T *C, long long ldc, long long sC,
                    bool sub) {
   constexpr int V = 16 / sizeof(T), BK = 128 / sizeof(T);
-  // partial products need scratch memory: none while the stream is captured
-  // (a graph's replays would outlive it)
-  mmpi::GemmPlan pl = plan4(batch, M, N, K, (int)sizeof(T), !sub);
-  if (pl.splits > 1) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(mmpi::stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
-      pl = plan4(batch, M, N, K, (int)sizeof(T), false);
-  }
-  if (!pl.tile) return mmpi::fail(MMP_E_ARG, "matmul grid too large");
-  const int nk = (K + BK - 1) / BK;
-  const int kspan = (nk + pl.splits - 1) / pl.splits;
-  const int splits = (nk + kspan - 1) / kspan;
   const long long total = (long long)M * N * batch;
+  mmpi::GemmPlan pl;
+  void *part;
+  if (int st = plan_with_partials(batch, M, N, K, (int)sizeof(T), !sub, (size_t)total * sizeof(T), &pl,
+                                  &part))
+    return st;
+  const int kspan = pl.kspan, splits = pl.splits;
   const int tile = pl.tile;
   const int tiles_m = (int)(((long long)M + tile - 1) / tile);
   const int tiles_n = (int)(((long long)N + tile - 1) / tile);
@@ -1415,11 +1425,9 @@ int launch_general(long long batch, int M, int N, int K, const T *A, long long l
   // one past each operand's last element
   const T *Aend = A + (batch - 1) * sA + (TA ? (K - 1LL) * lda + M : (M - 1LL) * lda + K);
   const T *Bend = B + (batch - 1) * sB + (TB ? (N - 1LL) * ldb + K : (K - 1LL) * ldb + N);
-  void *part = nullptr;
   T *out = C;
   long long oldc = ldc, osC = sC, osZ = 0;
   if (splits > 1) {
-    if (int st = mmp_alloc((size_t)splits * (size_t)total * sizeof(T), &part)) return st;
     out = (T *)part;
     oldc = N;
     osC = (long long)M * N;

@@ -122,6 +122,7 @@ inline int partials_slot(bool second) {
 struct GemmPlan {
   int tile;    // 128, 64 or 32; 0: none fits a grid
   int splits;  // K ranges
+  int kspan;   // 128-byte slabs of K in each but the last
   double us;
 };
 inline double rounds_us(double wgs, double per_cu, double slabs, double start, double shared,
@@ -134,7 +135,7 @@ inline double rounds_us(double wgs, double per_cu, double slabs, double start, d
 inline GemmPlan gemm_plan(long long batch, int M, int N, int K, int elem, bool may_split,
                           double cus) {
   const int nk = (int)(((long long)K * elem + 127) / 128);
-  GemmPlan best{0, 1, 1e30};
+  GemmPlan best{0, 1, nk, 1e30};
   const bool long_sum = may_split && batch == 1 && (double)M * N <= 16384 && K >= 16384;
   const int s0 = !long_sum ? 1 : K < 2048 * 65535 ? (K + 2047) / 2048 : 65535;  // grid limit
   for (int tile = 128; tile >= 32; tile /= 2) {
@@ -154,9 +155,11 @@ inline GemmPlan gemm_plan(long long batch, int M, int N, int K, int elem, bool m
       if (s > s0 && (!may_split || nk / s < 4 || wgs > 2 * cus * per_cu)) break;
       double t = rounds_us(wgs, per_cu, (nk + s - 1) / s, start, shared, alone, cus);
       if (s > 1) t += 4.0 + 2e-6 * s * (double)batch * M * N * (elem == 2 ? 4 : elem) / 6.0;
-      if (t < best.us * 0.98) best = GemmPlan{tile, s, t};
+      if (t < best.us * 0.98) best = GemmPlan{tile, s, 0, t};
     }
   }
+  best.kspan = (nk + best.splits - 1) / best.splits;
+  best.splits = (nk + best.kspan - 1) / best.kspan;
   return best;
 }
 

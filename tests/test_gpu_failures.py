@@ -180,3 +180,27 @@ def test_rawkernel_compile_error_carries_the_log(be):
     k = cp.RawKernel('extern "C" __global__ void bad(float* x) { x[0] = undefined_name; }', "bad")
     with pytest.raises(HipError, match="undefined_name"):
         k((64,), (cp.zeros(64, dtype=np.float32),))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.float16])
+@pytest.mark.parametrize("m,n,k", [(64, 64, 6000), (500, 500, 30000), (4, 4, 300_000)])
+def test_product_without_memory_for_partials(be, m, n, k, dtype):
+    """A product that would split its K range runs in one range when there is
+    no memory for the partial products (it needs none itself), and leaves
+    nothing allocated.  Integer values keep every sum exact."""
+    from macmetalpy_amd._dtypes import dtype_code
+    g = np.random.default_rng(k)
+    a, b = (g.integers(-1, 2, s).astype(dtype) for s in ((m, k), (k, n)))
+    b[2000:] = 0  # float16: sums stay below 2048
+    want = a[:, :2000].astype(np.float64) @ b[:2000].astype(np.float64)
+    da, db, c = (cp.array(x)._ensure_gpu() for x in (a, b, np.full((m, n), 7, dtype)))
+    code = dtype_code(np.dtype(dtype))
+    before = _in_use()
+    for armed in (True, False):
+        if armed:
+            be.debug_fail_next(1, 1)
+        be.matmul(code, 1, m, n, k, da._ptr, k, 0, db._ptr, n, 0, c._ptr, n, 0)
+        assert np.array_equal(c.get(), want.astype(dtype))
+        assert _in_use() == before
+    # the failure was met, by the first product: an allocation works again
+    assert be.create_buffer(16, np.dtype(np.float32)).ptr
