@@ -85,6 +85,22 @@ inline ColPlan argreduce_cols_plan(long long outer, long long len, long long inn
   return p;
 }
 
+// Axes so short that a workgroup of the plans above spends its time bringing
+// lanes and waves together: a thread per `vec` columns that walks the axis by
+// itself.  Up to `rows` of them always (us, plans above / a thread per columns;
+// sum, maximum, argmax over the middle axis): float32 60,000 x 16 x 9 90 / 8.5,
+// 91 / 8.9, 90 / 7.9; 625 x 16 x 1000 9.4 / 9.1, 9.9 / 9.5, 8.6 / 8.7; float16
+// 1 x 16 x 1,250,001 12.1 / 9.5, 13.7 / 12.4, 11.9 / 11.8; 1 x 32 x 625,001 9.8 /
+// 9.5, 12.9 / 18, 10 / 12.1.  Further on only where rows are shorter than a
+// workgroup and workgroups so many that starting them is the time: float32
+// 17,361 x 64 x 9 28 / 8.5, 30 / 17, 40 / 10.8, but 3125 x 64 x 50 8.6 / 8.6, 10 /
+// 17, 10.4 / 9.9; `heavy` (extremes of floats) by half as much.
+inline bool short_axis(long long outer, long long len, long long inner, int vec, int rows, bool heavy) {
+  const long long vecs = inner >= vec ? (inner + vec - 1) / vec : inner;
+  if (outer * vecs > 0xffffff00LL) return false;  // threads of one grid
+  return len <= rows || (inner < 256 && len <= (heavy ? 64 : 128) && outer >= (heavy ? 128 : 64) * len);
+}
+
 // Partials of a strided reduction: few are combined by the last workgroup to
 // arrive; more are left as they are, (outer, split, column), for a second
 // kernel whose many workgroups read them side by side.  One workgroup alone

@@ -64,6 +64,33 @@ def test_few_columns_nan(rows, cols):
     assert np.array_equal(cp.sum(cp.array(inf), axis=0).get(), np.sum(inf, axis=0), equal_nan=True)
 
 
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("outer,length,inner", [(5000, 20, 9), (9000, 60, 3), (4, 1, 700), (70, 16, 300),
+                                                (70, 17, 301), (1, 2, 100_001), (40_000, 3, 2),
+                                                (600, 15, 130), (3, 8, 4099)])
+def test_short_axes(outer, length, inner, dt):
+    """Axes of a few rows (a thread walks one by itself): every remainder of
+    the row loop, whole and cut-off column vectors, rows shorter than one, an
+    input that starts at any element; NaN and infinities."""
+    g = np.random.default_rng(length)
+    h = _data(g, (outer + 1, length, inner), dt)
+    if np.dtype(dt).kind == "f":
+        h[g.integers(0, outer, 20), g.integers(0, length, 20), g.integers(0, inner, 20)] = np.nan
+        h[g.integers(0, outer, 20), g.integers(0, length, 20), g.integers(0, inner, 20)] = -np.inf
+    d = cp.array(h)
+    for x, y in ((d, h), (d[1:], h[1:])):
+        for name in ("sum", "max", "min", "argmax", "argmin"):
+            f, nf = getattr(cp, name), getattr(np, name)
+            wide = name == "sum" and np.dtype(dt).kind == "f"
+            want = nf(y.astype(np.float64) if wide else y, axis=1)
+            want = want.astype(dt) if wide else want
+            got = f(x, axis=1).get()
+            assert got.dtype == want.dtype and np.array_equal(got, want, equal_nan=wide or
+                                                              name in ("max", "min")), name
+    if np.dtype(dt).kind == "f":
+        assert np.array_equal(cp.nanmax(d, axis=1).get(), np.fmax.reduce(h, axis=1), equal_nan=True)
+
+
 def test_partials_of_one_call_do_not_reach_the_next():
     """Reductions that leave raw partials for a second kernel, whose values
     are the numbers that calls are tagged with, between reductions that know

@@ -12,14 +12,22 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = r"""
 #include "mmp_plan.h"
 extern "C" {
-// out: splits, second kernel, slot of the partials
+// out: splits, second kernel, slot of the partials, workgroups along the columns
 void t_reduce(int arg, int elem, long long outer, long long len, long long inner, long long *out) {
-  const int vec = elem == 1 ? 4 : 16 / elem;
+  const int vec = arg ? 1 : elem == 1 ? 4 : 16 / elem;
+  if (mmpi::short_axis(outer, len, inner, vec, 16, false)) {
+    out[0] = 1;
+    out[1] = 0;
+    out[2] = mmpi::partials_slot(false);
+    out[3] = (outer * ((inner + vec - 1) / vec) + 255) / 256;
+    return;
+  }
   const mmpi::ColPlan p = arg ? mmpi::argreduce_cols_plan(outer, len, inner, 256)
                               : mmpi::reduce_cols_plan(outer, len, inner, vec, 256);
   out[0] = p.splits;
   out[1] = mmpi::second_kernel(p.splits, outer * len * inner * elem);
   out[2] = mmpi::partials_slot(out[1]);
+  out[3] = p.ncb;
 }
 // out: tile, K ranges, workgroups of a matrix
 void t_gemm(long long batch, int m, int n, int k, int elem, int may_split, long long *out) {
@@ -48,7 +56,7 @@ def plans(tmp_path_factory):
 
 
 def _reduce(plans, arg, elem, outer, length, inner):
-    out = (ctypes.c_longlong * 3)()
+    out = (ctypes.c_longlong * 4)()
     i64 = ctypes.c_longlong
     plans.t_reduce(arg, elem, i64(outer), i64(length), i64(inner), out)
     return tuple(out)
@@ -66,7 +74,7 @@ def test_raw_partials_stay_out_of_the_tagged_words(plans):
                     for inner in (2, 3, 50, 257, 1001, 20_000):
                         if outer * length * inner > 2e9:
                             continue
-                        splits, second, slot = _reduce(plans, arg, elem, outer, length, inner)
+                        splits, second, slot, _ = _reduce(plans, arg, elem, outer, length, inner)
                         assert splits >= 1 and slot < plans.t_slots()
                         assert (slot == plans.t_tagged_slot()) == (not second)
                         seen.add((splits > 1, second))
@@ -74,6 +82,18 @@ def test_raw_partials_stay_out_of_the_tagged_words(plans):
 
 
 MAX_ITEMS = 0xFFFFFFFF  # work-items per grid dimension
+
+
+def test_reductions_of_very_wide_rows_fit_a_grid(plans):
+    """Down the columns of rows as wide as the memory of a device holds (two
+    of 2^33 bytes and more): as many columns as a thread each could cover."""
+    for elem in (1, 2, 4, 8):
+        for inner in ((1 << 31) - 1, (1 << 31) + 1, (1 << 32) - 257):
+            for length in (2, 3, 8, 16, 17, 40):
+                if elem * inner * length > 288 * 10**9:
+                    continue
+                for arg in (0, 1):
+                    assert _reduce(plans, arg, elem, 1, length, inner)[3] * 256 <= MAX_ITEMS
 
 
 def _gemm(plans, batch, m, n, k, elem, may_split=True):
