@@ -17,7 +17,7 @@ enum { SCRATCH_REDUCE_PARTIALS = 0, SCRATCH_REDUCE_TICKETS = 1,
 inline bool grid_fits(long long blocks, int threads) { return blocks <= 0xffffffffLL / threads; }
 
 // Strided layouts: the split of the reduced axis that leaves the CUs most
-// evenly loaded, up to `per_cu` workgroups each and at least 64 steps of rows
+// evenly loaded, up to `per_cu` workgroups each and at least `least` steps of rows
 // (`steps`: rows over the rows a workgroup's lanes lie on side by side) to a
 // split.  Workgroups of a launch of this size all run together, so what
 // counts is that each CU gets as many: 40 column blocks x 6 splits (240
@@ -27,15 +27,18 @@ inline bool grid_fits(long long blocks, int threads) { return blocks <= 0xffffff
 // 5.4, 2048: 5.3), the arg kernel with four (argmax 4.76 TB/s; 512: 3.2,
 // 2048: 4.45).
 constexpr int kColVecPerCu = 1, kColPerCu = 4;
-inline int col_splits(long long col_blocks, long long steps, int per_cu, long long cus) {
-  long long most = steps / 64;
+inline int col_splits(long long col_blocks, long long steps, int per_cu, long long cus,
+                      int least = 64) {
+  long long most = steps / least;
   if (most > 1024) most = 1024;
   // enough workgroups already without splitting, or too few rows to split
   if (col_blocks >= 4 * cus * per_cu || most <= 1) return 1;
-  // up to per_cu per CU; where the column blocks alone are about that many,
-  // a few more, which fill the CUs better
-  long long top = cus * per_cu / col_blocks;
-  if (top < 4) top = 4;
+  // up to per_cu per CU; where the column blocks alone are about that many, a
+  // few more of a long axis, which fill the CUs better (a short one's partials
+  // cost more than that: float32 300 x 300 x 300 over the middle axis, 600
+  // blocks, 23.3 us whole and 25.4 in halves)
+  long long top = (cus * per_cu + col_blocks - 1) / col_blocks;
+  if (top < 4 && steps >= 1024) top = 4;
   if (top > most) top = most;
   int best = 1;
   double best_fill = 0.0;
@@ -64,15 +67,27 @@ struct ColPlan {
   int splits;
 };
 // Sums and extremes: a lane on `vec` adjacent columns, or on one where the
-// rows are shorter than that.
-inline ColPlan reduce_cols_plan(long long outer, long long len, long long inner, int vec,
-                                long long cus) {
+// rows are shorter than that.  A CU with one workgroup has a wave per SIMD: too
+// few where the arithmetic is what an element costs.  So `heavy` ones
+// (comparisons and NaN rules) get two, and four of eight columns a lane, which
+// also split from half the rows on; and many one-byte elements two (10,000 x
+// 10,001 39 -> 28 us for a mean, 20 MB and less 10 -> 13).
+// Maximum over axis 0, one workgroup a CU before and now (the comparisons also
+// became one expression): float32 10,000 x 10,001 112 -> 70 us, 300,000 x 333 154
+// -> 82, 8 x 4000 x 1001 over the middle axis 36 -> 25; float16 99 -> 38, 133 ->
+// 39, 41 -> 17.
+inline ColPlan reduce_cols_plan(long long outer, long long len, long long inner, int vec, bool heavy,
+                                int elem, long long cus) {
   const int vi = inner >= vec ? vec : 1;
   ColPlan p{0, 0, 0, 1};
   while (p.lanes < 6 && ((long long)vi << p.lanes) < inner) ++p.lanes;
   p.cw = vi << p.lanes;
   p.ncb = (inner + p.cw - 1) / p.cw;
-  p.splits = col_splits(outer * p.ncb, len >> (6 - p.lanes), kColVecPerCu, cus);
+  const bool hard = heavy && vi > 1;
+  const int per_cu = hard                                              ? (vi >= 8 ? 4 : 2)
+                     : elem == 1 && outer * len * inner >= (64LL << 20) ? 2
+                                                                        : kColVecPerCu;
+  p.splits = col_splits(outer * p.ncb, len >> (6 - p.lanes), per_cu, cus, hard && vi >= 8 ? 32 : 64);
   return p;
 }
 // Arg-reductions: a thread per column.

@@ -112,10 +112,7 @@ template <typename T> struct Red<MMP_R_MAX, T> {
   }
   static __device__ __forceinline__ A map(T v) { return (A)v; }
   static __device__ __forceinline__ A comb(A a, A b) {
-    if constexpr (mmp_t<T>::is_float) {
-      if (a != a) return a;
-      if (b != b) return b;
-    }
+    if constexpr (mmp_t<T>::is_float) return a == a && !(b <= a) ? b : a;  // a NaN b is taken
     return b > a ? b : a;
   }
 };
@@ -128,10 +125,7 @@ template <typename T> struct Red<MMP_R_MIN, T> {
   }
   static __device__ __forceinline__ A map(T v) { return (A)v; }
   static __device__ __forceinline__ A comb(A a, A b) {
-    if constexpr (mmp_t<T>::is_float) {
-      if (a != a) return a;
-      if (b != b) return b;
-    }
+    if constexpr (mmp_t<T>::is_float) return a == a && !(b >= a) ? b : a;  // a NaN b is taken
     return b < a ? b : a;
   }
 };
@@ -164,12 +158,9 @@ template <int OP, typename T> struct RedNanExt {  // OP: MMP_R_MAX or MMP_R_MIN
   }
   static __device__ __forceinline__ A map(T v) { return (A)v; }
   static __device__ __forceinline__ A comb(A a, A b) {
-    if constexpr (mmp_t<T>::is_float) {
-      if (a != a) return b;
-      if (b != b) return a;
-    }
-    if constexpr (OP == MMP_R_MAX) return b > a ? b : a;
-    else return b < a ? b : a;
+    // a NaN a is replaced, a NaN b is not taken
+    if constexpr (OP == MMP_R_MAX) return b > a || a != a ? b : a;
+    else return b < a || a != a ? b : a;
   }
 };
 template <typename T> struct Red<MMP_R_NANMAX, T> : RedNanExt<MMP_R_MAX, T> {};
@@ -923,7 +914,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_cols(const T *__restrict__ x,
 // time on when each lane has only a few rows.
 // float32 30,000 x 20 x 9 over the middle axis, sum 46 us with those, 18.7 with a
 // workgroup per outer index and a thread per column, 8.6 so; 2 x 3,000,000 over
-// axis 0 12, 9.7 and 10; float16 30,000 x 20 x 9 108, 16.7 and 9.
+// axis 0 12, 9.7 and 8.7; float16 30,000 x 20 x 9 108, 16.7 and 9.
 // A thread's outputs are at most 32 bytes, so that a wave's lie together
 // (int16 sums, 8 bytes each, of 2 x 3,000,000 15 us with eight columns, 10 with
 // four).
@@ -1111,7 +1102,8 @@ int launch_reduce(long long outer, long long len, long long inner, const void *x
     return mmpi::check_launch("mmp_reduce(short axis)");
   }
   const bool vec = inner >= col_vec<T>();
-  const mmpi::ColPlan pl = mmpi::reduce_cols_plan(outer, len, inner, col_vec<T>(), cus());
+  const mmpi::ColPlan pl = mmpi::reduce_cols_plan(outer, len, inner, col_vec<T>(), heavy<OP, T>(),
+                                                  (int)sizeof(T), cus());
   const int cw = pl.cw, lg = pl.lanes;
   const long long ncb = pl.ncb;
   int S = pl.splits;

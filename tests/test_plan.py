@@ -23,7 +23,7 @@ void t_reduce(int arg, int elem, long long outer, long long len, long long inner
     return;
   }
   const mmpi::ColPlan p = arg ? mmpi::argreduce_cols_plan(outer, len, inner, 256)
-                              : mmpi::reduce_cols_plan(outer, len, inner, vec, 256);
+                              : mmpi::reduce_cols_plan(outer, len, inner, vec, elem == 2, elem, 256);
   out[0] = p.splits;
   out[1] = mmpi::second_kernel(p.splits, outer * len * inner * elem);
   out[2] = mmpi::partials_slot(out[1]);
@@ -35,6 +35,12 @@ void t_gemm(long long batch, int m, int n, int k, int elem, int may_split, long 
   out[0] = p.tile;
   out[1] = p.splits;
   out[2] = p.tile ? ((m + (long long)p.tile - 1) / p.tile) * ((n + (long long)p.tile - 1) / p.tile) : 0;
+}
+// workgroups of a strided reduction
+long long t_groups(int heavy, int elem, long long outer, long long len, long long inner) {
+  const mmpi::ColPlan p =
+      mmpi::reduce_cols_plan(outer, len, inner, elem == 1 ? 4 : 16 / elem, heavy != 0, elem, 256);
+  return outer * p.ncb * p.splits;
 }
 int t_tagged_slot() { return mmpi::SCRATCH_REDUCE_PARTIALS; }
 int t_slots() { return mmpi::SCRATCH_NSLOTS; }
@@ -79,6 +85,22 @@ def test_raw_partials_stay_out_of_the_tagged_words(plans):
                         assert (slot == plans.t_tagged_slot()) == (not second)
                         seen.add((splits > 1, second))
     assert seen == {(False, 0), (True, 0), (True, 1)}  # every kind came up
+
+
+def test_workgroups_of_strided_reductions(plans):
+    """About one workgroup a CU (256), two and four where comparisons of floats
+    are what an element costs, and no short axis cut although its column blocks
+    alone outnumber the CUs."""
+    plans.t_groups.restype = ctypes.c_longlong
+
+    def groups(heavy, elem, *shape):
+        return plans.t_groups(heavy, elem, *(ctypes.c_longlong(v) for v in shape))
+
+    for shape in ((1, 10_000, 10_001), (8, 4000, 1001), (1, 300_000, 333)):
+        assert 200 <= groups(0, 4, *shape) <= 256 and 200 <= groups(0, 2, *shape) <= 256
+        assert 400 <= groups(1, 4, *shape) <= 512 and 800 <= groups(1, 2, *shape) <= 1024
+    assert groups(0, 1, 1, 10_000, 10_001) > 400 and groups(0, 1, 20, 30_000, 30) <= 256
+    assert groups(0, 4, 300, 300, 300) == 600 and groups(0, 4, 1, 300, 90_000) == 352
 
 
 MAX_ITEMS = 0xFFFFFFFF  # work-items per grid dimension
