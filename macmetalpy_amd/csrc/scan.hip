@@ -957,11 +957,8 @@ int launch_scan(long long outer, long long len, long long inner, const void *x, 
     if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided scan: outer extent %lld > 65535", outer);
     if constexpr (sizeof(Ti) >= 2) {
       constexpr int VI = scan_col_vec<Ti>();
-      // whole aligned vectors; or four or more columns a vector and enough rows
-      // to split (float32 50,000 x 1001 155 -> 126 us; float64 3000 x 3001 is
-      // quicker by column, 36 against 42, and so is 100 x 300,001)
       if ((inner % VI == 0 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)y & 15u) == 0) ||
-          (VI >= 4 && inner >= VI && len >= 128))
+          mmpi::scan_cols_by_vector(len, inner, (int)sizeof(Ti), (int)sizeof(To)))
         return launch_scan_cols_vec<OP, Ti, To>(outer, len, inner, x, y);
     }
     const long long ncb = mmpi::ceil_div(inner, kBlock);

@@ -42,6 +42,9 @@ long long t_groups(int heavy, int elem, long long outer, long long len, long lon
       mmpi::reduce_cols_plan(outer, len, inner, elem == 1 ? 4 : 16 / elem, heavy != 0, elem, 256);
   return outer * p.ncb * p.splits;
 }
+int t_scan(long long len, long long inner, int in, int out) {
+  return mmpi::scan_cols_by_vector(len, inner, in, out);
+}
 int t_tagged_slot() { return mmpi::SCRATCH_REDUCE_PARTIALS; }
 int t_slots() { return mmpi::SCRATCH_NSLOTS; }
 }
@@ -140,3 +143,14 @@ def test_product_grids_fit(plans, elem):
     assert _gemm(plans, 1, (1 << 31) - 1, 1, 2, elem)[0] == 0  # 2^24 tiles of 128
     # the largest that 32 wide tiles are laid over
     assert _gemm(plans, 1, (1 << 29) - 32, 1, 2, elem)[0] == 32
+
+
+@pytest.mark.parametrize("length,inner,sizes,vector", [
+    (10_000, 33, (4, 4), 1), (30_000, 1001, (4, 4), 1), (256, 100_001, (4, 4), 1), (3000, 1001, (4, 4), 1),
+    (1000, 1001, (4, 4), 0), (3000, 3001, (4, 4), 0), (256, 16_385, (4, 4), 0), (256, 65_537, (4, 4), 0),
+    (1_000_000, 33, (4, 4), 0), (10_000, 3, (4, 4), 0), (10_000, 333, (4, 8), 1), (100_000, 33, (4, 8), 1),
+    (3000, 1001, (4, 8), 0), (100_000, 5, (4, 8), 0), (1000, 40_001, (4, 8), 0), (10_000, 1001, (2, 2), 0),
+    (200, 50_001, (2, 2), 0), (10_000, 1001, (8, 8), 0)])
+def test_column_scans_by_vector(plans, length, inner, sizes, vector):
+    """The layout that was quicker for rows that are no whole aligned vectors."""
+    assert plans.t_scan(ctypes.c_longlong(length), ctypes.c_longlong(inner), *sizes) == vector
