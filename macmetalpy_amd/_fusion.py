@@ -405,6 +405,45 @@ _FLAT_UNROLL = 4  # 4-element vectors per thread of a flat kernel
 _FLAT_MIN = 1 << 16
 
 
+def _flat_cols(kinds, cols, n, wide, spread, tile):
+    """Whether rows of ``cols`` elements of at most ``wide`` bytes go flat, ``n``
+    elements in all.
+
+    A vector of a flat launch reads four elements of a row vector (or of an odd
+    row) one by one, which costs more than the row launch's scalar rows as long
+    as the data stay in the caches; the vectors are worth it where memory
+    streams.  Us by rows / flat for (x - r) * r with a row vector, (x - c) * c
+    with a value per row, r * c.  float32, 12,000,000 elements: 511 columns 19.6 /
+    19.5, 19.4 / 16.8, 17.2 / 16.8; 1023 16.9 / 19.5, 16.9 / 16.8, 12.8 / 16.8;
+    3001 16.2 / 19.9, 16.1 / 16.9, 10.5 / 16.9; 4097 (a tile and one element)
+    23.3 / 20.2, 23.3 / 16.7, 16.6 / 16.6; whole vectors: 900 17.7 / 16.7, 17.7 /
+    17, 13.3 / 9.1; 3500 16.3 / 17.2, 16.3 / 17, 10.8 / 8.8.  70,000,000: 511 156 /
+    97, 156 / 92, 89 / 76; 1023 132 / 97, 132 / 91, 66 / 76; 10,001 127 / 99, 127 /
+    91, 60 / 77; 3500 125 / 93, 126 / 91, 59 / 52.
+    float16, 12,000,000: 1023 14.2 / 13.8, 14.3 / 10.6, 11.1 / 11.4; 3001 12.4 /
+    13.9, 12.4 / 10.6, 9.5 / 11.2; 70,000,000: 3001 88 / 72, 87 / 47, 37 / 48.
+    float64 (32 bytes a thread), 12,000,000: 130 48 / 43, 48 / 42, 46 / 36; 200
+    36.5 / 39, 36 / 38, 35 / 34; 1023 29 / 45, 29 / 42, 20 / 35; with padded rows
+    ('v') 300 53 / 48, 700 48 / 49; with a transposed leaf (``spread``) 255 64 / 42;
+    70,000,000: 300 246 / 225, 241 / 220, 215 / 240; 511 201 / 259, 200 / 244, 176 /
+    246; 5001 335 / 266, 277 / 243, 159 / 239."""
+    big = n * wide >= 1 << 27
+    streams = "f" in kinds or "v" in kinds
+    empty = -(-cols // tile) * tile / cols if cols > tile else 1.0  # the row launch's tiles
+    if wide == 8:
+        limit = (400 if "v" in kinds else 255 if spread else 160 if not big else
+                 300 if streams else 200)
+        return cols <= limit or (big and streams and empty >= 1.36)
+    if cols % _ELEMS == 0:
+        return big or wide < 4 or cols <= 2048
+    if "p" not in kinds and "g" not in kinds:  # nothing read along an odd row
+        return big or wide < 4 or cols <= 1024 or cols > tile
+    if big and streams:
+        return True
+    return (cols <= (1024 if wide < 4 else 800 if big else 512)
+            or empty >= (1.6 if wide < 4 else 1.7))
+
+
 def _flat_kinds(outer, cols, leaf_str, ptrs, itemsizes, out_ptr, out_itemsize, tile):
     """Leaf classes of a flat launch, or None where the row launch stays.
 
@@ -420,8 +459,8 @@ def _flat_kinds(outer, cols, leaf_str, ptrs, itemsizes, out_ptr, out_itemsize, t
     'g' for any other strides, whose loads are spread too wide to take long
     rows flat).  (x - m) / d of a
     2,000,000 x 50 float32 x and row vectors m, d: 655 us by rows,
-    134 flat (6 TB/s); 12,000,000 x 8: 4965 and 126; 10,000 x 10,001: 182 and
-    140."""
+    134 flat (6 TB/s); 12,000,000 x 8: 4965 and 126.  How long rows may be is
+    _flat_cols's to say."""
     if len(outer) != 1 or (cols >= tile and cols % _ELEMS == 0):
         return None
     if not _FLAT_MIN <= outer[0] * cols < 1 << 31 or out_ptr % (_ELEMS * out_itemsize):
@@ -442,7 +481,9 @@ def _flat_kinds(outer, cols, leaf_str, ptrs, itemsizes, out_ptr, out_itemsize, t
             kinds.append("g")
         else:
             return None
-    return kinds
+    wide = max(itemsizes + [out_itemsize])
+    spread = any(k == "g" and st[1] != 1 for k, st in zip(kinds, leaf_str))
+    return kinds if _flat_cols(kinds, cols, outer[0] * cols, wide, spread, tile) else None
 
 
 def _flat_body(kinds, ct, vtypes, out_ct, expr_lines, res):

@@ -1185,23 +1185,44 @@ bool vec_ok(const Plan &pl, bool out_ok) {
   return true;
 }
 
+// The Python _flat_cols, which says why.
+bool flat_cols(const std::string &kinds, long long cols, long long n, int wide, bool spread,
+               long long tile) {
+  auto has = [&](char k) { return kinds.find(k) != std::string::npos; };
+  const bool big = n * wide >= 1LL << 27, streams = has('f') || has('v');
+  const double empty = cols > tile ? (double)((cols + tile - 1) / tile * tile) / (double)cols : 1.0;
+  if (wide == 8) {
+    const long long limit = has('v') ? 400 : spread ? 255 : !big ? 160 : streams ? 300 : 200;
+    return cols <= limit || (big && streams && empty >= 1.36);
+  }
+  if (cols % 4 == 0) return big || wide < 4 || cols <= 2048;
+  if (!has('p') && !has('g')) return big || wide < 4 || cols <= 1024 || cols > tile;
+  if (big && streams) return true;
+  return cols <= (wide < 4 ? 1024 : big ? 800 : 512) || empty >= (wide < 4 ? 1.6 : 1.7);
+}
+
 bool flat_kinds(const Plan &pl, unsigned long long outp, int out_dt, std::string *kinds) {
   if (pl.nouter != 1 || (pl.cols >= map_tile(pl.kinds) && pl.cols % 4 == 0)) return false;
   const long long n = pl.rows * pl.cols;
   if (n < kFlatMin || n >= (1LL << 31) || outp % (4ull * itemsize[out_dt])) return false;
   const bool whole = pl.cols % 4 == 0;
+  int wide = (int)itemsize[out_dt];
+  bool spread = false;
   kinds->clear();
   for (size_t k = 0; k < pl.p.leaves.size(); ++k) {
     const long long row = pl.cst[k][0], col = pl.cst[k][1];
+    if ((int)itemsize[pl.p.leaves[k].dt] > wide) wide = (int)itemsize[pl.p.leaves[k].dt];
     const bool aligned = pl.p.leaves[k].ptr % (4ull * itemsize[pl.p.leaves[k].dt]) == 0;
     if (row == pl.cols && col == 1 && aligned) kinds->push_back('f');
     else if (row == 0 && col == 1) kinds->push_back(whole && aligned ? 'q' : 'p');
     else if (col == 0) kinds->push_back(whole ? 'w' : 'r');
     else if (col == 1 && whole && aligned && row % 4 == 0) kinds->push_back('v');
-    else if (pl.cols < kBlock) kinds->push_back('g');
-    else return false;
+    else if (pl.cols < kBlock) {
+      kinds->push_back('g');
+      if (col != 1) spread = true;
+    } else return false;
   }
-  return true;
+  return flat_cols(*kinds, pl.cols, n, wide, spread, map_tile(pl.kinds));
 }
 
 // Kernel for the plan (mode 'm' map, 'f' flat map, 's' row sum), by structure;

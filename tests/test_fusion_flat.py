@@ -177,3 +177,46 @@ def test_column_sums_of_expressions(rows, cols, dtype, monkeypatch):
     if dtype != np.float16:
         v = x.astype(np.float64)
         assert np.allclose(cp.std(dx, axis=0).get(), v.std(axis=0), rtol=8 * np.finfo(dtype).eps)
+
+
+@pytest.mark.parametrize("kinds,cols,n,wide,flat", [
+    # rows that fill the row launch's workgroups, in the caches
+    ("fp", 511, 12_000_000, 4, True), ("fp", 1023, 12_000_000, 4, False),
+    ("fp", 3001, 12_000_000, 4, False), ("pr", 1023, 12_000_000, 4, False),
+    ("fr", 1023, 12_000_000, 4, True), ("fr", 3001, 12_000_000, 4, False),
+    ("fp", 4097, 12_000_000, 4, True), ("fp", 40_001, 12_000_000, 4, False),
+    ("fq", 900, 12_000_000, 4, True), ("fq", 3500, 12_000_000, 4, False),
+    ("fp", 1023, 12_000_000, 2, True), ("fp", 3001, 12_000_000, 2, False),
+    ("fr", 3001, 12_000_000, 2, True), ("fq", 3500, 12_000_000, 2, True),
+    ("fp", 130, 12_000_000, 8, True), ("fp", 255, 12_000_000, 8, False),
+    ("fq", 300, 12_000_000, 8, False), ("fqv", 300, 12_000_000, 8, True),
+    ("pr", 40_001, 12_000_000, 8, False),
+    # larger than those
+    ("fp", 3001, 70_000_000, 4, True), ("fp", 40_001, 70_000_000, 4, True),
+    ("pr", 3001, 70_000_000, 4, False), ("qw", 3500, 70_000_000, 4, True),
+    ("fp", 3001, 70_000_000, 2, True), ("pr", 3001, 70_000_000, 2, False),
+    ("fq", 300, 70_000_000, 8, True), ("fp", 511, 70_000_000, 8, False),
+    ("fp", 5001, 70_000_000, 8, True), ("pr", 5001, 70_000_000, 8, False)])
+def test_rows_go_flat_where_that_was_quicker(kinds, cols, n, wide, flat):
+    assert F._flat_cols(list(kinds), cols, n, wide, False, 4096) is flat
+
+
+_UNARY = ["sin", "cos", "tanh", "exp", "log1p", "sqrt", "arctan", "cbrt"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i,dtype,cols,rows", [(0, np.float64, 130, 3000), (1, np.float64, 200, 3000),
+                                               (2, np.float32, 513, 700), (3, np.float32, 3001, 90),
+                                               (4, np.float32, 4097, 40), (5, np.float32, 2052, 70),
+                                               (6, np.float16, 1025, 300), (7, np.float64, 301, 60_000)])
+def test_both_dispatchers_take_the_same_launch(i, dtype, cols, rows, monkeypatch):
+    """The native rule and the Python one agree: the modes of the kernels that
+    they ask for, for expressions that nothing else builds."""
+    x, r, c = (cp.array(np.ones(s, dtype)) for s in ((rows, cols), (cols,), (rows, 1)))
+    modes, source = [], F.generate_source
+    monkeypatch.setattr(F, "generate_source", lambda *a, **k: modes.append(a[5]) or source(*a, **k))
+    for native in (True, False):
+        cp.set_config(native_dispatch=native)
+        y = getattr(cp, _UNARY[i])(cp.fmax(cp.fmin(x - r, x * c), r - c))
+        (cp.floor(y) if native else cp.ceil(y))._materialize_if_lazy()
+    assert len(modes) == 2 and modes[0] == modes[1]
