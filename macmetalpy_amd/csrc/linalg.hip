@@ -435,9 +435,10 @@ __global__ __launch_bounds__(kT) void k_lu_swap(T *__restrict__ a, int n, int j0
 // the other rows, four threads on the 32 contiguous values of a row each.
 // A block's values are loaded ahead of the solve that they wait for, and the
 // next triangle ahead of the subtraction.  The backward solve's divisions go
-// through each diagonal element's reciprocal, corrected by the remainder (the
-// correctly rounded quotient but for rare last places), since a division
-// proper in each of the chain's steps would be most of its time.  Grid (batch, ceil(nrhs / kRhs)).
+// through each diagonal element's reciprocal, corrected by the remainder in
+// fused multiply-adds (Markstein's method: the correctly rounded quotient but
+// for rare last places), since a division proper in each of the chain's steps
+// would be most of its time.  Grid (batch, ceil(nrhs / kRhs)).
 // Bound by the chain of blocks: float64 n = 500 450 -> 215 us, n = 1024 with
 // 1024 right-hand sides 19 -> 1.3 ms, against a barrier per unknown.
 constexpr int kRhs = 8;
@@ -554,7 +555,9 @@ __global__ __launch_bounds__(512) void k_lu_solve(const T *__restrict__ lu, cons
   for (int t = tid; t < n * cw; t += nt) B[(long long)(t / cw) * nrhs + t % cw] = X[(t % cw) * n + t / cw];
 }
 
-// Orders whose right-hand sides do not fit LDS: workgroup (b, y) handles right-hand sides [y * kRhsChunk, ...) of matrix b.
+// Few unknowns (mmpi::solve_block_waves), and orders whose right-hand sides do
+// not fit LDS: workgroup (b, y) handles right-hand sides [y * kRhsChunk, ...) of
+// matrix b.
 template <typename T>
 __global__ __launch_bounds__(kT) void k_getrs(const T *__restrict__ lu, const int *__restrict__ piv,
                                               T *__restrict__ b, int n, int nrhs) {
@@ -1163,9 +1166,12 @@ extern "C" int mmp_lu_solve(int dtype, const void *lu, const int32_t *piv, void 
   if (batch == 0 || n == 0 || nrhs == 0) return MMP_OK;
   if (!lu || !piv || !b) return mmpi::fail(MMP_E_ARG, "mmp_lu_solve: null pointer");
   const size_t lds = (size_t)n * (size_t)(nrhs < kRhs ? nrhs : kRhs) * (dtype == MMP_F32 ? 4 : 8);
-  if (lds <= kSolveLds && mmpi::ceil_div(nrhs, kRhs) <= 65535) {
+  const int waves = mmpi::solve_block_waves(batch, (int)n, (int)(nrhs < 0x7fffffff ? nrhs : 0x7fffffff),
+                                            dtype == MMP_F32 ? 4 : 8,
+                                            mmpi::cu_count() > 0 ? mmpi::cu_count() : 256);
+  if (waves && lds <= kSolveLds && mmpi::ceil_div(nrhs, kRhs) <= 65535) {
     const dim3 g((unsigned)batch, (unsigned)mmpi::ceil_div(nrhs, kRhs));
-    const dim3 t(n <= 64 ? 64 : n <= 256 ? 256 : 512);
+    const dim3 t(64 * waves);
     if (dtype == MMP_F32)
       hipLaunchKernelGGL(k_lu_solve<float>, g, t, lds, mmpi::stream(), (const float *)lu,
                          (const int *)piv, (float *)b, (int)n, (int)nrhs);

@@ -210,4 +210,38 @@ inline bool scan_cols_by_vector(long long len, long long inner, int in_size, int
   return (len >= 3000 && inner <= 2048) || (len >= 256 && len * inner >= 24'000'000);
 }
 
+// Substitution with n unknowns: the kernel that solves blocks of 32 (8
+// right-hand sides a workgroup, a wave each), with `waves` waves a workgroup,
+// or 0: the one with a barrier per unknown and 32 right-hand sides a workgroup.
+// The block kernel's chain is 32 steps a block whatever n is, so few unknowns,
+// and many right-hand sides of them, are quicker by the other.  Us, by unknown /
+// by block; float64: 1 x (16, 1 right-hand side) 11 / 13, (32, 1) 20 / 14, (32, 4)
+// 20 / 22, (64, 8) 51 / 63, (128, 8) 139 / 123, (64, 40) 109 / 64; 2000 x (32, 1)
+// 28 / 21, (32, 40) 165 / 439, (64, 4) 102 / 101, (80, 40) 1300 / 1176; 20,000 x
+// (4, 40) 74 / 1794; float32: 1 x (32, 4) 20 / 17, (64, 8) 47 / 44; 2000 x (64, 4)
+// 66 / 72, (96, 40) 1140 / 774; 20,000 x (16, 1) 118 / 78.
+// Waves: one per right-hand side and enough for the rows below a block, but in
+// all what keeps a CU busy, since they divide the same work: float64 n = 300, one
+// right-hand side, of 300 matrices 175 / 162 / 157 / 276 with 1 / 2 / 4 / 8 waves,
+// of 1500 306 / 423 / 541 / 898; 20 x (1000, 1000), whose right-hand sides let
+// two workgroups into a CU's LDS, 27.6 / 17 / 9.8 / 12.6 ms.
+inline int solve_block_waves(long long batch, int n, int nrhs, int elem, long long cus) {
+  const long long wgs = batch * ((nrhs + 7) / 8);
+  const bool filled = wgs > 4 * cus;
+  const int least = nrhs == 1   ? (elem == 8 || batch <= 4096 ? 17 : 9)
+                    : nrhs == 2 ? (elem == 4 ? 24 : filled ? 56 : 32)
+                    : nrhs <= 4 ? (elem == 8 ? 88 : filled ? 80 : 32)
+                    : nrhs <= 8 ? (elem == 4 && !filled ? 64 : 96)
+                                : (filled ? 88 : nrhs >= 32 ? 48 : 64);
+  if (n < least) return 0;
+  int want = n <= 64 ? 1 : n <= 256 ? 2 : 8;
+  while (want < 8 && want < nrhs) want *= 2;
+  const long long lds = (long long)n * (nrhs < 8 ? nrhs : 8) * elem;
+  long long here = (wgs + cus - 1) / cus, fit = 160 * 1024 / lds;  // workgroups on a CU
+  if (here > fit) here = fit > 1 ? fit : 1;
+  int w = 8;
+  while (w > 1 && w * here > (elem == 8 ? 10 : 20)) w /= 2;
+  return want < w ? want : w;
+}
+
 }  // namespace mmpi

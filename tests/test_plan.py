@@ -45,6 +45,9 @@ long long t_groups(int heavy, int elem, long long outer, long long len, long lon
 int t_scan(long long len, long long inner, int in, int out) {
   return mmpi::scan_cols_by_vector(len, inner, in, out);
 }
+int t_solve(long long batch, int n, int nrhs, int elem) {
+  return mmpi::solve_block_waves(batch, n, nrhs, elem, 256);
+}
 int t_tagged_slot() { return mmpi::SCRATCH_REDUCE_PARTIALS; }
 int t_slots() { return mmpi::SCRATCH_NSLOTS; }
 }
@@ -154,3 +157,19 @@ def test_product_grids_fit(plans, elem):
 def test_column_scans_by_vector(plans, length, inner, sizes, vector):
     """The layout that was quicker for rows that are no whole aligned vectors."""
     assert plans.t_scan(ctypes.c_longlong(length), ctypes.c_longlong(inner), *sizes) == vector
+
+
+def test_substitution_plan(plans):
+    """The block kernel's waves: a power of two, none for a few unknowns, and
+    never more of them in a CU than its LDS and registers are planned for."""
+    seen = set()
+    for elem in (4, 8):
+        for batch in (1, 7, 300, 5000, 100_000):
+            for n in (1, 2, 8, 9, 16, 17, 23, 24, 31, 32, 64, 65, 100, 256, 257, 2000, 4096):
+                for nrhs in (1, 2, 3, 8, 9, 31, 32, 1000, 0x7FFFFFFF):
+                    w = plans.t_solve(ctypes.c_longlong(batch), n, nrhs, elem)
+                    assert w in (0, 1, 2, 4, 8)
+                    assert w or n < 97
+                    assert not w or n > 8
+                    seen.add(w)
+    assert seen == {0, 1, 2, 4, 8}
