@@ -36,6 +36,17 @@ def _batch_operand(x, batch_shape, mat_shape):
     return x._broadcast_copy(tuple(batch_shape) + tuple(mat_shape), x._dtype), _prod(mat_shape)
 
 
+def _whole(x, batch_shape, row, size):
+    """(transposed, row stride, batch stride) of a contiguous device operand
+    with the product's own batch, or one matrix for all of it; else None."""
+    if not x._is_device_contiguous():
+        return None
+    lead = x._shape[:-2]
+    if lead == batch_shape:
+        return False, row, size
+    return (False, row, 0) if _prod(lead) == 1 else None
+
+
 def _in_place(x, batch_shape):
     """(transposed, row stride, batch stride) of a device view that the
     general kernel can read where it lies, or None.  Its matrices have one
@@ -90,29 +101,26 @@ def matmul(x1, x2, out=None, **kwargs):
     K2, N = B._shape[-2:]
     if K != K2:
         raise ValueError(f"matmul shape mismatch: ({M},{K}) @ ({K2},{N})")
-    batch_shape = broadcast_shapes(A._shape[:-2], B._shape[:-2])
+    batch_shape = tuple(broadcast_shapes(A._shape[:-2], B._shape[:-2]))
     batch = _prod(batch_shape)
     if A._dtype != rdt:
         A = A.astype(rdt)
     if B._dtype != rdt:
         B = B.astype(rdt)
-    if (A._is_device_contiguous() and B._is_device_contiguous()
-            and A._shape[:-2] == B._shape[:-2]):
-        pa, pb = (False, K, M * K), (False, N, K * N)
-    else:
-        pa = pb = None
+    pa, pb = _whole(A, batch_shape, K, M * K), _whole(B, batch_shape, N, K * N)
+    if pa is None or pb is None:
         if rdt.kind == "f" and rdt.itemsize > 2:
             A._ensure_gpu()
             B._ensure_gpu()
             if rdt.itemsize == 8 or not _copy_kernel_shape(M, N, K, batch):
-                pa, pb = _in_place(A, batch_shape), _in_place(B, batch_shape)
+                pa, pb = pa or _in_place(A, batch_shape), pb or _in_place(B, batch_shape)
         if pa is None:
             A, sA = _batch_operand(A, batch_shape, (M, K))
             pa = False, K, sA
         if pb is None:
             B, sB = _batch_operand(B, batch_shape, (K, N))
             pb = False, N, sB
-    res = ndarray._empty_device(tuple(batch_shape) + (M, N), rdt)
+    res = ndarray._empty_device(batch_shape + (M, N), rdt)
     if res.size:
         if K == 0:
             res.fill(0)
