@@ -1064,7 +1064,7 @@ COL_SUM_MIN = 1 << 24
 def run_col_sum(root: FusionNode, out_dtype, out_ptr: int, scale: float) -> bool:
     """Sum of a 2-D floating ``root`` down its columns, times ``scale``, into
     ``out_ptr`` without materialising it; False where the leaves' strides are
-    not a column-sum launch's.  mean((x - m)**2, axis=0) of a 2,000,000 x 50
+    not a column-sum launch's.  The mean of (x - m)**2 down the columns of a 2,000,000 x 50
     float32 x: 210 us through a temporary, 72 fused."""
     prog = _Program(root)
     _, outer, cols, leaf_str, _ = _plan(prog, root._shape, keep_last=True)

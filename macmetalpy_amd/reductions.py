@@ -157,18 +157,6 @@ def _reduce(a, kind, axis=None, dtype=None, out=None, keepdims=False):
         run_sum(node, axes is not None, odt, res._ptr, kind == "mean")
         return _finish(res, out)
 
-    if (a._fusion_node is not None and kind in ("sum", "mean") and dtype is None and a.ndim == 2
-            and axes == (0,) and a._dtype.kind == "f" and get_config().fusion):
-        from ._fusion import COL_SUM_MIN, run_col_sum
-        # a float64 mean divides afterwards, as its own reduction does: a
-        # reciprocal's rounding would show there
-        wide = kind == "mean" and odt == np.float64
-        res = ndarray._empty_device(oshape, odt)
-        if a.size >= COL_SUM_MIN and run_col_sum(a._fusion_node, odt, res._ptr,
-                                                 1.0 / red_len if kind == "mean" and not wide
-                                                 else 1.0):
-            return _finish(res / float(red_len) if wide else res, out)
-
     x = a._ensure_contiguous()
     lay = _layout(x._shape, axes)
     if lay is None:
@@ -418,6 +406,27 @@ def cumprod(a, axis=None, dtype=None, out=None):
     return _scan(a, _abi.SCAN_CUMPROD, "cumprod", axis, dtype, out)
 
 
+def _mean_down(t, keepdims):
+    """mean(t, axis=0) of a lazy 2-D floating ``t`` in one pass that does not
+    write it, or None where that pass does not apply.  For expressions that
+    nothing else holds: a caller's own is evaluated once, by the reduction, and
+    kept, since its program may reduce it again or read it."""
+    if t._fusion_node is None or t._dtype.kind != "f" or not get_config().fusion:
+        return None
+    from ._fusion import COL_SUM_MIN, run_col_sum
+    if t.size < COL_SUM_MIN:
+        return None
+    odt = _np_out_dtype("mean", t._dtype)
+    rows = t._shape[0]
+    # a float64 mean divides afterwards, as its own reduction does: a
+    # reciprocal's rounding would show there
+    wide = odt == np.float64
+    res = ndarray._empty_device(_out_shape(t._shape, (0,), keepdims), odt)
+    if not run_col_sum(t._fusion_node, odt, res._ptr, 1.0 if wide else 1.0 / rows):
+        return None
+    return res / float(rows) if wide else res
+
+
 def var(a, axis=None, dtype=None, out=None, ddof=0, keepdims=False):
     """Variance as mean(|x - mean(x)|**2) * n / (n - ddof); with fusion on,
     the deviation, square and mean run as one kernel per pass."""
@@ -432,7 +441,11 @@ def var(a, axis=None, dtype=None, out=None, ddof=0, keepdims=False):
     m = mean(a, axis=axis, keepdims=True)
     if axes is None:
         m = m.reshape(())
-    v = mean(square(a - m), axis=axis, keepdims=keepdims)
+    dev2, v = square(a - m), None
+    if a.ndim == 2 and axes == (0,) and a._strides[-1] == 1:
+        v = _mean_down(dev2, keepdims)
+    if v is None:
+        v = mean(dev2, axis=axis, keepdims=keepdims)
     if ddof:
         v = v * (n / builtins.max(n - ddof, 0)) if n - ddof > 0 else v * np.inf
     return _finish(v, out)

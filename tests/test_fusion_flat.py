@@ -165,7 +165,15 @@ def test_column_sums_of_expressions(rows, cols, dtype, monkeypatch):
         g.integers(-3, 4, (rows, 1)).astype(dtype)
     dw, dr, dc = cp.array(wide), cp.array(r), cp.array(c)
     dx = dw[:, 1:cols + 1]
-    print("colsum", rows, cols, np.dtype(dtype), flush=True)
+    def down(expr):  # the one-pass sum itself
+        from macmetalpy_amd.ndarray import ndarray
+        res = ndarray._empty_device((cols,), expr._dtype)
+        assert F.run_col_sum(expr._fusion_node, expr._dtype, res._ptr, 1.0)
+        return res
+
+    for got, e in ((down((dx - dr) * dc), (x - r) * c), (down(dx * dx.copy() + dc), x * x + c)):
+        want = np.sum(e.astype(np.float64), axis=0).astype(dtype)
+        assert got.dtype == want.dtype and np.array_equal(got.get(), want, equal_nan=True)
     for got, e in ((cp.sum((dx - dr) * dc, axis=0), (x - r) * c),
                    (cp.sum(dx * dx.copy() + dc, axis=0, keepdims=True), x * x + c)):
         want = np.sum(e.astype(np.float64), axis=0, keepdims=got.ndim == 2).astype(dtype)
@@ -177,6 +185,30 @@ def test_column_sums_of_expressions(rows, cols, dtype, monkeypatch):
     if dtype != np.float16:
         v = x.astype(np.float64)
         assert np.allclose(cp.std(dx, axis=0).get(), v.std(axis=0), rtol=8 * np.finfo(dtype).eps)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_callers_expression_is_evaluated_once(native, monkeypatch):
+    """A lazy expression that its program holds is evaluated by the first
+    reduction down its columns and kept for the next; var's own deviations,
+    which nothing else holds, are not written at all."""
+    monkeypatch.setattr(F, "COL_SUM_MIN", 1 << 18)
+    ran = []
+    monkeypatch.setattr(F, "run_col_sum", lambda *a, f=F.run_col_sum: ran.append(1) or f(*a))
+    cp.set_config(native_dispatch=native)
+    x = np.random.default_rng(2).integers(-8, 9, (6000, 50)).astype(np.float32)
+    d = cp.array(x)
+    for f, want in ((cp.sum, x * 2 + 1), (cp.mean, None), (cp.var, None), (cp.std, None)):
+        t = d * 2.0 + 1.0
+        first = f(t, axis=0).get()
+        assert t._fusion_node is None
+        if want is not None:
+            assert np.array_equal(first, want.sum(axis=0)) and np.array_equal(t.get(), want)
+    assert len(ran) == 2  # var and std
+    assert np.allclose(cp.var(d, axis=0).get(), x.astype(np.float64).var(axis=0), rtol=1e-6)
+    assert np.allclose(cp.var(d.T, axis=0).get(), x.T.astype(np.float64).var(axis=0), rtol=1e-6)
+    assert len(ran) == 3  # not down the columns of a transposed view
 
 
 @pytest.mark.parametrize("kinds,cols,n,wide,flat", [
