@@ -39,7 +39,7 @@ constexpr int kMaxSweeps = 60;
 constexpr int kMaxEighN = 2048;   // rotation table in LDS: kMaxEighN / 2 pairs
 constexpr int kMaxSvdRows = 8192;
 constexpr int kNb = 64;             // panel width in memory (Cholesky, tall LU panels)
-constexpr int kBlockedMinN = 256;   // from this order a few matrices use the blocked Cholesky
+constexpr int kBlockedMinN = 256;   // from this order a few matrices use products of blocks
 constexpr int kBlockedMaxBatch = 64;
 constexpr int kRhsChunk = 32;       // right-hand sides per workgroup in the substitution
 
@@ -127,7 +127,15 @@ __device__ __forceinline__ void pair_of(int r, int pi, int N, int &p, int &q) {
 // panel of kLuW (or fewer) columns: k_lu_panel factors the panel with its
 // rows in registers, k_lu_swap applies the panel's row swaps to the other
 // columns and forms U12 = L11^-1 A12, and the trailing update
-// A22 -= L21 U12 is the matrix-product kernel subtracting in place.
+// A22 -= L21 U12 is k_lu_update, or for a few large matrices the
+// matrix-product kernel subtracting in place.
+//
+// With k_lu_update every element goes through the operations of elimination
+// column by column, in their order, each rounded by itself: the factors do not
+// depend on the blocks, and a row that repeats another one ends in exact zeros,
+// so that the matrix is reported as singular.  Sums in the matrix cores round
+// differently from the triangular solve, and leave such a row a last place off
+// zero.
 //
 // What bounds it is the chain of n pivot steps (each an argmax over the
 // column, a row handed round, a division), not arithmetic: float64 n = 500
@@ -396,7 +404,10 @@ __global__ __launch_bounds__(kT) void k_lu_swap(T *__restrict__ a, int n, int j0
     if (srow[q] >= 0 && on) A[(long long)srow[q] * n + c] = t[u];
   }
   __syncthreads();
-  if (wave != 0 || !on || c < j0 + jb) return;
+  if (wave != 0) return;
+  const int dk = j0 + (lane < jb ? lane : 0);  // a zero pivot eliminates nothing
+  const unsigned long long zero = __ballot(lane < jb && A[(long long)dk * n + dk] == T(0));
+  if (!on || c < j0 + jb) return;
   T x[kLuW];
 #pragma unroll
   for (int i = 0; i < kLuW; ++i) {
@@ -407,7 +418,7 @@ __global__ __launch_bounds__(kT) void k_lu_swap(T *__restrict__ a, int n, int j0
   for (int kk = 0; kk < kLuW; kk += 4) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      if (kk + s < jb) {
+      if (kk + s < jb && !((zero >> (kk + s)) & 1)) {
         const T *l = &Lt[kk + s][kk];
         const T xk = x[s];
 #pragma unroll
@@ -425,6 +436,80 @@ __global__ __launch_bounds__(kT) void k_lu_swap(T *__restrict__ a, int n, int j0
       if (kk + s < jb) A[(long long)(j0 + kk + s) * n + c] = x[s];
 #pragma unroll
     for (int i = 0; i + 4 < kLuW; ++i) x[i] = x[i + 4];
+  }
+}
+
+// A22 -= L21 U12 by the panel's `jb` columns (8, 16 or 32) from `j0`, whose rows
+// end at row `r1`: 64 x 64 outputs per workgroup, 4 x 4 per thread, L21 and U12
+// in LDS.  Each product and each difference is rounded, column after column; a
+// column whose pivot is zero eliminates nothing.  Grid (tiles^2, batch).
+// Determinants by sums in the matrix cores / by this: 200 float64 matrices of
+// 300 1146 / 1171 us, 100 of 100 242 / 254, float32 300 of 128 275 / 286.
+template <typename T>
+__global__ __launch_bounds__(kT) void k_lu_update(T *__restrict__ a, int n, int j0, int jb, int r1,
+                                                  int tiles) {
+  constexpr int TS = 64;
+  __shared__ __attribute__((aligned(16))) T Ls[kLuW][TS + 4];  // L21 transposed
+  __shared__ __attribute__((aligned(16))) T Us[kLuW][TS];
+  T *A = a + (long long)blockIdx.y * n * n;
+  const int tid = threadIdx.x, lane = tid & 63, tx = tid & 15, ty = tid >> 4;
+  const int r0 = r1 + (int)(blockIdx.x / (unsigned)tiles) * TS;
+  const int c0 = r1 + (int)(blockIdx.x % (unsigned)tiles) * TS;
+  {
+    const int i = tid >> 2, k = (tid & 3) * 8;
+    T l[8];
+    if (k < jb) {
+      load_row<8>(l, A + (long long)(r0 + i < n ? r0 + i : n - 1) * n + j0 + k, 8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) Ls[k + e][i] = l[e];
+    }
+  }
+  {
+    const int k = tid >> 3, c = (tid & 7) * 8;
+    T u[8];
+    if (k < jb) {
+      load_row<8>(u, A + (long long)(j0 + k) * n + c0 + c, n - c0 - c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) Us[k][c + e] = u[e];
+    }
+  }
+  const int dk = j0 + (lane < jb ? lane : 0);
+  const unsigned long long zero = __ballot(lane < jb && A[(long long)dk * n + dk] == T(0));
+  T acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = r0 + ty + 16 * i;
+    load_row<4>(acc[i], A + (long long)(r < n ? r : n - 1) * n + c0 + tx * 4, n - c0 - tx * 4);
+  }
+  __syncthreads();
+  for (int k0 = 0; k0 < jb; k0 += 8) {
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      const int k = k0 + kk;
+      if (zero && ((zero >> k) & 1)) continue;  // uniform
+      T l[4], u[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) l[i] = Ls[k][ty + 16 * i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = Us[k][tx * 4 + j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] -= l[i] * u[j];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = r0 + ty + 16 * i;
+    if (r >= n) continue;
+    T *o = A + (long long)r * n + c0 + tx * 4;
+    if (c0 + tx * 4 + 4 <= n) {
+      __builtin_memcpy(o, acc[i], sizeof(acc[i]));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (c0 + tx * 4 + j < n) o[j] = acc[i][j];
+    }
   }
 }
 
@@ -709,7 +794,7 @@ void launch_panel(T *A, long long batch, int n, int j0, int jb, int *piv, int *i
 }
 
 template <typename T>
-int lu_blocked(int dtype, T *A, long long batch, int n, int *piv, int *info) {
+int lu_blocked(int dtype, T *A, long long batch, int n, int *piv, int *info, bool in_order) {
   constexpr int F = 8 / (int)sizeof(T);  // float rows in the registers of a double row
   const long long nn = (long long)n * n;
   for (int j0 = 0, jb; j0 < n; j0 += jb) {
@@ -742,7 +827,14 @@ int lu_blocked(int dtype, T *A, long long batch, int n, int *piv, int *info) {
     }
     if (int st = mmpi::check_launch("mmp_lu")) return st;
     const int n2 = n - j0 - jb;
-    if (n2 > 0) {
+    if (n2 > 0 && in_order) {
+      const unsigned tiles = (unsigned)mmpi::ceil_div(n2, 64);
+      for (int k = 0; k < jb; k += kLuW)
+        hipLaunchKernelGGL(k_lu_update<T>, dim3(tiles * tiles, (unsigned)batch), dim3(kT), 0,
+                           mmpi::stream(), A, n, j0 + k, jb - k < kLuW ? jb - k : kLuW, j0 + jb,
+                           (int)tiles);
+      if (int st = mmpi::check_launch("mmp_lu")) return st;
+    } else if (n2 > 0) {
       T *P = A + (long long)j0 * n + j0;
       if (int st = mmpi::matmul_sub(dtype, batch, n2, n2, jb, P + (long long)jb * n, n, nn, P + jb, n,
                                     nn, P + (long long)jb * n + jb, n, nn))
@@ -1146,12 +1238,14 @@ extern "C" int mmp_lu(int dtype, void *a, int64_t batch, int64_t n, int32_t *piv
   if (n < 0 || n > 32768) return mmpi::fail(MMP_E_ARG, "mmp_lu: n %lld", (long long)n);
   if (batch == 0 || n == 0) return MMP_OK;
   if (!a || !piv || !info) return mmpi::fail(MMP_E_ARG, "mmp_lu: null pointer");
+  // few large matrices: their arithmetic is worth the matrix cores
+  const bool in_order = n < kBlockedMinN || batch > kBlockedMaxBatch;
   for (int64_t b0 = 0; b0 < batch; b0 += 65535) {  // a grid dimension's limit
     const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
     int *P = (int *)piv + b0 * n, *I = (int *)info + b0;
     const int st = dtype == MMP_F32
-                       ? lu_blocked<float>(dtype, (float *)a + b0 * n * n, nb, (int)n, P, I)
-                       : lu_blocked<double>(dtype, (double *)a + b0 * n * n, nb, (int)n, P, I);
+                       ? lu_blocked<float>(dtype, (float *)a + b0 * n * n, nb, (int)n, P, I, in_order)
+                       : lu_blocked<double>(dtype, (double *)a + b0 * n * n, nb, (int)n, P, I, in_order);
     if (st) return st;
   }
   return MMP_OK;

@@ -86,3 +86,51 @@ def test_solve(batch, n, nrhs, dtype):
     a, b, x = (t.astype(np.float64) for t in (a, b, x))
     bound = 8 * n * np.finfo(dtype).eps * (np.abs(a) @ np.abs(x) + np.abs(b))
     assert np.all(np.abs(a @ x - b) <= bound)
+
+
+def _eliminate(a):
+    """Elimination column by column with partial pivoting (the first row of
+    largest |a|), each product and difference rounded by itself."""
+    a, n, info = a.copy(), len(a), 0
+    piv = np.arange(n)
+    for k in range(n):
+        p = k + int(np.argmax(np.abs(a[k:, k])))
+        piv[k] = p
+        a[[k, p]] = a[[p, k]]
+        if a[k, k] == 0:
+            info = info or k + 1
+            continue
+        a[k + 1:, k] /= a[k, k]
+        a[k + 1:, k + 1:] -= a[k + 1:, k, None] * a[k, k + 1:]
+    return a, piv, info
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("batch,n", [(2, 31), (2, 33), (1, 65), (3, 100), (1, 129), (2, 200), (1, 255),
+                                     (65, 260)])
+def test_factors_are_elimination_by_columns(batch, n, dtype):
+    """Below 256 unknowns, and for many matrices, blocks change nothing: the
+    factors, pivots (with ties) and info are those of elimination column by
+    column, bit for bit; repeated rows and columns of zeros are exactly singular."""
+    g = np.random.default_rng(n)
+    for kind in ("normal", "ties", "repeated row", "zero column", "wide range"):
+        a = g.standard_normal((batch, n, n)).astype(dtype)
+        if kind == "ties":
+            a = np.sign(a) + (a > 1.5)
+        if kind == "repeated row":
+            a[:, n - 1] = a[:, 0]
+        if kind == "zero column":
+            a[:, :, n // 2] = 0
+        if kind == "wide range":
+            a *= (2.0 ** g.integers(-20, 20, a.shape)).astype(dtype)
+        a = a.astype(dtype)
+        lu, piv, info = _factor(a)
+        for b in (0, batch - 1):
+            want, wpiv, winfo = _eliminate(a[b])
+            assert np.array_equal(piv[b], wpiv) and info[b] == winfo, kind
+            assert np.array_equal(lu[b], want), kind
+        if kind in ("repeated row", "zero column"):
+            assert np.all(info > 0)
+        if kind == "repeated row":
+            with pytest.raises(np.linalg.LinAlgError):
+                cp.linalg.solve(cp.array(a), cp.array(a[:, :, :1]))
