@@ -124,6 +124,9 @@ def matmul(x1, x2, out=None, **kwargs):
     if res.size:
         if K == 0:
             res.fill(0)
+        elif not (pa[0] or pb[0]):
+            HipBackend().matmul(dtype_code(rdt), batch, M, N, K, A._ptr, pa[1], pa[2], B._ptr, pb[1],
+                                pb[2], res._ptr, N, M * N)
         else:
             HipBackend().matmul_t(dtype_code(rdt), pa[0], pb[0], batch, M, N, K, A._ptr, pa[1], pa[2],
                                   B._ptr, pb[1], pb[2], res._ptr, N, M * N)
