@@ -105,7 +105,6 @@ def test_flat_matches_numpy(cols, native):
             t = g.standard_normal((cols, rows), dtype=np.float32)
             i = g.integers(-9, 9, (rows, cols)).astype(np.int32)
             dx, dwide, dr, dc, dt, di = (cp.array(a) for a in (x, wide, r, c, t, i))
-            print("flat", rows, cols, flush=True)
             _same(((dx - dr) / dr).get(), (x - r) / r)
             _same(((dx - dc) * dr).get(), (x - c) * r)
             _same((dx * dwide[:, :cols] - dr).get(), x * wide[:, :cols] - r)

@@ -27,7 +27,6 @@ def _factor(a):
 def test_factors_multiply_back(batch, n, dtype):
     """P A = L U row for row: |L| <= 1 (partial pivoting), and the product is
     within the factorization's backward error bound, n u |L| |U|."""
-    print("lu", batch, n, np.dtype(dtype), flush=True)
     g = np.random.default_rng(n)
     a = g.standard_normal((batch, n, n)).astype(dtype)
     lu, piv, info = _factor(a)
@@ -77,7 +76,6 @@ def test_zero_and_nan_columns():
 def test_solve(batch, n, nrhs, dtype):
     """Residual within the substitution's backward error: n u (|A| + |L| |U|)
     |x| is below 8 n u of |A| |x| for these diagonally weighted matrices."""
-    print("solve", batch, n, nrhs, np.dtype(dtype), flush=True)
     g = np.random.default_rng(n + nrhs)
     a = g.standard_normal((batch, n, n)).astype(dtype) + (n ** 0.5 * np.eye(n)).astype(dtype)
     b = g.standard_normal((batch, n, nrhs)).astype(dtype)

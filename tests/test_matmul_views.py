@@ -86,7 +86,6 @@ def test_general_kernel_exact(batch, m, n, k, dtype):
     lead = (batch,) if batch > 1 else ()
     a, b = _ints(g, lead + (m, k), dtype), _ints(g, lead + (k, n), dtype)
     at, bt = np.ascontiguousarray(a.swapaxes(-1, -2)), np.ascontiguousarray(b.swapaxes(-1, -2))
-    print("general", batch, m, n, k, np.dtype(dtype), flush=True)
     for x in (cp.array(a), cp.array(at).swapaxes(-1, -2)):
         for y in (cp.array(b), cp.array(bt).swapaxes(-1, -2)):
             _exact(a, b, cp.matmul(x, y).get())
@@ -102,7 +101,6 @@ def test_general_half_kernel_exact(batch, m, n, k):
     g = np.random.default_rng(m * 1000 + n + k)
     lead = (batch,) if batch > 1 else ()
     a, b = (g.integers(-1, 2, lead + s).astype(np.float16) for s in ((m, k), (k, n)))
-    print("half", batch, m, n, k, flush=True)
     want = np.matmul(a.astype(np.float32), b.astype(np.float32))
     assert np.abs(want).max() <= 2048
     got = cp.matmul(cp.array(a), cp.array(b)).get()
@@ -118,6 +116,60 @@ def test_general_half_kernel_exact(batch, m, n, k):
                             n + 5, 0, dc._ptr, n + 1, 0)
         out = dc.get()
         assert np.array_equal(out[:, :n].astype(np.float32), want) and np.all(out[:, n:] == 7.0)
+
+
+def _to_bf16(x):
+    """Bits of the bfloat16 values of ``x``, which are exact there."""
+    bits = np.ascontiguousarray(x, np.float32).view(np.uint32)
+    assert not np.any(bits & 0xFFFF)
+    return (bits >> 16).astype(np.uint16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,n,k", [(1, 1, 2, 1), (1, 65, 63, 17), (1, 129, 257, 65), (1, 64, 64, 5000),
+                                         (70, 20, 30, 40), (1, 1030, 700, 100), (1, 300, 1, 4000),
+                                         (2, 640, 384, 448), (1, 2304, 2304, 64), (8, 1024, 1024, 128)])
+def test_bfloat16_products_exact(batch, m, n, k):
+    """bfloat16 has no NumPy type: its products through the entry point, all
+    kernels of the 16-bit types (general, whole aligned tiles, 256 wide tiles).
+    Products of -1, 0 and 1 over at most 200 terms are exact in eight bits."""
+    from macmetalpy_amd._backend import HipBackend
+    g = np.random.default_rng(m + n + k)
+    a, b = g.integers(-1, 2, (batch, m, k)), g.integers(-1, 2, (batch, k, n))
+    b[:, 200:] = 0
+    da, db = (cp.array(_to_bf16(x))._ensure_gpu() for x in (a, b))
+    c = cp.array(np.full((batch, m, n), 7, np.uint16))._ensure_gpu()
+    HipBackend().matmul(10, batch, m, n, k, da._ptr, k, m * k, db._ptr, n, k * n, c._ptr, n, m * n)
+    want = np.matmul(a.astype(np.float32), b.astype(np.float32))
+    assert np.array_equal(c.get(), _to_bf16(want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.float16])
+def test_rows_too_far_apart_for_lane_offsets(dtype):
+    """Row strides of 2^24 elements and more take the guarded loads: as the
+    left and the right operand, as stored and transposed."""
+    from macmetalpy_amd._backend import HipBackend
+    from macmetalpy_amd._dtypes import dtype_code
+    g = np.random.default_rng(9)
+    ld, rows, cols = (1 << 24) + 5, 5, 150
+    a = _ints(g, (rows, cols), dtype)
+    big = cp.zeros((rows, ld), dtype=dtype)
+    v = big[:, 3:3 + cols]
+    v[...] = cp.array(a)
+    x, y = _ints(g, (cols, 70), dtype), _ints(g, (rows, 40), dtype)
+    _exact(a, x, cp.matmul(v, cp.array(x)).get())
+    _exact(a.T, y, cp.matmul(v.T, cp.array(y)).get())
+    _exact(x.T, a.T, cp.matmul(cp.array(x).T, v.T).get())
+    _exact(y.T, a, cp.matmul(cp.array(y).T, v).get())
+    be, dc = HipBackend(), dtype_code(np.dtype(dtype))  # copies are Python's: the strides themselves
+    dx, dy = cp.array(x)._ensure_gpu(), cp.array(np.ascontiguousarray(y.T))._ensure_gpu()
+    c = cp.array(np.zeros((rows, 70), dtype))._ensure_gpu()
+    be.matmul(dc, 1, rows, 70, cols, v._ptr, ld, 0, dx._ptr, 70, 0, c._ptr, 70, 0)
+    _exact(a, x, c.get())
+    c = cp.array(np.zeros((40, cols), dtype))._ensure_gpu()
+    be.matmul(dc, 1, 40, cols, rows, dy._ptr, rows, 0, v._ptr, ld, 0, c._ptr, cols, 0)
+    _exact(y.T, a, c.get())
 
 
 @pytest.mark.gpu

@@ -79,14 +79,11 @@ def test_noalloc_matches_reduce_twice(op, dt, odt, first, second):
 
 
 def test_noalloc_lowered_strided_split_within_tolerance():
-    """Column sums along axis 0.  (65536, 2047) takes the column-per-thread
-    kernel (2047 is not a multiple of 4): 8 column blocks x 128 splits x 256
-    columns x 16 bytes of tagged slots is 4 MiB, more than the static
-    scratch's 4 MiB - 16 KiB of partials, so the no-alloc variant lowers the
-    split count to 127 (float64 partials either way): float32 results
-    within 1e-5 relative of the float64 sums, integer sums bit-exact.
-    (65536, 2048) takes the column-vector kernel (32 splits, 1 MiB: not
-    lowered); then a smaller input."""
+    """Column sums along axis 0 (float64 partials): 8 column blocks x 32
+    splits, whose partials a second kernel combines (rows that are whole
+    vectors and rows that are not), and 2 x 64 combined by the last workgroup.
+    float32 results within 1e-5 relative of the float64 sums, integer sums
+    bit-exact.  The splits that have to be lowered are the next test's."""
     be = HipBackend()
     lib = load_library()
     rng = np.random.default_rng(95)
@@ -104,13 +101,21 @@ def test_noalloc_lowered_strided_split_within_tolerance():
 
 
 def test_noalloc_lowered_split_nanmean():
-    """nanmean along axis 0 of (65536, 3) float32: one column block, 1024
-    splits of (sum, count) pairs (32 bytes of tagged slots per column) need
-    8 MiB, so the no-alloc variant lowers the split count to 510; results
-    within 1e-5 relative of the float64 NaN-skipping means."""
+    """nanmean along axis 0, (sum, count) pairs of 32 bytes of tagged slots
+    per column and split.  (4096, 4096) float16: 8 column blocks of 512 x 32
+    splits are 4 MiB, more than the static scratch's 4 MiB - 16 KiB, so the
+    no-alloc variant lowers the split count to 31; results within 1e-5 relative
+    of the float64 NaN-skipping means.  Then few columns."""
     be = HipBackend()
     lib = load_library()
     rng = np.random.default_rng(96)
+    x = rng.standard_normal((4096, 4096)).astype(np.float16)
+    x[::89, :] = np.nan
+    r1, r2, s0, s1 = _both(be, lib, _abi.REDUCE_NANMEAN, x, np.float32, 1, 4096, 4096)
+    assert s0 == s1
+    want = np.nanmean(x.astype(np.float64), axis=0)
+    scale = np.nanmean(np.abs(x).astype(np.float64), axis=0)
+    assert np.all(np.abs(r1 - want) <= 1e-5 * scale) and np.all(np.abs(r2 - want) <= 1e-5 * scale)
     for rows, cols in ((65536, 3), (4096, 5)):
         x = rng.standard_normal((rows, cols)).astype(np.float32)
         x[::89, :] = np.nan
@@ -156,10 +161,15 @@ def _hip_runtime():
 HIP_STREAM_CAPTURE_MODE_RELAXED = 2
 
 GRAPH_CASES = [
-    # (op, dtype, out dtype, (outer, len, inner)): split rows, then column partials
+    # (op, dtype, out dtype, (outer, len, inner)): split rows, then column
+    # partials: 42 combined by the last workgroup, 256 by a second kernel,
+    # none of a short axis
     (_abi.REDUCE_SUM, np.float32, np.float32, (1, 1 << 22, 1)),
     (_abi.REDUCE_SUM, np.int32, np.int64, (2, 1 << 20, 1)),
+    (_abi.REDUCE_MEAN, np.float32, np.float32, (1, 2700, 300)),
     (_abi.REDUCE_MEAN, np.float32, np.float32, (1, 4096, 300)),
+    (_abi.REDUCE_SUM, np.float32, np.float32, (1, 300_000, 40)),
+    (_abi.REDUCE_SUM, np.int32, np.int64, (3000, 12, 7)),
 ]
 
 
@@ -227,6 +237,52 @@ def test_noalloc_graph_replays_match_eager(op, dt, odt, shape):
                 assert np.all(np.abs(got - ref) <= 1e-5 * scale), rep
             else:
                 assert np.array_equal(got, v.sum(axis=1, dtype=np.int64).reshape(-1)), rep
+    finally:
+        if exe.value:
+            hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.float16])
+def test_captured_product_runs_unsplit(dt):
+    """A product that would split its K range takes no memory while the stream
+    is captured: it is recorded in one range, and its replays follow the
+    operands.  Sums of whole numbers, exact however they are cut."""
+    be, lib, hip = HipBackend(), load_library(), _hip_runtime()
+    rng = np.random.default_rng(98)
+    m, n, k = 64, 64, 6000
+    code = _abi.DTYPE_CODES[np.dtype(dt)]
+
+    def draw():
+        a, b = (rng.integers(-1, 2, s).astype(dt) for s in ((m, k), (k, n)))
+        b[2000:] = 0  # float16: sums stay below 2048
+        return a, b, (a.astype(np.float64) @ b.astype(np.float64)).astype(dt)
+
+    pa, pb, pc = be.create_buffer(m * k, dt), be.create_buffer(k * n, dt), be.create_buffer(m * n, dt)
+    a, b, want = draw()
+    be.write_buffer(pa, 0, a.ravel())
+    be.write_buffer(pb, 0, b.ravel())
+    be.matmul(code, 1, m, n, k, pa.ptr, k, 0, pb.ptr, n, 0, pc.ptr, n, 0)  # split, eagerly
+    assert np.array_equal(be.read_buffer(pc, 0, np.empty(m * n, dt)), want.ravel())
+    be.synchronize()
+    stats = be.memory_stats()
+    stream, graph, exe = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.mmp_stream(ctypes.byref(stream)) == 0 and stream.value
+    assert hip.hipStreamBeginCapture(stream, HIP_STREAM_CAPTURE_MODE_RELAXED) == 0
+    try:
+        be.matmul(code, 1, m, n, k, pa.ptr, k, 0, pb.ptr, n, 0, pc.ptr, n, 0)
+    finally:
+        end = hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+    assert end == 0 and graph.value and be.memory_stats() == stats
+    try:
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for rep in range(3):
+            a, b, want = draw()
+            be.write_buffer(pa, 0, a.ravel())
+            be.write_buffer(pb, 0, b.ravel())
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            be.synchronize()
+            assert np.array_equal(be.read_buffer(pc, 0, np.empty(m * n, dt)), want.ravel()), rep
     finally:
         if exe.value:
             hip.hipGraphExecDestroy(exe)
