@@ -466,17 +466,19 @@ int mmp_svd(int dtype, void *w, void *vt, int64_t batch, int64_t rows, int64_t l
  * stride ldb, C (M,N) row stride ldc; batch strides sA/sB/sC in elements
  * (0 broadcasts an operand).  dtype: MMP_F32, MMP_F16, MMP_BF16, MMP_F64
  * (float accumulation in fp32 for 16-bit inputs, fp64 for f64) or an
- * integer dtype (exact, wrapping). */
+ * integer dtype (exact, wrapping).  Floating products whose outputs are too
+ * few to fill the device split the K range and add the ranges' partial
+ * products in fp64; the partial products take memory from the allocator for
+ * the call.  While the stream is captured, or where there is no memory, the
+ * product runs in one range and allocates nothing: the same sums in another
+ * order, so their last places may differ. */
 int mmp_matmul(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                const void *A, int64_t lda, int64_t sA, const void *B,
                int64_t ldb, int64_t sB, void *C, int64_t ldc, int64_t sC);
 
 /* mmp_matmul with operands stored transposed: trans_a, A holds (K,M) with
  * row stride lda >= M; trans_b, B holds (N,K) with row stride ldb >= K.
- * Transposed operands: MMP_F32 and MMP_F64.  Products whose outputs are too
- * few to fill the device split the K range: their partial products take
- * memory from the allocator for the call (not while the stream is captured:
- * such a call runs unsplit). */
+ * Transposed operands: MMP_F32 and MMP_F64. */
 int mmp_matmul_t(int dtype, int trans_a, int trans_b, int64_t batch, int64_t M,
                  int64_t N, int64_t K, const void *A, int64_t lda, int64_t sA,
                  const void *B, int64_t ldb, int64_t sB, void *C, int64_t ldc,

@@ -7,10 +7,11 @@
 // Row-major operands: A (M, K) row stride lda, B (K, N) row stride ldb,
 // C (M, N) row stride ldc; batch strides sA, sB, sC (0 broadcasts).
 //
-// Floating kernels: a 128 x 128 (or 64 x 64, k_gemm4) output tile per
-// 256-thread workgroup, four wave64s in a 2 x 2 arrangement, each owning
-// 64 x 64 = 4 x 4 MFMA 16x16 tiles (64 fp32 accumulators per lane).  K advances in 128-byte slabs
-// (BK = 64 halves / 32 floats / 16 doubles) through two LDS buffers: the
+// Floating kernels: an output tile of 128 x 128 (in the general kernels 64 x 64
+// or 32 x 32 where mmpi::gemm_plan says so) per 256-thread workgroup, four
+// wave64s in a 2 x 2 arrangement, each owning a quarter of it in MFMA 16 x 16
+// tiles (4 x 4 of a 128 x 128 tile, 64 fp32 accumulators per lane).  K advances
+// in 128-byte slabs (BK = 64 halves / 32 floats / 16 doubles) through two LDS buffers: the
 // next slab is fetched into registers while the current one feeds the
 // MFMAs, then written to the other buffer (one barrier per slab).
 //  * float16 / bfloat16: v_mfma_f32_16x16x32_{f16,bf16}.  A lane's operand

@@ -140,14 +140,20 @@ inline int partials_slot(bool second) {
 // over the CUs (two 128, four 64 or eight 32 wide tiles fit one), each a
 // start-up plus its slabs, at the matrix cores' rate for the workgroups that
 // share a CU but no faster than one alone hides its loads; and the partials
-// at 6 TB/s plus a launch.  At most 16,384 outputs over a K of 16,384 or more
-// are always cut into ranges of at most 2048, whose sums meet in float64:
-// float32 sums of 10^7 terms then stay within 5e-8 of exact (2e-6 with ranges
-// of 6000).  Measured over tiles and splits, the choice is the
-// fastest or within a tenth of it: float32 1000^3 28 us (32 wide, unsplit; 64
-// wide 30, 128 wide in four splits 34), 2049^3 198 (64 wide; 128 wide 231),
-// 4000 x 70 x 3000 35 (32 wide in two; unsplit 128 wide 94); float64 500 x 500
-// x 100,000 0.84 ms (128 wide in 32; unsplit 15.8).
+// at 6 TB/s plus a launch.  A single product (batch 1) of at most 16,384
+// outputs over a K of 16,384 or more that may be split is always cut into
+// ranges of at most 2048 (up to K = 134,215,680; the grid has 65,535 of them),
+// whose sums meet in float64: float32 sums of 10^7 terms then stay within 5e-8
+// of exact (2e-6 with ranges of 6000).  A product that may not (the stream is
+// captured, or there is no memory for the partials) sums its K in one chain, so
+// its last places differ.
+// Measured over tiles and splits of 30 products, the choice is the fastest or
+// within a tenth of it but for float64 300 x (200 x 200 x 200), 204 us where 64
+// wide tiles take 151, and float64 4000 x 70 x 3000, 66 where four ranges take
+// 58.  float32 1000^3 28 us (32 wide, unsplit; 64 wide 30, in four 36), 2049^3
+// 198 (64 wide; 32 wide 200), 4000 x 70 x 3000 37 (32 wide in two; in four 35);
+// float64 500 x 500 x 100,000 0.85 ms (128 wide in 32; 64 wide in 16 0.81;
+// unsplit 15.8).
 // A tile whose workgroups are more than a grid holds is no choice (from 2^29
 // rows of one column on 32 wide ones are).
 struct GemmPlan {
