@@ -200,6 +200,19 @@ inline GemmPlan gemm_plan(long long batch, int M, int N, int K, int elem, bool m
   return best;
 }
 
+// Rows from which unaligned ones, each longer than a tile, are scanned by a
+// workgroup each instead of in tiles that look back.  What a row's waves walk
+// is paid in latency, so fewer rows need more bytes a step.  40,000,000
+// elements, us in tiles / by rows at 260, 416, 900 and 2000 rows: float32 157 /
+// 119, 152 / 90, 153 / 76, 191 / 73; int32 to int64 209 / 164, 208 / 129, 205 /
+// 113, 272 / 116; float64 209 / 200, 206 / 158, 221 / 148, 224 / 141; int64 166 /
+// 200, 162 / 159, 191 / 147, 187 / 141; float16 97 / 122, 87 / 77, 93 / 65, 130 /
+// 55; int16 to int64 104 / 171, 107 / 133, 100 / 119, 133 / 121.
+inline long long scan_by_rows_least(int in_size, int out_size) {
+  if (in_size <= 2 && out_size == 8) return 2000;
+  return in_size == 4 ? 256 : 400;
+}
+
 // Whether a scan down `inner` columns whose rows are not whole aligned vectors
 // takes 16-byte vectors (with a pass of its own for the chunks' carries) or a
 // column per thread.  Vectors pay where the carries are what a thread per column

@@ -922,7 +922,9 @@ int launch_scan(long long outer, long long len, long long inner, const void *x, 
                                        (len * (long long)sizeof(To)) % 16 == 0));
       // rows for the short-row kernel alone: under a tile, or unaligned and
       // enough of them to fill the device
-      const bool by_rows = len < kTile || (!vec && outer >= 256);
+      const bool by_rows =
+          len < kTile ||
+          (!vec && outer >= mmpi::scan_by_rows_least((int)sizeof(Ti), (int)sizeof(To)));
       const long long tpr = by_rows ? 0 : vec ? len / kTile : mmpi::ceil_div(len, kTile);
       const long long ntiles = outer * tpr;
       if (ntiles > 0x7fffffffLL || outer > 0x7fffffffLL)

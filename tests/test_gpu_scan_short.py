@@ -50,7 +50,8 @@ def test_unaligned_long_rows(dt):
                          ids=lambda d: np.dtype(d).name)
 def test_odd_columns(dt):
     g = np.random.default_rng(2)
-    for rows, cols in ((1, 5), (63, 9), (700, 1023), (1500, 7), (1500, 17), (130, 2051), (2000, 3)):
+    for rows, cols in ((1, 5), (63, 9), (700, 1023), (1500, 7), (1500, 17), (130, 2051), (2000, 3),
+                       (3000, 4), (3001, 7), (9000, 33), (3000, 1023), (8200, 37)):
         _check(_data(g, (rows, cols), dt), 0)
     h = _data(g, (3, 200, 33), dt)
     _check(h, 1)

@@ -48,6 +48,7 @@ int t_scan(long long len, long long inner, int in, int out) {
 int t_solve(long long batch, int n, int nrhs, int elem) {
   return mmpi::solve_block_waves(batch, n, nrhs, elem, 256);
 }
+long long t_scan_rows(int in, int out) { return mmpi::scan_by_rows_least(in, out); }
 int t_tagged_slot() { return mmpi::SCRATCH_REDUCE_PARTIALS; }
 int t_slots() { return mmpi::SCRATCH_NSLOTS; }
 }
@@ -173,3 +174,11 @@ def test_substitution_plan(plans):
                     assert not w or n > 8
                     seen.add(w)
     assert seen == {0, 1, 2, 4, 8}
+
+
+@pytest.mark.parametrize("sizes,tiled,by_rows", [((4, 4), 255, 260), ((4, 8), 255, 260), ((2, 2), 260, 416),
+                                                 ((8, 8), 260, 416), ((2, 8), 900, 2000), ((1, 8), 900, 2000)])
+def test_unaligned_rows_scanned_by_workgroups(plans, sizes, tiled, by_rows):
+    """Row counts at which scans in tiles, and by rows, were quicker."""
+    plans.t_scan_rows.restype = ctypes.c_longlong
+    assert tiled < plans.t_scan_rows(*sizes) <= by_rows
