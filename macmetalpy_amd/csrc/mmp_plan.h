@@ -106,7 +106,9 @@ inline ColPlan argreduce_cols_plan(long long outer, long long len, long long inn
 // sum, maximum, argmax over the middle axis): float32 60,000 x 16 x 9 90 / 8.5,
 // 91 / 8.9, 90 / 7.9; 625 x 16 x 1000 9.4 / 9.1, 9.9 / 9.5, 8.6 / 8.7; float16
 // 1 x 16 x 1,250,001 12.1 / 9.5, 13.7 / 12.4, 11.9 / 11.8; 1 x 32 x 625,001 9.8 /
-// 9.5, 12.9 / 18, 10 / 12.1.  Further on only where rows are shorter than a
+// 9.5, 12.9 / 18, 10 / 12.1; sums of 4 and 8 bytes at 64 rows: float32 1 x
+// 156,251 11.2 / 9.2, 78 x 1000 9.4 / 9, 3125 x 50 8.6 / 8.6, float64 1 x 78,125
+// 11 / 9.  Further on only where rows are shorter than a
 // workgroup and workgroups so many that starting them is the time: float32
 // 17,361 x 64 x 9 28 / 8.5, 30 / 17, 40 / 10.8, but 3125 x 64 x 50 8.6 / 8.6, 10 /
 // 17, 10.4 / 9.9; `heavy` (extremes of floats) by half as much.

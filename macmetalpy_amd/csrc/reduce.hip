@@ -984,18 +984,27 @@ __global__ __launch_bounds__(kBlock) void k_argreduce_short(const T *__restrict_
     C bv = R::ident().v;
     unsigned bi = kNone;
     const T *p = x + in;
-    for (long long l = 0; l < len; l += kColUnroll) {
-      T q[kColUnroll];
+    unsigned l = 0;
+    auto rows = [&](auto n) {  // n rows, loads ahead of the arithmetic
+      constexpr int N = decltype(n)::value;
+      T q[N];
 #pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) q[u] = p[(l + u < len ? l + u : len - 1) * inner];
+      for (int u = 0; u < N; ++u) q[u] = p[u * inner];
 #pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) {
+      for (int u = 0; u < N; ++u) {
         const C e = (C)q[u];
-        const bool upd = l + u < len && (R::seq_better(e, bv) | (bi == kNone)) & R::eligible(e);
+        const bool upd = (R::seq_better(e, bv) | (bi == kNone)) & R::eligible(e);
         bv = upd ? e : bv;
-        bi = upd ? (unsigned)(l + u) : bi;
+        bi = upd ? l + u : bi;
       }
-    }
+      p += N * inner;
+      l += N;
+    };
+    for (long long m = len; m >= kColUnroll; m -= kColUnroll)
+      rows(std::integral_constant<int, kColUnroll>());
+    if (len & 4) rows(std::integral_constant<int, 4>());
+    if (len & 2) rows(std::integral_constant<int, 2>());
+    if (len & 1) rows(std::integral_constant<int, 1>());
     out[at] = bi == kNone ? R::ident().i : (long long)bi;
   });
 }
@@ -1088,7 +1097,8 @@ int launch_reduce(long long outer, long long len, long long inner, const void *x
   }
   if (outer > 65535) return mmpi::fail(MMP_E_ARG, "strided reduction: outer extent %lld > 65535", outer);
   constexpr int SV = short_vec<T, To>();
-  if (mmpi::short_axis(outer, len, inner, SV, heavy<OP, T>() ? 16 : 24, heavy<OP, T>())) {
+  if (mmpi::short_axis(outer, len, inner, SV, heavy<OP, T>() ? 16 : sizeof(T) >= 4 ? 48 : 24,
+                       heavy<OP, T>())) {
     const bool whole = inner >= SV;
     const unsigned vecs = (unsigned)mmpi::ceil_div(inner, whole ? SV : 1);
     const unsigned total = (unsigned)outer * vecs;
