@@ -405,9 +405,9 @@ _FLAT_UNROLL = 4  # 4-element vectors per thread of a flat kernel
 _FLAT_MIN = 1 << 16
 
 
-def _flat_cols(kinds, cols, n, wide, spread, tile):
-    """Whether rows of ``cols`` elements of at most ``wide`` bytes go flat, ``n``
-    elements in all.
+def _flat_cols(kinds, cols, traffic, wide, spread, tile):
+    """Whether rows of ``cols`` elements of at most ``wide`` bytes go flat;
+    ``traffic``: bytes of the output and of the leaves as large as it.
 
     A vector of a flat launch reads four elements of a row vector (or of an odd
     row) one by one, which costs more than the row launch's scalar rows as long
@@ -427,7 +427,7 @@ def _flat_cols(kinds, cols, n, wide, spread, tile):
     ('v') 300 53 / 48, 700 48 / 49; with a transposed leaf (``spread``) 255 64 / 42;
     70,000,000: 300 246 / 225, 241 / 220, 215 / 240; 511 201 / 259, 200 / 244, 176 /
     246; 5001 335 / 266, 277 / 243, 159 / 239."""
-    big = n * wide >= 1 << 27
+    big = traffic >= 192 << 20  # float32 rows of 5001: 200 MB 38.8 / 37.6, 38.8 / 33, 26 / 28.7
     streams = "f" in kinds or "v" in kinds
     empty = -(-cols // tile) * tile / cols if cols > tile else 1.0  # the row launch's tiles
     if wide == 8:
@@ -483,7 +483,8 @@ def _flat_kinds(outer, cols, leaf_str, ptrs, itemsizes, out_ptr, out_itemsize, t
             return None
     wide = max(itemsizes + [out_itemsize])
     spread = any(k == "g" and st[1] != 1 for k, st in zip(kinds, leaf_str))
-    return kinds if _flat_cols(kinds, cols, outer[0] * cols, wide, spread, tile) else None
+    traffic = outer[0] * cols * (out_itemsize + sum(s for k, s in zip(kinds, itemsizes) if k in "fvg"))
+    return kinds if _flat_cols(kinds, cols, traffic, wide, spread, tile) else None
 
 
 def _flat_body(kinds, ct, vtypes, out_ct, expr_lines, res):

@@ -1186,10 +1186,10 @@ bool vec_ok(const Plan &pl, bool out_ok) {
 }
 
 // The Python _flat_cols, which says why.
-bool flat_cols(const std::string &kinds, long long cols, long long n, int wide, bool spread,
+bool flat_cols(const std::string &kinds, long long cols, long long traffic, int wide, bool spread,
                long long tile) {
   auto has = [&](char k) { return kinds.find(k) != std::string::npos; };
-  const bool big = n * wide >= 1LL << 27, streams = has('f') || has('v');
+  const bool big = traffic >= 192LL << 20, streams = has('f') || has('v');
   const double empty = cols > tile ? (double)((cols + tile - 1) / tile * tile) / (double)cols : 1.0;
   if (wide == 8) {
     const long long limit = has('v') ? 400 : spread ? 255 : !big ? 160 : streams ? 300 : 200;
@@ -1222,7 +1222,10 @@ bool flat_kinds(const Plan &pl, unsigned long long outp, int out_dt, std::string
       if (col != 1) spread = true;
     } else return false;
   }
-  return flat_cols(*kinds, pl.cols, n, wide, spread, map_tile(pl.kinds));
+  long long each = itemsize[out_dt];
+  for (size_t k = 0; k < pl.p.leaves.size(); ++k)
+    if ((*kinds)[k] == 'f' || (*kinds)[k] == 'v' || (*kinds)[k] == 'g') each += itemsize[pl.p.leaves[k].dt];
+  return flat_cols(*kinds, pl.cols, n * each, wide, spread, map_tile(pl.kinds));
 }
 
 // Kernel for the plan (mode 'm' map, 'f' flat map, 's' row sum), by structure;

@@ -227,9 +227,12 @@ def test_callers_expression_is_evaluated_once(native, monkeypatch):
     ("pr", 3001, 70_000_000, 4, False), ("qw", 3500, 70_000_000, 4, True),
     ("fp", 3001, 70_000_000, 2, True), ("pr", 3001, 70_000_000, 2, False),
     ("fq", 300, 70_000_000, 8, True), ("fp", 511, 70_000_000, 8, False),
-    ("fp", 5001, 70_000_000, 8, True), ("pr", 5001, 70_000_000, 8, False)])
+    ("fp", 5001, 70_000_000, 8, True), ("pr", 5001, 70_000_000, 8, False),
+    # 153 MB read, 38 written (a comparison's result): the caches hold it
+    ("fp", 145_921, 19_000_000, 4, False)])
 def test_rows_go_flat_where_that_was_quicker(kinds, cols, n, wide, flat):
-    assert F._flat_cols(list(kinds), cols, n, wide, False, 4096) is flat
+    traffic = n * wide * (1 + sum(k in "fv" for k in kinds))
+    assert F._flat_cols(list(kinds), cols, traffic, wide, False, 4096) is flat
 
 
 _UNARY = ["sin", "cos", "tanh", "exp", "log1p", "sqrt", "arctan", "cbrt"]
