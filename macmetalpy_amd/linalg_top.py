@@ -107,19 +107,20 @@ def matmul(x1, x2, out=None, **kwargs):
         A = A.astype(rdt)
     if B._dtype != rdt:
         B = B.astype(rdt)
-    pa, pb = _whole(A, batch_shape, K, M * K), _whole(B, batch_shape, N, K * N)
-    if pa is None or pb is None:
-        if rdt.kind == "f" and rdt.itemsize > 2:
+    pa = pb = None
+    if rdt.kind == "f" and rdt.itemsize > 2:
+        pa, pb = _whole(A, batch_shape, K, M * K), _whole(B, batch_shape, N, K * N)
+        if pa is None or pb is None:
             A._ensure_gpu()
             B._ensure_gpu()
             if rdt.itemsize == 8 or not _copy_kernel_shape(M, N, K, batch):
                 pa, pb = pa or _in_place(A, batch_shape), pb or _in_place(B, batch_shape)
-        if pa is None:
-            A, sA = _batch_operand(A, batch_shape, (M, K))
-            pa = False, K, sA
-        if pb is None:
-            B, sB = _batch_operand(B, batch_shape, (K, N))
-            pb = False, N, sB
+    if pa is None:
+        A, sA = _batch_operand(A, batch_shape, (M, K))
+        pa = False, K, sA
+    if pb is None:
+        B, sB = _batch_operand(B, batch_shape, (K, N))
+        pb = False, N, sB
     res = ndarray._empty_device(batch_shape + (M, N), rdt)
     if res.size:
         if K == 0:
