@@ -221,14 +221,14 @@ inline long long scan_by_rows_least(int in_size, int out_size) {
 // spends its time on, and for the largest inputs; 2-byte elements, whose eight
 // running sums a lane are too long a chain, and 8-byte ones, never.  By column /
 // by vectors, us: float32 10,000 x 33 44 / 19, 30,000 x 1001 101 / 73, 100,000 x
-// 333 125 / 89, 256 x 100,001 57 / 52, but 1000 x 1001 11 / 15, 3000 x 3001 25 /
+// 333 125 / 89, 10,000 x 5001 135 / 123, 256 x 100,001 57 / 52, but 1000 x 1001 11 / 15, 3000 x 3001 25 /
 // 26.5, 256 x 65,537 35.5 / 40.5, 1,000,000 x 33 375 / 498 (the axis is cut 256
 // times at most); int32 to int64 10,000 x 333 50 / 27, 100,000 x 33 97 / 73, but
 // 3000 x 1001 23 / 26, 100,000 x 5 53 / 59; float16 10,000 x 1001 53 / 82.
 inline bool scan_cols_by_vector(long long len, long long inner, int in_size, int out_size) {
   if (in_size != 4 || inner < 4 || len > (1 << 18)) return false;
-  if (out_size > 4) return len >= 8192 && inner >= 32 && inner <= 2048;
-  return (len >= 3000 && inner <= 2048) || (len >= 256 && len * inner >= 24'000'000);
+  if (out_size > 4) return len >= 8192 && inner >= 32 && inner <= 4096;
+  return len >= 8192 || (len >= 3000 && inner <= 2048) || (len >= 256 && len * inner >= 24'000'000);
 }
 
 // Substitution with n unknowns: the kernel that solves blocks of 32 (8

@@ -150,7 +150,7 @@ def test_product_grids_fit(plans, elem):
 
 
 @pytest.mark.parametrize("length,inner,sizes,vector", [
-    (10_000, 33, (4, 4), 1), (30_000, 1001, (4, 4), 1), (256, 100_001, (4, 4), 1), (3000, 1001, (4, 4), 1),
+    (10_000, 33, (4, 4), 1), (30_000, 1001, (4, 4), 1), (10_382, 2258, (4, 4), 1), (256, 100_001, (4, 4), 1), (3000, 1001, (4, 4), 1),
     (1000, 1001, (4, 4), 0), (3000, 3001, (4, 4), 0), (256, 16_385, (4, 4), 0), (256, 65_537, (4, 4), 0),
     (1_000_000, 33, (4, 4), 0), (10_000, 3, (4, 4), 0), (10_000, 333, (4, 8), 1), (100_000, 33, (4, 8), 1),
     (3000, 1001, (4, 8), 0), (100_000, 5, (4, 8), 0), (1000, 40_001, (4, 8), 0), (10_000, 1001, (2, 2), 0),
