@@ -149,9 +149,14 @@ inline int partials_slot(bool second) {
 // of exact (2e-6 with ranges of 6000).  A product that may not (the stream is
 // captured, or there is no memory for the partials) sums its K in one chain, so
 // its last places differ.
+// A slab of a 32 wide float64 tile loads twice as much for its arithmetic as one
+// of a 64 wide tile; where eight of them fill every CU and more wait, that is
+// what bounds them, and the slab counts for a third more.  Us with 32 / 64 / 128
+// wide tiles: 300 products of 200^3 204 / 157 / 161, 1000 of them 648 / 516 / 495, of
+// 160^3 306 / 238 / 382, 200 of 224^3 167 / 118 / 134; but 1500 x 700 x 900, 1034
+// tiles of 32, 62 / 73 / 81.
 // Measured over tiles and splits of 30 products, the choice is the fastest or
-// within a tenth of it but for float64 300 x (200 x 200 x 200), 204 us where 64
-// wide tiles take 151, and float64 4000 x 70 x 3000, 66 where four ranges take
+// within a tenth of it but for float64 4000 x 70 x 3000, 66 us where four ranges take
 // 58.  float32 1000^3 28 us (32 wide, unsplit; 64 wide 30, in four 36), 2049^3
 // 198 (64 wide; 32 wide 200), 4000 x 70 x 3000 37 (32 wide in two; in four 35);
 // float64 500 x 500 x 100,000 0.85 ms (128 wide in 32; 64 wide in 16 0.81;
@@ -182,11 +187,12 @@ inline GemmPlan gemm_plan(long long batch, int M, int N, int K, int elem, bool m
     if (!grid_fits(one, 256)) break;  // nor do smaller tiles
     const double tiles = (double)one * (double)batch;
     const double per_cu = tile == 128 ? 2 : tile == 64 ? 4 : 8;
+    const bool crowded = elem == 8 && tiles > cus * per_cu;  // (of 32 wide ones)
     const double start = tile == 128 ? 6.0 : tile == 64 ? 3.0 : 1.5;  // and the result's stores
     // a slab of one workgroup: of several sharing a CU, and alone on it (the
     // 16-bit matrix rate leaves a slab to its loads and LDS traffic)
     const double shared = elem == 2 ? (tile == 128 ? 0.85 : tile == 64 ? 0.4 : 0.18)
-                                    : (tile == 128 ? 1.85 : tile == 64 ? 0.5 : 0.15);
+                                    : (tile == 128 ? 1.85 : tile == 64 ? 0.5 : crowded ? 0.2 : 0.15);
     const double alone = elem == 2 ? (tile == 128 ? 1.05 : tile == 64 ? 0.55 : 0.35)
                                    : (tile == 128 ? 2.2 : tile == 64 ? 0.65 : 0.25);
     for (int s = s0; s <= 65535; s *= 2) {

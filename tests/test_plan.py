@@ -149,6 +149,15 @@ def test_product_grids_fit(plans, elem):
     assert _gemm(plans, 1, (1 << 29) - 32, 1, 2, elem)[0] == 32
 
 
+@pytest.mark.parametrize("batch,m,n,k,elem,tiles", [
+    (300, 200, 200, 200, 8, (64, 128)), (1000, 200, 200, 200, 8, (64, 128)), (200, 224, 224, 224, 8, (64, 128)),
+    (1000, 160, 160, 160, 8, (64,)), (1, 1500, 700, 900, 8, (32,)), (5000, 32, 32, 32, 8, (32,)),
+    (300, 200, 250, 33, 4, (32,)), (500, 120, 100, 90, 4, (128,))])
+def test_product_tiles(plans, batch, m, n, k, elem, tiles):
+    """The tiles that were quicker."""
+    assert _gemm(plans, batch, m, n, k, elem, batch == 1)[0] in tiles
+
+
 @pytest.mark.parametrize("length,inner,sizes,vector", [
     (10_000, 33, (4, 4), 1), (30_000, 1001, (4, 4), 1), (10_382, 2258, (4, 4), 1), (256, 100_001, (4, 4), 1), (3000, 1001, (4, 4), 1),
     (1000, 1001, (4, 4), 0), (3000, 3001, (4, 4), 0), (256, 16_385, (4, 4), 0), (256, 65_537, (4, 4), 0),
